@@ -2111,11 +2111,11 @@ struct Mfma<double> {
 };
 
 // Block shape of spread_mfma_kernel: 4 waves = (CPB / 16 column groups) x
-// (plane groups of ZH planes): 32 columns, the planes split over two waves, which
-// halves the accumulator registers and lets more blocks overlap their staging.
-template <typename R, int RX, int ZSB>
+// (plane groups of ZH planes).  CPB = 32 splits the planes over two waves, CPB = 16 over
+// four: fewer accumulators per wave, more blocks, and no idle column group when a batch
+// has no more than 16 real columns.
+template <int ZSB, int CPB>
 struct SpreadShape {
-    static constexpr int CPB = 32;
     static constexpr int NPG = 4 / (CPB / 16);
     static constexpr int ZH = (ZSB + NPG - 1) / NPG;
 };
@@ -2244,17 +2244,22 @@ __device__ inline RegionAt region_at(const RegionGeom& rg, int reg) {
 }
 
 // FP32: held to 128 registers (four waves per SIMD; at the compiler's 140 three, and the
-// N = 4000 monolayer's 1272 blocks took 1.7 rounds instead of 1.2: 39.4 against 37.0 us)
-template <typename R, int RX, int ZSB>
+// N = 4000 monolayer's 1272 blocks took 1.7 rounds instead of 1.2: 39.4 against 37.0 us).
+//
+// CPB = 16 is the form for few blocks (spread_cpb): there a region's candidates come in
+// several chunks and nothing else hides their loads, so the next chunk's values and
+// weights are fetched while the current chunk's products run.
+template <typename R, int RX, int ZSB, int CPB>
 __global__ __launch_bounds__(256, sizeof(R) == 4 ? 4 : 2) void spread_mfma_kernel(SlotTable tab, int B, RegionGeom rg,
                                                           const R* __restrict__ regw,
                                                           const int* __restrict__ reg_start,
-                                                          const int* __restrict__ reg_items, int N,
+                                                          const int* __restrict__ reg_items,
                                                           typename C2<R>::T* __restrict__ out) {
     using CT = typename C2<R>::T;
     using M = Mfma<R>;
-    using Sh = SpreadShape<R, RX, ZSB>;
-    constexpr int KC = kMfmaKC, CPB = Sh::CPB, ZH = Sh::ZH;
+    using Sh = SpreadShape<ZSB, CPB>;
+    constexpr int KC = kMfmaKC, ZH = Sh::ZH;
+    constexpr bool PREFETCH = CPB == 16;
     using L = RegionW<RX, ZSB>;
     __shared__ R s_v[KC][CPB + 1];
     __shared__ __align__(16) R s_w[KC][L::NW];
@@ -2277,28 +2282,66 @@ __global__ __launch_bounds__(256, sizeof(R) == 4 ? 4 : 2) void spread_mfma_kerne
         for (int p = 0; p < ZH; ++p) acc[xi][p] = typename M::V4{R(0), R(0), R(0), R(0)};
 
     // staged columns of this thread: s_v[q][scol] for q = tid / CPB + (256 / CPB) t
-    constexpr int QS = 256 / CPB;
+    constexpr int QS = 256 / CPB, TV = KC / QS;
+    constexpr int TW = (KC * L::NW + 255) / 256;  // weight-row entries of this thread
     const int scol = tid % CPB, sqc = col_base + scol;
     // columns past the batch read column 0 and stage zeros
     const bool scok = sqc < ncols;
     const int sq = scok ? sqc : 0;
     const double* xcol = reinterpret_cast<const double*>(tab.x[sq / 6]) + 2 * ((sq >> 1) % 3) + (sq & 1);
+    // candidate ids of the chunk of cnt candidates at c0 (clamped to the last one past its
+    // end), its values (component (b, c), real or imaginary part) and its weight rows (zero
+    // past its end): every load of a group is issued before the first use
+    auto load_ids = [&](int c0, int cnt, int (&id)[TV]) {
+#pragma unroll
+        for (int t = 0; t < TV; ++t) id[t] = reg_items[c0 + min(tid / CPB + QS * t, cnt - 1)];
+    };
+    auto load_vals = [&](int cnt, const int (&id)[TV], R (&vv)[TV]) {
+#pragma unroll
+        for (int t = 0; t < TV; ++t)
+            vv[t] = keep_if((R)xcol[6 * (size_t)id[t]], scok && tid / CPB + QS * t < cnt);
+    };
+    auto load_wts = [&](int c0, R (&ww)[TW]) {
+        const int n = min(KC, k1 - c0) * L::NW;
+        const R* w = regw + (size_t)c0 * L::NW;
+#pragma unroll
+        for (int t = 0; t < TW; ++t) ww[t] = keep_if(w[min(tid + 256 * t, n - 1)], tid + 256 * t < n);
+    };
+    int id[TV];
+    R vv[TV], ww[TW];
+    if (PREFETCH && k0 < k1) {
+        load_ids(k0, min(KC, k1 - k0), id);
+        load_vals(min(KC, k1 - k0), id, vv);
+        load_wts(k0, ww);
+        if (k0 + KC < k1) load_ids(k0 + KC, min(KC, k1 - k0 - KC), id);
+    }
     for (int c0 = k0; c0 < k1; c0 += KC) {
         const int cnt = min(KC, k1 - c0);
         __syncthreads();
-        // values: s_v[k][col] = component (b, c), real or imaginary part, of candidate k;
-        // all candidate ids first, then all values (two memory latencies per chunk)
-        int id[KC / QS];
+        if constexpr (PREFETCH) {
 #pragma unroll
-        for (int t = 0; t < KC / QS; ++t) id[t] = reg_items[c0 + min(tid / CPB + QS * t, cnt - 1)];
-        R vv[KC / QS];
+            for (int t = 0; t < TW; ++t)
+                if (tid + 256 * t < KC * L::NW) (&s_w[0][0])[tid + 256 * t] = ww[t];
 #pragma unroll
-        for (int t = 0; t < KC / QS; ++t)
-            vv[t] = keep_if((R)xcol[6 * (size_t)id[t]], scok && tid / CPB + QS * t < cnt);
-        stage_weights<R, RX, ZSB>(&s_w[0][0], cnt, regw + (size_t)c0 * L::NW);
+            for (int t = 0; t < TV; ++t) s_v[tid / CPB + QS * t][scol] = vv[t];
+        } else {
+            int idc[TV];
 #pragma unroll
-        for (int t = 0; t < KC / QS; ++t) s_v[tid / CPB + QS * t][scol] = vv[t];
+            for (int t = 0; t < TV; ++t) idc[t] = reg_items[c0 + min(tid / CPB + QS * t, cnt - 1)];
+            R vc[TV];
+#pragma unroll
+            for (int t = 0; t < TV; ++t)
+                vc[t] = keep_if((R)xcol[6 * (size_t)idc[t]], scok && tid / CPB + QS * t < cnt);
+            stage_weights<R, RX, ZSB>(&s_w[0][0], cnt, regw + (size_t)c0 * L::NW);
+#pragma unroll
+            for (int t = 0; t < TV; ++t) s_v[tid / CPB + QS * t][scol] = vc[t];
+        }
         __syncthreads();
+        if (PREFETCH && c0 + KC < k1) {
+            load_vals(min(KC, k1 - c0 - KC), id, vv);
+            load_wts(c0 + KC, ww);
+            if (c0 + 2 * KC < k1) load_ids(c0 + 2 * KC, min(KC, k1 - c0 - 2 * KC), id);
+        }
         if (wcol0 < ncols && p0 < Zs) {
             const int i = lane & 15;
             for (int ks = 0; ks < cnt; ks += 4) {
@@ -5330,7 +5373,20 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
     if (slab || (!poly && !quads)) {
         const int RX = slab ? (zs_bucket(Zs) <= 10 ? 4 : 2) : 4, RY = kMfmaRY;
         const int arow = slab ? 1 : 2;  // axis of the 16 contiguous rows
-        const int pblk = slab ? Zs : kFullRegionPlanes;
+        int pblk = slab ? Zs : kFullRegionPlanes;
+        if (!slab) {
+            // a region's candidates on average (the particles whose stencil meets it)
+            double cand = (double)Nn;
+            const int ext[3] = {4, kFullRegionPlanes, RY};
+            double nreg8 = 1.0;
+            for (int d = 0; d < 3; ++d) {
+                cand *= std::min(1.0, (double)(ext[d] + W - 1) / S.n[d]);
+                nreg8 *= (S.n[d] + ext[d] - 1) / ext[d];
+            }
+            // dense regions too few to give every SIMD a block: half as many planes each
+            // (15,000 particles, FP64, 6 right-hand sides: an apply 618 -> 563 us)
+            if (cand > 32.0 && nreg8 < 1024.0) pblk = 4;
+        }
         reg_rx = RX;
         reg_full = !slab;
         reg_pblk = pblk;
@@ -5602,7 +5658,7 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
         // region-local separable weights of every (region, candidate) slot, in the row
         // layout of the matrix-core kernels: x at [0, RX), planes at [4, 4 + ZSB), rows at
         // [4 + ZSB4, 4 + ZSB4 + 16); sums over stencil points that fold
-        const int zsb = slab ? zs_bucket(Zs) : kFullRegionPlanes, zsb4 = (zsb + 3) & ~3;
+        const int zsb = slab ? zs_bucket(Zs) : reg_pblk, zsb4 = (zsb + 3) & ~3;
         const int NW = 4 + zsb4 + kMfmaRY;
         const size_t nw = (size_t)std::max(reg_slots, 1) * NW;
         if (nw > d_regw64.n) d_regw64.reserve(nw + nw / 8);
@@ -5811,14 +5867,7 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
     }
     // the matrix-core kernels address the grid with 32-bit element offsets
     const int nreg = reg_nrx * reg_npb * reg_nry;
-    // full grid: the region kernels need enough (region, column group) waves to fill the
-    // GPU; with fewer than a quarter of the per-particle gather's waves (small grids and
-    // batches, e.g. 512 particles on 32^3 with one right-hand side: 64 against 512) the
-    // per-particle path is faster
-    const long long region_waves = (long long)nreg * ((6 * B + 15) / 16);
-    const bool full_ok = reg_full && 4 * region_waves >= (long long)N * ((B + 3) / 4);
-    const bool regions = reg_rx > 0 && (SLAB || full_ok) &&
-                         2ull * (unsigned long long)B * grid_elems_per_rhs() < (1ull << 32);
+    const bool regions = reg_rx > 0 && 2ull * (unsigned long long)B * grid_elems_per_rhs() < (1ull << 32);
     // the matrix-core contractions load whole vectors of two complex when an even row
     // count and stride and an aligned grid keep every pair aligned and both of its rows
     // inside or outside together (16-byte stores in the spread measured slower: kept at
@@ -5827,25 +5876,28 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
     const bool vec = aligned && (SLAB ? (nyp % 2 == 0 && S.n[1] % 2 == 0) : S.n[2] % 2 == 0);
     if (parts & MPM_PART_RECIP) {
         if (phases & 1) {
-            if (regions && !SLAB) {
+            if (regions) {
                 ProfScope ps("spread", s, B);
-                constexpr int CPB = 32;  // SpreadShape<R, ...>::CPB
-                const dim3 gs((unsigned)nreg, (unsigned)((6 * B + CPB - 1) / CPB));
-                ps.kernel("spread_mfma_kernel", {type_name<R>(), "4", std::to_string(kFullRegionPlanes)});
-                hipLaunchKernelGGL((spread_mfma_kernel<R, 4, kFullRegionPlanes>), gs, dim3(256), 0, s, t, B, rg, regw,
-                                   d_reg_start.p, d_reg_items.p, Ni, grid);
-                MPM_HIP(hipGetLastError());
-            } else if (regions) {
-                ProfScope ps("spread", s, B);
-                constexpr int CPB = 32;  // SpreadShape<R, ...>::CPB
-                const dim3 gs((unsigned)nreg, (unsigned)((6 * B + CPB - 1) / CPB));
-    #define MPM_SM(RXV, ZSV)                                                                                          \
-        case ZSV:                                                                                                     \
-            ps.kernel("spread_mfma_kernel", {type_name<R>(), #RXV, #ZSV});                                            \
-            hipLaunchKernelGGL((spread_mfma_kernel<R, RXV, ZSV>), gs, dim3(256), 0, s, t, B, rg, regw, d_reg_start.p, \
-                               d_reg_items.p, Ni, grid);                                                             \
+                // 32 columns per block, or 16 where a batch has no more, and on the full grid
+                // while those blocks are fewer than eight per CU (7001 particles on
+                // 47 x 47 x 48, 5 right-hand sides: 36.2 -> 28.8 us; the slab's regions hold
+                // about one chunk of candidates, which leaves nothing to prefetch)
+                const int cpb = 6 * B <= 16 || (!SLAB && (long long)nreg * ((6 * B + 31) / 32) < 2048) ? 16 : 32;
+                const dim3 gs((unsigned)nreg, (unsigned)((6 * B + cpb - 1) / cpb));
+    #define MPM_SM1(RXV, ZSV, CPBV)                                                                                   \
+        do {                                                                                                          \
+            ps.kernel("spread_mfma_kernel", {type_name<R>(), #RXV, #ZSV, #CPBV});                                     \
+            hipLaunchKernelGGL((spread_mfma_kernel<R, RXV, ZSV, CPBV>), gs, dim3(256), 0, s, t, B, rg, regw,          \
+                               d_reg_start.p, d_reg_items.p, grid);                                                   \
+        } while (0)
+    #define MPM_SM(RXV, ZSV)                   \
+        case ZSV:                              \
+            if (cpb == 16)                     \
+                MPM_SM1(RXV, ZSV, 16);         \
+            else                               \
+                MPM_SM1(RXV, ZSV, 32);         \
             break;
-                switch (zs_bucket(Zs)) {
+                switch (SLAB ? zs_bucket(Zs) : reg_pblk) {
                     MPM_SM(4, 4)
                     MPM_SM(4, 6)
                     MPM_SM(4, 8)
@@ -5857,6 +5909,7 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
                         throw Error(MPM_ERR_RUNTIME, "slab size out of range");
                 }
     #undef MPM_SM
+    #undef MPM_SM1
                 MPM_HIP(hipGetLastError());
             } else {
                 ProfScope ps("spread", s, B);
@@ -6044,7 +6097,17 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
     }
     if (!(phases & 4)) return;
     const R* part = nullptr;
-    if (regions && (parts & MPM_PART_RECIP)) {
+    // The contraction as part of the per-particle gather instead of on the regions: for
+    // batches that take that kernel anyway (B < 4, below) and give it no more than a wave per
+    // SIMD (launches and latency decide; 400 particles on the slab, 3 right-hand sides: 76
+    // against 85 us an apply), and on the full
+    // grid with stencils of at most 5 points per axis (125 voxels per particle are cheaper
+    // to gather than the zero-padded products of its regions: 30,000 particles, 10 right-hand
+    // sides 830 against 893 us; with 7 points 6 right-hand sides of 15,000 particles take
+    // 563 on the regions, 644 gathered) or one right-hand side and few regions
+    const bool per_particle = (B < 4 && N <= 1024) ||
+                              (!SLAB && (S.width <= 5 || (B == 1 && 4ll * nreg < (long long)N)));
+    if (regions && !per_particle && (parts & MPM_PART_RECIP)) {
         ProfScope ps("contract", s, B);
         // column groups of 16 per block: 4 when there are enough right-hand sides,
         // else fewer, with the region's planes split over the remaining waves; slab
@@ -6054,7 +6117,25 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
         const dim3 gs((unsigned)nreg, (unsigned)((ngrp + ncg - 1) / ncg));
         const dim3 gn((unsigned)nreg, (unsigned)ngrp);
         R* pbuf = reinterpret_cast<R*>(d_partial64.p);  // sized for FP64, shared by FP32
-        if (!SLAB && vec) {
+        // full grid with more than 32 candidates per region on average: four waves per region
+        // and column group take a candidate block each (30,000 particles, 4 right-hand sides:
+        // an apply 814 us, 839 with contract_full_mfma_kernel, 984 with contract_mfma_kernel)
+        if (!SLAB && (reg_pblk == 4 || reg_slots > 32ll * nreg)) {
+#define MPM_CF(ZSV, VECV)                                                                                      \
+    do {                                                                                                       \
+        ps.kernel("contract_nb_mfma_kernel", {type_name<R>(), "4", #ZSV, #VECV});                              \
+        hipLaunchKernelGGL((contract_nb_mfma_kernel<R, 4, ZSV, VECV>), gn, dim3(256), 0, s, B, rg, regw,       \
+                           d_reg_start.p, d_reg_items.p, Ni, grid, pbuf);                                      \
+    } while (0)
+            if (reg_pblk == 4) {
+                if (vec) MPM_CF(4, true);
+                else MPM_CF(4, false);
+            } else {
+                if (vec) MPM_CF(8, true);
+                else MPM_CF(8, false);
+            }
+#undef MPM_CF
+        } else if (!SLAB && vec) {
             ps.kernel("contract_full_mfma_kernel",
                       {type_name<R>(), "4", std::to_string(kFullRegionPlanes), std::to_string(kFullContractNB)});
             const int nitems = nreg * ngrp;
