@@ -50,7 +50,7 @@
 #include <numeric>
 #include <thread>
 
-#include "mpm_internal.h"
+#include "region_mfma.h"
 
 namespace mpm {
 
@@ -744,16 +744,6 @@ struct FftPlans {
 // ---------------------------------------------------------------------------
 // Device kernels
 // ---------------------------------------------------------------------------
-template <typename R>
-struct C2;
-template <>
-struct C2<double> {
-    using T = double2;
-};
-template <>
-struct C2<float> {
-    using T = float2;
-};
 
 // ---------------------------------------------------------------------------
 // Built-in batched line FFT: unnormalised complex DFTs of length n along one
@@ -1717,12 +1707,6 @@ struct LineFft {
 // k-space Green's tensor at wave vector (Gx - kbx, Gy - kby, Gz): (k^x, k^y, k^z, sc)
 // with sc = 9 (sin k / k - cos k)^2 exp(-(k^2 - sum_d G_d^2 eta_d) / (4 xi^2)) / k^4 / V
 // and zero at k = 0.  monodisperse_ewald_electric_field.cu:1300-1404.
-struct KParams {
-    int nx, ny, nz;
-    int tcols;  // slab columns ordered ky * nxp + kx (else kx * ny + ky)
-    int nxp;    // row stride of the transposed columns (nx rounded up to whole cache lines)
-    double Lx, Ly, Lz, kbx, kby, xi, etax, etay, etaz, invV;
-};
 
 // (kx, ky) of a slab column; ix >= nx marks a padding column
 __device__ inline void col_xy(const KParams& q, int col, int& ix, int& iy) {
@@ -1803,6 +1787,9 @@ struct SpreadGeom {
     int nyp;            // slab row stride (ny rounded up to whole cache lines when padded)
 };
 
+constexpr size_t kMaxFusedLds = 64 * 1024;  // LDS of one xtoeplitz_kernel block
+// Radius classes of the polydisperse operator up to which pair tables are built.
+constexpr int kPolyTableClasses = 64;
 constexpr int kChunk = 64;       // particles staged in LDS per round
 constexpr int kMaxWidth = 13;    // stencil points per axis
 constexpr int kListMax = 12;     // candidate bins per axis
@@ -2050,774 +2037,6 @@ __global__ __launch_bounds__(256) void scale_kernel(typename C2<R>::T* __restric
             o.x = dr * kz;
             o.y = di * kz;
             gp[2 * V] = o;
-        }
-    }
-}
-
-// ---- spread on the matrix cores ----
-//
-// For a region of RX x (planes) x 16 rows (slab: RX x 16 y over all slab planes;
-// full grid: 4 x 8 y-planes x 16 z, see RegionGeom) and 16 real columns
-// q = 6 b + 2 c + (0: real, 1: imaginary) of the right-hand sides,
-//   grid^T[q][voxel] = sum_k V[k][q] W[k][voxel],
-//   W[k][(x, plane, row)] = wx_k(x) wp_k(plane) wr_k(row)
-// over the candidate particles k of the region (every particle whose stencil
-// footprint meets it, in ascending id order), one 16x16x4 MFMA (FP32 or FP64)
-// per four candidates and (x, plane) pair: A = V^T (16 columns x 4 candidates),
-// B = W^T (4 candidates x 16 consecutive rows).  The region-local separable weights
-// (stencil folding on small grids included) are staged per candidate chunk in
-// LDS.  Every voxel is written exactly once, without atomics; the sum order is
-// fixed (deterministic).
-constexpr int kMfmaRY = 16;    // y voxels per region (the MFMA N dimension)
-constexpr size_t kMaxFusedLds = 64 * 1024;  // LDS of one xtoeplitz_kernel block
-// Radius classes of the polydisperse operator up to which pair tables are built.
-constexpr int kPolyTableClasses = 64;
-constexpr int kMfmaKC = 64;    // candidates staged per chunk
-// Planes (y) per region on the full grid and candidate blocks of 16 per chunk of
-// its contraction: 4 x 8 x 16-voxel regions, about 28 candidates each in a
-// packing of volume fraction 0.3 with 9-point stencils on a 256^3 grid.
-constexpr int kFullRegionPlanes = 8;
-constexpr int kFullContractNB = 2;
-
-typedef float mpm_f32x4 __attribute__((ext_vector_type(4)));
-typedef double mpm_f64x4 __attribute__((ext_vector_type(4)));
-
-// 16x16x4 MFMA: lane l holds A[l % 16][l / 16] and B[l / 16][l % 16]; its
-// accumulator entry r is D[drow(l / 16, r)][l % 16], with drow = 4 g + r for
-// FP32 and g + 4 r for FP64 (measured on gfx950).  rowcol(i) is the real
-// column a spread wave feeds into A row i so that accumulator entries (0, 1)
-// and (2, 3) of every lane are the real and imaginary parts of one complex
-// column: complex column 2 g + h of the wave sits in entries (2 h, 2 h + 1).
-template <typename R>
-struct Mfma;
-template <>
-struct Mfma<float> {
-    using V4 = mpm_f32x4;
-    static __device__ __forceinline__ V4 mac(float a, float b, V4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int drow(int g, int r) { return 4 * g + r; }
-    static __device__ __forceinline__ int rowcol(int i) { return i; }
-};
-template <>
-struct Mfma<double> {
-    using V4 = mpm_f64x4;
-    static __device__ __forceinline__ V4 mac(double a, double b, V4 c) {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int drow(int g, int r) { return g + 4 * r; }
-    // row i = g + 4 r -> complex column 2 g + r / 2, part r % 2
-    static __device__ __forceinline__ int rowcol(int i) { return 2 * (2 * (i & 3) + (i >> 3)) + ((i >> 2) & 1); }
-};
-
-// Block shape of spread_mfma_kernel: 4 waves = (CPB / 16 column groups) x
-// (plane groups of ZH planes).  CPB = 32 splits the planes over two waves, CPB = 16 over
-// four: fewer accumulators per wave, more blocks, and no idle column group when a batch
-// has no more than 16 real columns.
-template <int ZSB, int CPB>
-struct SpreadShape {
-    static constexpr int NPG = 4 / (CPB / 16);
-    static constexpr int ZH = (ZSB + NPG - 1) / NPG;
-};
-
-// Region-local separable weights of a candidate, one LDS row per candidate:
-// x weights at [0, RX), slab-plane weights at [4, 4 + ZSB), y weights at
-// [4 + ZSB4, 4 + ZSB4 + 16) (ZSB4 = ZSB rounded up to 4), so that 4-wide
-// groups start on 16-byte boundaries.  A voxel's weight sums the stencil points
-// that land on it (stencils fold onto themselves on grids narrower than the
-// stencil).
-template <int RX, int ZSB>
-struct RegionW {
-    static constexpr int ZSB4 = (ZSB + 3) & ~3;
-    static constexpr int X = 0, Z = 4, Y = 4 + ZSB4;
-    static constexpr int NW = Y + kMfmaRY;
-};
-
-// Copies the precomputed region-local weight rows of a chunk of cnt <= KC
-// candidates into LDS (zero rows past cnt) and ends with a barrier.
-// v where c holds, else +0, by a bit mask rather than a select: the compiler turns a
-// select of a loaded value into a branch around the load, which then waits for
-// the load at the branch's end.
-__device__ __forceinline__ float keep_if(float v, bool c) {
-    return __uint_as_float(__float_as_uint(v) & (c ? 0xffffffffu : 0u));
-}
-__device__ __forceinline__ double keep_if(double v, bool c) {
-    return __longlong_as_double(__double_as_longlong(v) & (c ? -1LL : 0LL));
-}
-
-// Blocks of 256 threads; every load is issued before the first store (one memory
-// latency per chunk, not one per element).
-template <typename R, int RX, int ZSB, int KC = kMfmaKC>
-__device__ inline void stage_weights(R* s_w, int cnt, const R* __restrict__ regw) {
-    using L = RegionW<RX, ZSB>;
-    constexpr int T = (KC * L::NW + 255) / 256;
-    const int n = cnt * L::NW;
-    R v[T];
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        const int e = (int)threadIdx.x + 256 * t;
-        v[t] = e < n ? regw[e] : R(0);
-    }
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        const int e = (int)threadIdx.x + 256 * t;
-        if (e < KC * L::NW) s_w[e] = v[t];
-    }
-    __syncthreads();
-}
-
-// Plane loop of the matrix-core contractions, software-pipelined over two operand
-// buffers: the loads of the next plane are in flight while the current plane's
-// products run.  load(p, buf) issues plane p's loads into buf, mma(buf, p)
-// consumes them; planes first, first + step, ... below end.  The loop body has no
-// branch between a load and its use (a branch would let the compiler sink the
-// loads next to their use): the last pair loads its second plane again, and an
-// odd plane count ends with one more product.  Scheduling barriers keep each group
-// of loads whole and ahead of the other buffer's products, so that the products
-// wait only for their own (older) loads.
-template <typename Buf, typename LoadF, typename MmaF>
-__device__ __forceinline__ void plane_pipeline(int first, int step, int end, Buf& ga, Buf& gb, LoadF&& load,
-                                               MmaF&& mma) {
-    if (first >= end) return;
-    const int n = (end - first + step - 1) / step;
-    const int last = first + (n - 1) * step;
-    load(first, ga);
-    int i = 0, p = first;
-    for (; i + 1 < n; i += 2, p += 2 * step) {
-        __builtin_amdgcn_sched_barrier(0);
-        load(p + step, gb);
-        __builtin_amdgcn_sched_barrier(0);
-        mma(ga, p);
-        __builtin_amdgcn_sched_barrier(0);
-        load(min(p + 2 * step, last), ga);
-        __builtin_amdgcn_sched_barrier(0);
-        mma(gb, p + step);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    if (i < n) mma(ga, p);
-}
-
-// Vector form of the contractions' grid operands: the four voxels a lane feeds into
-// the four products of a plane and x are rows 4 r + u (r = lane / 16, u = 0..3) of
-// its real column (even lane) or imaginary column (odd lane); the two lanes of a
-// complex column load rows (4 r, 4 r + 1) and (4 r + 2, 4 r + 3) as whole complex
-// pairs v = (re, im, re, im) and swap halves with a neighbour-lane move, so that one
-// 16-byte load per lane reads the 16 rows of eight complex components (one whole
-// 128-byte line each for FP32).  g receives rows 4 r + u of this lane's part.
-template <typename R, typename V4>
-__device__ __forceinline__ void pair_rows(const V4& v, int part, R (&g)[4]) {
-    const R s0 = part ? v[0] : v[1], s1 = part ? v[2] : v[3];
-    const R t0 = __shfl_xor(s0, 1, 64), t1 = __shfl_xor(s1, 1, 64);
-    g[0] = part ? t0 : v[0];
-    g[1] = part ? t1 : v[2];
-    g[2] = part ? v[1] : t0;
-    g[3] = part ? v[3] : t1;
-}
-
-// Where the regions sit in a grid buffer.  A region is RX consecutive x, up to
-// pblk consecutive planes and 16 consecutive rows, rows contiguous in memory:
-// in the slab layout the planes are the occupied z-planes (all in one region)
-// and the rows y; on the full grid the planes are y (blocks of pblk) and the
-// rows z.  Regions are numbered (x block, plane block, row block), row block
-// fastest.  Strides are in complex elements.
-struct RegionGeom {
-    int nx, nrow, nplane;  // extents along x, rows, planes
-    int nrr, npb, pblk;    // row blocks, plane blocks, planes per region
-    unsigned xs, ps, cs;   // strides of x, plane, component (b, c)
-};
-
-struct RegionAt {
-    int x0, plane0, row0, np;  // origin and number of planes present
-};
-
-template <int RX>
-__device__ inline RegionAt region_at(const RegionGeom& rg, int reg) {
-    const int per_x = rg.npb * rg.nrr;
-    const int rx = reg / per_x, rem = reg - rx * per_x;
-    const int pb = rem / rg.nrr, rr = rem - pb * rg.nrr;
-    RegionAt a;
-    a.x0 = rx * RX;
-    a.plane0 = pb * rg.pblk;
-    a.row0 = rr * kMfmaRY;
-    a.np = min(rg.pblk, rg.nplane - a.plane0);
-    return a;
-}
-
-// FP32: held to 128 registers (four waves per SIMD; at the compiler's 140 three, and the
-// N = 4000 monolayer's 1272 blocks took 1.7 rounds instead of 1.2: 39.4 against 37.0 us).
-//
-// CPB = 16 is the form for few blocks (spread_cpb): there a region's candidates come in
-// several chunks and nothing else hides their loads, so the next chunk's values and
-// weights are fetched while the current chunk's products run.
-template <typename R, int RX, int ZSB, int CPB>
-__global__ __launch_bounds__(256, sizeof(R) == 4 ? 4 : 2) void spread_mfma_kernel(SlotTable tab, int B, RegionGeom rg,
-                                                          const R* __restrict__ regw,
-                                                          const int* __restrict__ reg_start,
-                                                          const int* __restrict__ reg_items,
-                                                          typename C2<R>::T* __restrict__ out) {
-    using CT = typename C2<R>::T;
-    using M = Mfma<R>;
-    using Sh = SpreadShape<ZSB, CPB>;
-    constexpr int KC = kMfmaKC, ZH = Sh::ZH;
-    constexpr bool PREFETCH = CPB == 16;
-    using L = RegionW<RX, ZSB>;
-    __shared__ R s_v[KC][CPB + 1];
-    __shared__ __align__(16) R s_w[KC][L::NW];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int cg = wave % (CPB / 16), pg = wave / (CPB / 16);
-    const int reg = blockIdx.x;
-    const RegionAt ra = region_at<RX>(rg, reg);
-    const int x0 = ra.x0, y0 = ra.row0;
-    const int col_base = blockIdx.y * CPB;
-    const int wcol0 = col_base + cg * 16;
-    const int ncols = 6 * B;
-    const int Zs = ra.np;    // planes of this region
-    const int p0 = pg * ZH;  // this wave's planes [p0, p0 + ZH) of the region
-    const int k0 = reg_start[reg], k1 = reg_start[reg + 1];
-
-    typename M::V4 acc[RX][ZH];
-#pragma unroll
-    for (int xi = 0; xi < RX; ++xi)
-#pragma unroll
-        for (int p = 0; p < ZH; ++p) acc[xi][p] = typename M::V4{R(0), R(0), R(0), R(0)};
-
-    // staged columns of this thread: s_v[q][scol] for q = tid / CPB + (256 / CPB) t
-    constexpr int QS = 256 / CPB, TV = KC / QS;
-    constexpr int TW = (KC * L::NW + 255) / 256;  // weight-row entries of this thread
-    const int scol = tid % CPB, sqc = col_base + scol;
-    // columns past the batch read column 0 and stage zeros
-    const bool scok = sqc < ncols;
-    const int sq = scok ? sqc : 0;
-    const double* xcol = reinterpret_cast<const double*>(tab.x[sq / 6]) + 2 * ((sq >> 1) % 3) + (sq & 1);
-    // candidate ids of the chunk of cnt candidates at c0 (clamped to the last one past its
-    // end), its values (component (b, c), real or imaginary part) and its weight rows (zero
-    // past its end): every load of a group is issued before the first use
-    auto load_ids = [&](int c0, int cnt, int (&id)[TV]) {
-#pragma unroll
-        for (int t = 0; t < TV; ++t) id[t] = reg_items[c0 + min(tid / CPB + QS * t, cnt - 1)];
-    };
-    auto load_vals = [&](int cnt, const int (&id)[TV], R (&vv)[TV]) {
-#pragma unroll
-        for (int t = 0; t < TV; ++t)
-            vv[t] = keep_if((R)xcol[6 * (size_t)id[t]], scok && tid / CPB + QS * t < cnt);
-    };
-    auto load_wts = [&](int c0, R (&ww)[TW]) {
-        const int n = min(KC, k1 - c0) * L::NW;
-        const R* w = regw + (size_t)c0 * L::NW;
-#pragma unroll
-        for (int t = 0; t < TW; ++t) ww[t] = keep_if(w[min(tid + 256 * t, n - 1)], tid + 256 * t < n);
-    };
-    int id[TV];
-    R vv[TV], ww[TW];
-    if (PREFETCH && k0 < k1) {
-        load_ids(k0, min(KC, k1 - k0), id);
-        load_vals(min(KC, k1 - k0), id, vv);
-        load_wts(k0, ww);
-        if (k0 + KC < k1) load_ids(k0 + KC, min(KC, k1 - k0 - KC), id);
-    }
-    for (int c0 = k0; c0 < k1; c0 += KC) {
-        const int cnt = min(KC, k1 - c0);
-        __syncthreads();
-        if constexpr (PREFETCH) {
-#pragma unroll
-            for (int t = 0; t < TW; ++t)
-                if (tid + 256 * t < KC * L::NW) (&s_w[0][0])[tid + 256 * t] = ww[t];
-#pragma unroll
-            for (int t = 0; t < TV; ++t) s_v[tid / CPB + QS * t][scol] = vv[t];
-        } else {
-            int idc[TV];
-#pragma unroll
-            for (int t = 0; t < TV; ++t) idc[t] = reg_items[c0 + min(tid / CPB + QS * t, cnt - 1)];
-            R vc[TV];
-#pragma unroll
-            for (int t = 0; t < TV; ++t)
-                vc[t] = keep_if((R)xcol[6 * (size_t)idc[t]], scok && tid / CPB + QS * t < cnt);
-            stage_weights<R, RX, ZSB>(&s_w[0][0], cnt, regw + (size_t)c0 * L::NW);
-#pragma unroll
-            for (int t = 0; t < TV; ++t) s_v[tid / CPB + QS * t][scol] = vc[t];
-        }
-        __syncthreads();
-        if (PREFETCH && c0 + KC < k1) {
-            load_vals(min(KC, k1 - c0 - KC), id, vv);
-            load_wts(c0 + KC, ww);
-            if (c0 + 2 * KC < k1) load_ids(c0 + 2 * KC, min(KC, k1 - c0 - 2 * KC), id);
-        }
-        if (wcol0 < ncols && p0 < Zs) {
-            const int i = lane & 15;
-            for (int ks = 0; ks < cnt; ks += 4) {
-                const int kq = ks + (lane >> 4);  // rows >= cnt hold zeros
-                const R a = s_v[kq][cg * 16 + M::rowcol(i)];
-                const R wy = s_w[kq][L::Y + i];
-                R wx[RX], wz[ZH];
-#pragma unroll
-                for (int xi = 0; xi < RX; ++xi) wx[xi] = s_w[kq][L::X + xi] * wy;
-#pragma unroll
-                for (int p = 0; p < ZH; ++p) wz[p] = (p0 + p < ZSB) ? s_w[kq][L::Z + p0 + p] : R(0);
-                // planes past Zs carry zero weights: no branch around the accumulators
-#pragma unroll
-                for (int p = 0; p < ZH; ++p) {
-#pragma unroll
-                    for (int xi = 0; xi < RX; ++xi) acc[xi][p] = M::mac(a, wx[xi] * wz[p], acc[xi][p]);
-                }
-            }
-        }
-    }
-    // lane holds complex columns 2 (lane >> 4) + h of the wave (entries 2 h, 2 h + 1)
-    // at row y0 + (lane & 15)
-    const int y = y0 + (lane & 15);
-    if (y >= rg.nrow || wcol0 >= ncols) return;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int qc = wcol0 + 4 * (lane >> 4) + 2 * h;
-        if (qc >= ncols) continue;
-        const int b = qc / 6, c = (qc >> 1) % 3;
-        CT* o = out + ((size_t)b * 3 + c) * rg.cs + (size_t)ra.plane0 * rg.ps + y;
-#pragma unroll
-        for (int xi = 0; xi < RX; ++xi) {
-            const int x = x0 + xi;
-            if (x >= rg.nx) continue;
-#pragma unroll
-            for (int p = 0; p < ZH; ++p)
-                if (p0 + p < Zs) {
-                    CT v;
-                    v.x = acc[xi][p][2 * h];
-                    v.y = acc[xi][p][2 * h + 1];
-                    o[(size_t)(p0 + p) * rg.ps + (size_t)x * rg.xs] = v;
-                }
-        }
-    }
-}
-
-// ---- contraction on the matrix cores ----
-//
-// The transpose of spread_mfma_kernel over the same regions: for the candidate
-// particles k of a region and 16 real columns q,
-//   D[k][q] = sum_{voxels v of the region} W[k][v] G[v][q],
-// one 16x16x4 MFMA per four voxels and 16 candidates (A = W, B = G), every
-// loaded operand feeding all candidate blocks.  Each wave reads its B operands
-// straight from the grid: lane (j, u) loads column j at row 4 u + (lane >> 4),
-// so the four loads of a 16-voxel row consume whole cache lines, or with VEC
-// (pair_rows) one 16-byte complex pair per lane and x; waves run without
-// barriers after the one weight-staging step.  D goes to the particle's
-// slot of the region (the CSR position of the pair); the per-particle sum over
-// its regions happens in the finish step, in a fixed order.
-template <typename R, int RX, int ZSB, int NB, bool VEC>
-__global__ __launch_bounds__(256, sizeof(R) == 4 ? 3 : 2) void contract_mfma_kernel(int B, RegionGeom rg,
-                                                                                    const R* __restrict__ regw,
-                                                            const int* __restrict__ reg_start,
-                                                            const int* __restrict__ reg_items, int N,
-                                                            const typename C2<R>::T* __restrict__ grid,
-                                                            R* __restrict__ partial, int ncg) {
-    using M = Mfma<R>;
-    using V4 = typename M::V4;
-    constexpr int KC = 16 * NB;  // candidates per chunk, in NB blocks of 16
-    using L = RegionW<RX, ZSB>;
-    __shared__ __align__(16) R s_w[KC][L::NW];
-    __shared__ V4 s_red[4][NB][64];  // per-wave partial accumulators
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // 4 waves = ncg column groups x (4 / ncg) plane groups
-    const int npg = 4 / ncg, cg = wave % ncg, pg = wave / ncg;
-    const int reg = blockIdx.x;
-    const RegionAt ra = region_at<RX>(rg, reg);
-    const int x0 = ra.x0, y0 = ra.row0;
-    const int wcol0 = (blockIdx.y * ncg + cg) * 16;
-    const int ncols = 6 * B;
-    const bool active = wcol0 < ncols;
-    const int Zs = ra.np;  // planes of this region
-    const unsigned plane = rg.ps;
-    const int k0 = reg_start[reg], k1 = reg_start[reg + 1];
-
-    // this lane's B-operand column and its rows of the region, as 32-bit offsets
-    // (in R) from the uniform grid base: the launch keeps 6 B x (complex per
-    // component) below 2^32
-    const R* gf = reinterpret_cast<const R*>(grid);
-    const int qc = wcol0 + (lane & 15);
-    const bool cvalid = qc < ncols;
-    // column offset at the region origin (cbase, an in-grid voxel of every plane of the
-    // region) and at this lane's row; bit 4 xi + u of vmask: (x0 + xi, y0 + 4 u + lane / 16)
-    // inside the grid.  VEC (pair_rows): the lane's complex pair at rows y0 + 4 r + 2 part
-    // and the next, bit xi of vmask: (x0 + xi, y0 + 4 r + 2 part) inside; even rows keep
-    // both rows of a pair inside together.
-    const int r = lane >> 4, part = lane & 1;
-    unsigned cbase = 0, coff = 0, vmask = 0;
-    if (cvalid) {
-        const int b = qc / 6, c = (qc >> 1) % 3;
-        cbase = 2u * (unsigned)(b * 3 + c) * rg.cs + (VEC ? 0u : (unsigned)(qc & 1)) +
-                2u * ((unsigned)ra.plane0 * rg.ps + (unsigned)x0 * rg.xs + (unsigned)y0);
-        if (VEC) {
-            coff = cbase + 2u * (unsigned)(4 * r + 2 * part);
-#pragma unroll
-            for (int xi = 0; xi < RX; ++xi)
-                if (x0 + xi < rg.nx && y0 + 4 * r + 2 * part < rg.nrow) vmask |= 1u << xi;
-        } else {
-            coff = cbase + 2u * (unsigned)(lane >> 4);
-#pragma unroll
-            for (int xi = 0; xi < RX; ++xi)
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (x0 + xi < rg.nx && y0 + 4 * u + (lane >> 4) < rg.nrow) vmask |= 1u << (4 * xi + u);
-        }
-    }
-    const unsigned xstep = 2u * rg.xs;
-
-    for (int c0 = k0; c0 < k1; c0 += KC) {
-        const int cnt = min(KC, k1 - c0);
-        __syncthreads();
-        stage_weights<R, RX, ZSB, KC>(&s_w[0][0], cnt, regw + (size_t)c0 * L::NW);
-        V4 acc[NB];
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) acc[nb] = V4{R(0), R(0), R(0), R(0)};
-        if (active) {
-            // per-lane weights: candidate k = 16 nb + (lane & 15) at x = x0 + xi and rows
-            // y0 + 4 u + r (VEC: y0 + 4 r + u)
-            R wyl[NB][4], wxl[NB][RX];
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                const int k = nb * 16 + (lane & 15);
-#pragma unroll
-                for (int u = 0; u < 4; ++u) wyl[nb][u] = s_w[k][L::Y + (VEC ? 4 * r + u : 4 * u + r)];
-#pragma unroll
-                for (int xi = 0; xi < RX; ++xi) wxl[nb][xi] = s_w[k][L::X + xi];
-            }
-            if constexpr (VEC) {
-                struct PlaneBuf {
-                    V4 g[RX];
-                };
-                auto load_plane = [&](int p, PlaneBuf& dst) {
-                    const unsigned poff = coff + 2u * (unsigned)p * plane, pin = cbase + 2u * (unsigned)p * plane;
-#pragma unroll
-                    for (int xi = 0; xi < RX; ++xi) {
-                        const bool in = (vmask >> xi) & 1u;
-                        dst.g[xi] = *reinterpret_cast<const V4*>(gf + (in ? poff + xi * xstep : pin));
-                    }
-                };
-                auto mma = [&](PlaneBuf& pb, int p) {
-                    R wz[NB];
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb) wz[nb] = s_w[nb * 16 + (lane & 15)][L::Z + p];
-#pragma unroll
-                    for (int xi = 0; xi < RX; ++xi) {
-                        R gv[4];
-                        pair_rows<R>(pb.g[xi], part, gv);
-#pragma unroll
-                        for (int nb = 0; nb < NB; ++nb) {
-                            const R wxz = wxl[nb][xi] * wz[nb];
-#pragma unroll
-                            for (int u = 0; u < 4; ++u) acc[nb] = M::mac(wyl[nb][u] * wxz, gv[u], acc[nb]);
-                        }
-                    }
-                };
-                PlaneBuf ga, gb;
-                plane_pipeline(pg, npg, Zs, ga, gb, load_plane, mma);
-            } else {
-            // the next plane's operands are loaded while this plane's products run
-            auto load_plane = [&](int p, R (&dst)[RX][4]) {
-                const unsigned poff = coff + 2u * (unsigned)p * plane, pin = cbase + 2u * (unsigned)p * plane;
-#pragma unroll
-                for (int xi = 0; xi < RX; ++xi)
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        // lanes outside the grid read the region's origin instead, which
-                        // meets a zero weight (the weight rows are zero past the grid's
-                        // edges): no branch around the load and no use of it before the
-                        // products
-                        const bool in = (vmask >> (4 * xi + u)) & 1u;
-                        dst[xi][u] = gf[in ? poff + xi * xstep + 8u * u : pin];
-                    }
-            };
-            auto mma = [&](R (&gv)[RX][4], int p) {
-                R wz[NB];
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb) wz[nb] = s_w[nb * 16 + (lane & 15)][L::Z + p];
-                // every candidate block, filled or not (rows past cnt hold zero weights):
-                // a branch here would make the compiler copy the accumulators around it
-#pragma unroll
-                for (int xi = 0; xi < RX; ++xi)
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb) {
-                        const R wxz = wxl[nb][xi] * wz[nb];
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) acc[nb] = M::mac(wyl[nb][u] * wxz, gv[xi][u], acc[nb]);
-                    }
-            };
-            R ga[RX][4], gb[RX][4];
-            plane_pipeline(pg, npg, Zs, ga, gb, load_plane, mma);
-            }
-        }
-        // plane groups of one column group are summed in plane-group order
-        if (npg > 1) {
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) s_red[wave][nb][lane] = acc[nb];
-            __syncthreads();
-            if (pg == 0) {
-                for (int q = 1; q < npg; ++q)
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb) acc[nb] += s_red[q * ncg + cg][nb][lane];
-            }
-        }
-        // lane holds D[16 nb + drow(lane >> 4, r)][lane & 15]
-        if (pg == 0 && cvalid) {
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int k = nb * 16 + M::drow(lane >> 4, q);
-                    if (k < cnt) partial[(size_t)(c0 + k) * ncols + qc] = acc[nb][q];
-                }
-        }
-    }
-}
-
-// Narrow-batch variant of the contraction: a block is one column group of 16
-// and four waves, one per block of 16 candidates, so a wave holds few registers
-// and, when only one or two column groups exist, the region's candidates still
-// spread over four waves; the next plane's operands are loaded while the
-// current plane's products run.
-template <typename R, int RX, int ZSB, bool VEC>
-__global__ __launch_bounds__(256) void contract_nb_mfma_kernel(int B, RegionGeom rg, const R* __restrict__ regw,
-                                                               const int* __restrict__ reg_start,
-                                                               const int* __restrict__ reg_items, int N,
-                                                               const typename C2<R>::T* __restrict__ grid,
-                                                               R* __restrict__ partial) {
-    using M = Mfma<R>;
-    using V4 = typename M::V4;
-    constexpr int KC = kMfmaKC;
-    using L = RegionW<RX, ZSB>;
-    __shared__ __align__(16) R s_w[KC][L::NW];
-    const int tid = threadIdx.x, lane = tid & 63, nb = tid >> 6;  // candidate block of this wave
-    const int reg = blockIdx.x;
-    const RegionAt ra = region_at<RX>(rg, reg);
-    const int x0 = ra.x0, y0 = ra.row0;
-    const int wcol0 = blockIdx.y * 16;
-    const int ncols = 6 * B;
-    const int Zs = ra.np;  // planes of this region
-    const unsigned plane = rg.ps;
-    const int k0 = reg_start[reg], k1 = reg_start[reg + 1];
-    const R* gf = reinterpret_cast<const R*>(grid);
-    const int qc = wcol0 + (lane & 15);
-    const bool cvalid = qc < ncols;
-    // column offset at the region origin (cbase, an in-grid voxel of every plane of the
-    // region) and at this lane's row; bit 4 xi + u of vmask: (x0 + xi, y0 + 4 u + lane / 16)
-    // inside the grid.  VEC (pair_rows): the lane's complex pair at rows y0 + 4 r + 2 part
-    // and the next, bit xi of vmask: (x0 + xi, y0 + 4 r + 2 part) inside.
-    const int r = lane >> 4, part = lane & 1;
-    unsigned cbase = 0, coff = 0, vmask = 0;
-    if (cvalid) {
-        const int b = qc / 6, c = (qc >> 1) % 3;
-        cbase = 2u * (unsigned)(b * 3 + c) * rg.cs + (VEC ? 0u : (unsigned)(qc & 1)) +
-                2u * ((unsigned)ra.plane0 * rg.ps + (unsigned)x0 * rg.xs + (unsigned)y0);
-        if (VEC) {
-            coff = cbase + 2u * (unsigned)(4 * r + 2 * part);
-#pragma unroll
-            for (int xi = 0; xi < RX; ++xi)
-                if (x0 + xi < rg.nx && y0 + 4 * r + 2 * part < rg.nrow) vmask |= 1u << xi;
-        } else {
-            coff = cbase + 2u * (unsigned)(lane >> 4);
-#pragma unroll
-            for (int xi = 0; xi < RX; ++xi)
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (x0 + xi < rg.nx && y0 + 4 * u + (lane >> 4) < rg.nrow) vmask |= 1u << (4 * xi + u);
-        }
-    }
-    const unsigned xstep = 2u * rg.xs;
-    for (int c0 = k0; c0 < k1; c0 += KC) {
-        const int cnt = min(KC, k1 - c0);
-        __syncthreads();
-        stage_weights<R, RX, ZSB>(&s_w[0][0], cnt, regw + (size_t)c0 * L::NW);
-        if (nb * 16 >= cnt) continue;  // no candidates for this wave (no barrier follows in this chunk)
-        const int k = nb * 16 + (lane & 15);
-        R wyl[4], wxl[RX];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) wyl[u] = s_w[k][L::Y + (VEC ? 4 * r + u : 4 * u + r)];
-#pragma unroll
-        for (int xi = 0; xi < RX; ++xi) wxl[xi] = s_w[k][L::X + xi];
-        V4 acc = V4{R(0), R(0), R(0), R(0)};
-        if constexpr (VEC) {
-            struct PlaneBuf {
-                V4 g[RX];
-            };
-            auto load_plane = [&](int p, PlaneBuf& dst) {
-                const unsigned poff = coff + 2u * (unsigned)p * plane, pin = cbase + 2u * (unsigned)p * plane;
-#pragma unroll
-                for (int xi = 0; xi < RX; ++xi) {
-                    const bool in = (vmask >> xi) & 1u;
-                    dst.g[xi] = *reinterpret_cast<const V4*>(gf + (in ? poff + xi * xstep : pin));
-                }
-            };
-            auto mma = [&](PlaneBuf& pb, int p) {
-                const R wz = s_w[k][L::Z + p];
-#pragma unroll
-                for (int xi = 0; xi < RX; ++xi) {
-                    R gv[4];
-                    pair_rows<R>(pb.g[xi], part, gv);
-                    const R wxz = wxl[xi] * wz;
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) acc = M::mac(wyl[u] * wxz, gv[u], acc);
-                }
-            };
-            PlaneBuf ga, gb;
-            plane_pipeline(0, 1, Zs, ga, gb, load_plane, mma);
-        } else {
-            auto load_plane = [&](int p, R (&dst)[RX][4]) {
-                const unsigned poff = coff + 2u * (unsigned)p * plane, pin = cbase + 2u * (unsigned)p * plane;
-#pragma unroll
-                for (int xi = 0; xi < RX; ++xi)
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        // lanes outside the grid read the region's origin, which meets a zero weight
-                        const bool in = (vmask >> (4 * xi + u)) & 1u;
-                        dst[xi][u] = gf[in ? poff + xi * xstep + 8u * u : pin];
-                    }
-            };
-            auto mma = [&](R (&gv)[RX][4], int p) {
-                const R wz = s_w[k][L::Z + p];
-#pragma unroll
-                for (int xi = 0; xi < RX; ++xi) {
-                    const R wxz = wxl[xi] * wz;
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) acc = M::mac(wyl[u] * wxz, gv[xi][u], acc);
-                }
-            };
-            R ga[RX][4], gb[RX][4];
-            plane_pipeline(0, 1, Zs, ga, gb, load_plane, mma);
-        }
-        // lane holds D[16 nb + drow(lane >> 4, q)][lane & 15]
-        if (cvalid) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int kk = nb * 16 + M::drow(lane >> 4, q);
-                if (kk < cnt) partial[(size_t)(c0 + kk) * ncols + qc] = acc[q];
-            }
-        }
-    }
-}
-
-// Full-grid contraction on the matrix cores: the products of contract_mfma_kernel
-// over RX x PB x 16-voxel regions (x, y planes, z rows), one wave per (region,
-// column group of 16), work item = region x column groups + group, so that the
-// groups of a region run in neighbouring waves and share its weights in the caches.
-// Waves are independent (no LDS, no barriers).
-//
-// Memory access is in whole 16-byte vectors: the four voxels a lane feeds into the
-// four products of a plane and x are rows 4 r + u (r = lane / 16, u = 0..3), and the
-// two lanes of a complex column pair (real part j even, imaginary part j + 1) load
-// rows (4 r, 4 r + 1) and (4 r + 2, 4 r + 3) as complex pairs, then swap halves with
-// a neighbour-lane move; so one load instruction per x and plane reads the 16 rows
-// of eight complex components, one whole 128-byte line each.  The candidates'
-// weights come the same way, a vector each for x, the planes and the lane's rows.
-// Needs an even number of rows (z) and 16-byte aligned grid and weight rows.
-// The next plane's operands are loaded while the current plane's products run.
-template <typename R, int RX, int PB, int NB>
-__global__ __launch_bounds__(256) void contract_full_mfma_kernel(int B, RegionGeom rg, const R* __restrict__ regw,
-                                                                 const int* __restrict__ reg_start, int nitems,
-                                                                 int ngrp, const typename C2<R>::T* __restrict__ grid,
-                                                                 R* __restrict__ partial) {
-    using M = Mfma<R>;
-    using V4 = typename M::V4;  // four R: a complex pair of the grid, or four weights
-    using L = RegionW<RX, PB>;
-    static_assert(RX == 4 && PB == 8, "one weight vector for x, two for the planes");
-    static_assert(L::Z == 4 && L::Y == 12 && L::NW == 28, "weight row: x at 0, planes at 4, rows at 12");
-    constexpr int KC = 16 * NB;
-    const int lane = threadIdx.x & 63;
-    const int item = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (item >= nitems) return;  // the whole wave leaves: nothing below synchronises
-    const int reg = item / ngrp;
-    const RegionAt ra = region_at<RX>(rg, reg);
-    const int x0 = ra.x0, y0 = ra.row0, np = ra.np;
-    const int ncols = 6 * B;
-    const int r = lane >> 4, part = lane & 1;
-    const int qc = (item - reg * ngrp) * 16 + (lane & 15);
-    const bool cvalid = qc < ncols;
-    const R* gf = reinterpret_cast<const R*>(grid);
-    // 32-bit offsets in R from the uniform grid base (the launch keeps them below 2^32):
-    // cbase = the component's voxel (x0, plane0, y0), an in-grid pair of rows of every
-    // plane; this lane loads rows y0 + 4 r + 2 part and the next (vmask bit xi: inside)
-    unsigned cbase = 2u * ((unsigned)ra.plane0 * rg.ps + (unsigned)x0 * rg.xs + (unsigned)y0), coff = cbase,
-             vmask = 0;
-    if (cvalid) {
-        const int b = qc / 6, c = (qc >> 1) % 3;
-        cbase += 2u * (unsigned)(b * 3 + c) * rg.cs;
-        coff = cbase + 2u * (unsigned)(4 * r + 2 * part);
-#pragma unroll
-        for (int xi = 0; xi < RX; ++xi)
-            if (x0 + xi < rg.nx && y0 + 4 * r + 2 * part < rg.nrow) vmask |= 1u << xi;
-    }
-    const unsigned xstep = 2u * rg.xs, pstep = 2u * rg.ps;
-    const int k0 = reg_start[reg], k1 = reg_start[reg + 1];
-    struct PlaneBuf {
-        V4 g[RX];
-    };
-    for (int c0 = k0; c0 < k1; c0 += KC) {
-        const int cnt = min(KC, k1 - c0);
-        // this lane's candidates k = 16 nb + (lane & 15): x weights, plane weights (zero
-        // past the region's planes and for candidates past cnt) and rows 4 r .. 4 r + 3
-        R wyl[NB][4], wxl[NB][RX], wzl[NB][PB];
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            const int k = nb * 16 + (lane & 15);
-            const bool kin = k < cnt;
-            const V4* wr = reinterpret_cast<const V4*>(regw + (size_t)(c0 + (kin ? k : 0)) * L::NW);
-            const V4 wx = wr[0], wz0 = wr[1], wz1 = wr[2], wy = wr[3 + r];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                wxl[nb][q] = wx[q];
-                wzl[nb][q] = keep_if(wz0[q], kin && q < np);
-                wzl[nb][4 + q] = keep_if(wz1[q], kin && 4 + q < np);
-                wyl[nb][q] = wy[q];
-            }
-        }
-        // an opaque zero, redefined per chunk: keeps the compiler from hoisting all eight
-        // planes' loads out of the chunk loop (128 registers, no overlap with the products)
-        unsigned salt = 0;
-        asm volatile("" : "+v"(salt));
-        auto load_plane = [&](int p, PlaneBuf& dst) {
-            const int pc = min(p, np - 1);  // planes past the region's reload its last one
-            const unsigned poff = coff + salt + (unsigned)pc * pstep, pin = cbase + salt + (unsigned)pc * pstep;
-#pragma unroll
-            for (int xi = 0; xi < RX; ++xi) {
-                const bool in = (vmask >> xi) & 1u;
-                dst.g[xi] = *reinterpret_cast<const V4*>(gf + (in ? poff + xi * xstep : pin));
-            }
-        };
-        V4 acc[NB];
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) acc[nb] = V4{R(0), R(0), R(0), R(0)};
-        auto mma = [&](PlaneBuf& pb, int p) {
-#pragma unroll
-            for (int xi = 0; xi < RX; ++xi) {
-                R gv[4];
-                pair_rows<R>(pb.g[xi], part, gv);
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb) {
-                    const R wxz = wxl[nb][xi] * wzl[nb][p];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) acc[nb] = M::mac(wyl[nb][u] * wxz, gv[u], acc[nb]);
-                }
-            }
-        };
-        PlaneBuf ga, gb;
-        load_plane(0, ga);
-#pragma unroll
-        for (int p = 0; p < PB; p += 2) {
-            __builtin_amdgcn_sched_barrier(0);
-            load_plane(p + 1, gb);
-            __builtin_amdgcn_sched_barrier(0);
-            mma(ga, p);
-            __builtin_amdgcn_sched_barrier(0);
-            if (p + 2 < PB) load_plane(p + 2, ga);
-            __builtin_amdgcn_sched_barrier(0);
-            mma(gb, p + 1);
-        }
-        // lane holds D[16 nb + drow(lane >> 4, r)][lane & 15]
-        if (cvalid) {
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int k = nb * 16 + M::drow(lane >> 4, q);
-                    if (k < cnt) partial[(size_t)(c0 + k) * ncols + qc] = acc[nb][q];
-                }
         }
     }
 }
@@ -3302,11 +2521,6 @@ __global__ __launch_bounds__(256, ZS <= 10 ? 3 : 2) void xtoeplitz_kernel(typena
     }
 }
 
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
 
 // One wavefront per (particle, group of G right-hand sides; blockIdx.y strides the
 // groups): Gaussian contraction of the (inverse-transformed)
@@ -3317,7 +2531,7 @@ __global__ __launch_bounds__(256) void gather_kernel(
     const int* __restrict__ zmap, const int* __restrict__ base, const R* __restrict__ wts, int N, double h3,
     const double* __restrict__ pos, const int* __restrict__ nb_start, const int* __restrict__ nb_j,
     const double2* __restrict__ nb_f, double Lx, double Ly, double Lz, double kbx, double kby,
-    const double2* __restrict__ selfc, double self_perp, int jacobi, const R* __restrict__ partial,
+    const double2* __restrict__ selfc, double self_perp, int jacobi, const R* __restrict__ partial, int part64,
     const int* __restrict__ ps_start, const int* __restrict__ ps_items, const int* __restrict__ order) {
     __shared__ int s_off[kMaxWidth * kMaxWidth * kMaxWidth];
     const int lane = threadIdx.x & 63;
@@ -3376,14 +2590,22 @@ __global__ __launch_bounds__(256) void gather_kernel(
             // particle's region slots (ascending region order)
             const int s1 = partial ? ps_start[i + 1] : 0;
             for (int t = (partial ? ps_start[i] : 0) + lane; t < s1; t += 64) {
-                const R* pp = partial + (size_t)ps_items[t] * (6 * B);
+                const size_t p0 = (size_t)ps_items[t] * (6 * B);
+                const double* p64 = reinterpret_cast<const double*>(partial) + p0;
+                const R* pr = partial + p0;
 #pragma unroll
                 for (int j = 0; j < G; ++j) {
                     if (g0 + j >= B) break;
 #pragma unroll
                     for (int c = 0; c < 3; ++c) {
-                        racc[j][c][0] += (R)pp[6 * (g0 + j) + 2 * c];
-                        racc[j][c][1] += (R)pp[6 * (g0 + j) + 2 * c + 1];
+                        const int e = 6 * (g0 + j) + 2 * c;
+                        if (sizeof(R) == 8 || !part64) {
+                            racc[j][c][0] += pr[e];
+                            racc[j][c][1] += pr[e + 1];
+                        } else {
+                            acc[j][c][0] += p64[e];
+                            acc[j][c][1] += p64[e + 1];
+                        }
                     }
                 }
             }
@@ -3421,8 +2643,10 @@ __global__ __launch_bounds__(256) void gather_kernel(
             for (int j = 0; j < G; ++j)
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
-                    acc[j][c][0] = (double)racc[j][c][0] * h3;
-                    acc[j][c][1] = (double)racc[j][c][1] * h3;
+                    acc[j][c][0] = (sizeof(R) == 8 ? 0.0 : acc[j][c][0]) + (double)racc[j][c][0];
+                    acc[j][c][1] = (sizeof(R) == 8 ? 0.0 : acc[j][c][1]) + (double)racc[j][c][1];
+                    acc[j][c][0] *= h3;
+                    acc[j][c][1] *= h3;
                 }
         }
         if (parts & MPM_PART_REAL) {
@@ -3893,334 +3117,6 @@ __global__ __launch_bounds__(256) void poly_gather_kernel(SlotTable tab, int B, 
 }
 
 // ---------------------------------------------------------------------------
-// Quadrupole kernels (monodisperse, full grid [B][8][nx*ny*nz]: the field's 3
-// components, then the 5 quadrupole-gradient components)
-// ---------------------------------------------------------------------------
-
-// Per voxel: khat (3), sc, scQ, scGP, scGQ, Qfactor (5), Qdot (5) (:1301-1404).
-__global__ void quad_kspace_kernel(double* __restrict__ k64, float* __restrict__ k32, KParams q) {
-    const size_t V = (size_t)q.nx * q.ny * q.nz;
-    for (size_t v = blockIdx.x * (size_t)blockDim.x + threadIdx.x; v < V; v += (size_t)gridDim.x * blockDim.x) {
-        const int ix = (int)(v / ((size_t)q.ny * q.nz)), iy = (int)((v / q.nz) % q.ny), iz = (int)(v % q.nz);
-        const double fx = ix <= (q.nx - 1) / 2 ? ix : ix - q.nx;
-        const double fy = iy <= (q.ny - 1) / 2 ? iy : iy - q.ny;
-        const double fz = iz <= (q.nz - 1) / 2 ? iz : iz - q.nz;
-        const double Gx = fx * 2.0 * kPi / q.Lx, Gy = fy * 2.0 * kPi / q.Ly, Gz = fz * 2.0 * kPi / q.Lz;
-        const double kx = Gx - q.kbx, ky = Gy - q.kby, kz = Gz;
-        const double k2 = kx * kx + ky * ky + kz * kz, k = sqrt(k2);
-        double o[16];
-        for (int c = 0; c < 16; ++c) o[c] = 0.0;
-        if (k >= 1e-12) {
-            const double h0 = kx / k, h1 = ky / k, h2 = kz / k;
-            const double etak2 = k2 - (Gx * Gx * q.etax + Gy * Gy * q.etay + Gz * Gz * q.etaz);
-            double sk, ck;
-            sincos(k, &sk, &ck);
-            const double t = sk / k - ck;
-            const double ex = exp(-etak2 / (4.0 * q.xi * q.xi));
-            const double j1 = t / k, j2 = (3.0 / k2 - 1.0) * sk / k - 3.0 * ck / k2;
-            const double e2 = ex / k2 * q.invV;
-            o[0] = h0;
-            o[1] = h1;
-            o[2] = h2;
-            o[3] = 9.0 * t * t * ex / (k2 * k2) * q.invV;
-            o[4] = -22.5 * j1 * j2 * e2;
-            o[5] = 45.0 * j1 * j2 * e2;
-            o[6] = 112.5 * j2 * j2 * e2;
-            o[7] = h0 * h0 - 1.0 / 3.0;
-            o[8] = h0 * h1;
-            o[9] = h0 * h2;
-            o[10] = h1 * h1 - 1.0 / 3.0;
-            o[11] = h1 * h2;
-            o[12] = h0 * h0 - h2 * h2;
-            o[13] = 2.0 * h0 * h1;
-            o[14] = 2.0 * h0 * h2;
-            o[15] = h1 * h1 - h2 * h2;
-        }
-        // Qdot[4] = 2 h1 h2 does not fit the 16 slots: the scale kernel forms it from khat
-        for (int c = 0; c < 16; ++c) {
-            k64[16 * v + c] = o[c];
-            k32[16 * v + c] = (float)o[c];
-        }
-    }
-}
-
-// Owner-computes spread of dipoles (field grid) and quadrupoles (gradient grid)
-// with the Gaussian weights: a thread per voxel and G right-hand sides.
-template <typename R, int G>
-__global__ __launch_bounds__(256) void quad_spread_kernel(SlotTable tab, int B, int N, int V, int SS,
-                                                          const int* __restrict__ vox_start,
-                                                          const int* __restrict__ vox_items,
-                                                          const R* __restrict__ sw, const int* __restrict__ qmap,
-                                                          typename C2<R>::T* __restrict__ out) {
-    using CT = typename C2<R>::T;
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= V) return;
-    const int g0 = blockIdx.y * G;
-    R ar[G][8], ai[G][8];
-#pragma unroll
-    for (int j = 0; j < G; ++j)
-#pragma unroll
-        for (int c = 0; c < 8; ++c) ar[j][c] = ai[j][c] = R(0);
-    const int e0 = vox_start[v], e1 = vox_start[v + 1];
-    for (int e = e0; e < e1; ++e) {
-        const int item = vox_items[e];
-        const int pid = item / SS;
-        const R w = sw[item];
-        const int q = qmap[pid];
-#pragma unroll
-        for (int j = 0; j < G; ++j) {
-            if (g0 + j < B) {
-                const double2* x = tab.x[g0 + j];
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    const double2 pv = x[3 * (size_t)pid + c];
-                    ar[j][c] += w * (R)pv.x;
-                    ai[j][c] += w * (R)pv.y;
-                }
-                if (q >= 0) {
-#pragma unroll
-                    for (int c = 0; c < 5; ++c) {
-                        const double2 qv = x[3 * (size_t)N + 5 * (size_t)q + c];
-                        ar[j][3 + c] += w * (R)qv.x;
-                        ai[j][3 + c] += w * (R)qv.y;
-                    }
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-        if (g0 + j < B) {
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                CT o;
-                o.x = ar[j][c];
-                o.y = ai[j][c];
-                out[((size_t)(g0 + j) * 8 + c) * V + v] = o;
-            }
-        }
-    }
-}
-
-// Joint k-space coupling of field and gradient grids (scale_kernel_joint,
-// :1435-1487): Edk = E.khat, GQ = G.Qdot; E <- (sc Edk + i scQ GQ) khat,
-// G <- (i scGP Edk + scGQ GQ) Qfactor.
-template <typename R>
-__global__ __launch_bounds__(256) void quad_scale_kernel(typename C2<R>::T* __restrict__ grid,
-                                                         const R* __restrict__ kq, size_t V, size_t total) {
-    using CT = typename C2<R>::T;
-    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x) {
-        const size_t b = e / V, v = e - b * V;
-        CT* g = grid + b * 8 * V + v;
-        const R* k = kq + 16 * v;
-        const R h0 = k[0], h1 = k[1], h2 = k[2];
-        const R qd[5] = {k[12], k[13], k[14], k[15], R(2) * h1 * h2};
-        CT f[8];
-#pragma unroll
-        for (int c = 0; c < 8; ++c) f[c] = g[c * V];
-        const R er = f[0].x * h0 + f[1].x * h1 + f[2].x * h2, ei = f[0].y * h0 + f[1].y * h1 + f[2].y * h2;
-        R gr = R(0), gi = R(0);
-#pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            gr += f[3 + c].x * qd[c];
-            gi += f[3 + c].y * qd[c];
-        }
-        // i a (x + i y) = -a y + i a x
-        const R sr = k[3] * er - k[4] * gi, si = k[3] * ei + k[4] * gr;
-        const R tr = -k[5] * ei + k[6] * gr, ti = k[5] * er + k[6] * gi;
-        const R hh[3] = {h0, h1, h2};
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            CT o;
-            o.x = sr * hh[c];
-            o.y = si * hh[c];
-            g[c * V] = o;
-        }
-#pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            CT o;
-            o.x = tr * k[7 + c];
-            o.y = ti * k[7 + c];
-            g[(3 + c) * V] = o;
-        }
-    }
-}
-
-// A wave per (particle i, group of G right-hand sides): reciprocal field and,
-// for a quadrupole particle, gradient (h^3 sum of the Gaussian weights times the
-// grids), the real-space couplings of every neighbour's dipole and quadrupole
-// (dipole -> field, quadrupole -> field, dipole -> gradient, quadrupole ->
-// gradient, :1631-1869 with the cross-term signs of tests/quadrupole_field.py:214-215),
-// the self terms (sc + self_perp for the field, 2.5 sc + self_grad / 2 for the
-// gradient) and the optional left Jacobi scaling; FP64 sums, one reduction.
-// Pair data [16]: u (3), perp, para - perp, cos, sin, field_quad_1..3, grad_quad_1..4.
-template <typename R, int G>
-__global__ __launch_bounds__(256) void quad_gather_kernel(SlotTable tab, int B, int parts, int N, int V, int SS,
-                                                          const typename C2<R>::T* __restrict__ grid,
-                                                          const R* __restrict__ sw, const int* __restrict__ pidx,
-                                                          const int* __restrict__ qmap, double h3,
-                                                          const int* __restrict__ nb_start,
-                                                          const int* __restrict__ nb_j,
-                                                          const double* __restrict__ pairq,
-                                                          const double2* __restrict__ selfc, double self_perp,
-                                                          double self_grad, int jacobi,
-                                                          const int* __restrict__ order) {
-    using CT = typename C2<R>::T;
-    const int lane = threadIdx.x & 63;
-    const int wv = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (wv >= N) return;  // whole wave
-    const int i = order[wv];  // spatial order: neighbouring waves share stencil voxels
-    const int g0 = blockIdx.y * G;
-    const int qi = qmap[i];
-    const int nc = qi >= 0 ? 8 : 3;
-    double acc[G][8][2];
-#pragma unroll
-    for (int j = 0; j < G; ++j)
-#pragma unroll
-        for (int c = 0; c < 8; ++c) acc[j][c][0] = acc[j][c][1] = 0.0;
-    if (parts & MPM_PART_RECIP) {
-        for (int o = lane; o < SS; o += 64) {
-            const size_t item = (size_t)i * SS + o;
-            const int v = pidx[item];
-            const double w = (double)sw[item] * h3;
-#pragma unroll
-            for (int j = 0; j < G; ++j) {
-                if (g0 + j < B) {
-#pragma unroll
-                    for (int c = 0; c < 8; ++c) {
-                        if (c < nc) {
-                            const CT gv = grid[((size_t)(g0 + j) * 8 + c) * V + v];
-                            acc[j][c][0] += w * (double)gv.x;
-                            acc[j][c][1] += w * (double)gv.y;
-                        }
-                    }
-                }
-            }
-        }
-    }
-    if (parts & MPM_PART_REAL) {
-        const int k0 = nb_start[i], k1 = nb_start[i + 1];
-        const double I5[5] = {1.0, 0.0, 0.0, 1.0, 0.0};
-        for (int k = k0 + lane; k < k1; k += 64) {
-            const int jn = nb_j[k];
-            const int qs = qmap[jn];
-            const double* pc = pairq + 16 * (size_t)k;
-            const double u[3] = {pc[0], pc[1], pc[2]};
-            const double cp = pc[3], cd = pc[4], ec = pc[5], es = pc[6];
-            const double t0 = pc[7], t1 = pc[8], t2 = pc[9], g1 = pc[10], g2 = pc[11], g3 = pc[12], g4 = pc[13];
-            const double rr[5] = {u[0] * u[0], u[0] * u[1], u[0] * u[2], u[1] * u[1], u[1] * u[2]};
-#pragma unroll
-            for (int j = 0; j < G; ++j) {
-                if (g0 + j < B) {
-                    const double2* x = tab.x[g0 + j];
-                    const double2 pp[3] = {x[3 * (size_t)jn], x[3 * (size_t)jn + 1], x[3 * (size_t)jn + 2]};
-                    double f[8][2];
-                    const double rpr = pp[0].x * u[0] + pp[1].x * u[1] + pp[2].x * u[2];
-                    const double rpi = pp[0].y * u[0] + pp[1].y * u[1] + pp[2].y * u[2];
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) {
-                        f[c][0] = cp * pp[c].x + cd * rpr * u[c];
-                        f[c][1] = cp * pp[c].y + cd * rpi * u[c];
-                    }
-#pragma unroll
-                    for (int c = 3; c < 8; ++c) f[c][0] = f[c][1] = 0.0;
-                    double Qr[3][2] = {{0, 0}, {0, 0}, {0, 0}}, Qrr[2] = {0, 0};
-                    double2 qq[5];
-                    if (qs >= 0) {
-#pragma unroll
-                        for (int c = 0; c < 5; ++c) qq[c] = x[3 * (size_t)N + 5 * (size_t)qs + c];
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) {
-                            const double q0 = h ? qq[0].y : qq[0].x, q1 = h ? qq[1].y : qq[1].x,
-                                         q2 = h ? qq[2].y : qq[2].x, q3 = h ? qq[3].y : qq[3].x,
-                                         q4 = h ? qq[4].y : qq[4].x;
-                            Qr[0][h] = q0 * u[0] + q1 * u[1] + q2 * u[2];
-                            Qr[1][h] = q1 * u[0] + q3 * u[1] + q4 * u[2];
-                            Qr[2][h] = q2 * u[0] + q4 * u[1] - (q0 + q3) * u[2];
-                            Qrr[h] = Qr[0][h] * u[0] + Qr[1][h] * u[1] + Qr[2][h] * u[2];
-#pragma unroll
-                            for (int c = 0; c < 3; ++c) f[c][h] += 0.5 * (Qrr[h] * t0 * u[c] + 2.0 * t1 * Qr[c][h]);
-                        }
-                    }
-                    if (qi >= 0) {
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) {
-                            const double rp = h ? rpi : rpr;
-                            const double p0 = h ? pp[0].y : pp[0].x, p1 = h ? pp[1].y : pp[1].x,
-                                         p2 = h ? pp[2].y : pp[2].x;
-                            const double PrrP[5] = {2.0 * p0 * u[0], p0 * u[1] + p1 * u[0], p0 * u[2] + p2 * u[0],
-                                                    2.0 * p1 * u[1], p1 * u[2] + p2 * u[1]};
-#pragma unroll
-                            for (int c = 0; c < 5; ++c)
-                                f[3 + c][h] = -(rp * (t0 * rr[c] + (t1 + t2) * I5[c]) + PrrP[c] * t1);
-                            if (qs >= 0) {
-                                const double qv[5] = {h ? qq[0].y : qq[0].x, h ? qq[1].y : qq[1].x, h ? qq[2].y : qq[2].x,
-                                                      h ? qq[3].y : qq[3].x, h ? qq[4].y : qq[4].x};
-                                const double QrrQ[5] = {2.0 * Qr[0][h] * u[0], Qr[0][h] * u[1] + Qr[1][h] * u[0],
-                                                        Qr[0][h] * u[2] + Qr[2][h] * u[0], 2.0 * Qr[1][h] * u[1],
-                                                        Qr[1][h] * u[2] + Qr[2][h] * u[1]};
-#pragma unroll
-                                for (int c = 0; c < 5; ++c)
-                                    f[3 + c][h] += 0.5 * (Qrr[h] * ((g1 + g3) * I5[c] + g4 * rr[c]) + qv[c] * g2 +
-                                                          2.0 * g3 * QrrQ[c]);
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int c = 0; c < 8; ++c) {
-                        acc[j][c][0] += f[c][0] * ec - f[c][1] * es;
-                        acc[j][c][1] += f[c][0] * es + f[c][1] * ec;
-                    }
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < G; ++j)
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            acc[j][c][0] = wave_sum(acc[j][c][0]);
-            acc[j][c][1] = wave_sum(acc[j][c][1]);
-        }
-    if (lane >= G * 8) return;
-    const int j = lane / 8, c = lane % 8;  // lane (j, c) stores component c of right-hand side g0 + j
-    if (g0 + j >= B || c >= nc) return;
-    double yr = 0.0, yi = 0.0;
-    const double2* xb = nullptr;
-    double2* yb = nullptr;
-    int row = 0;
-#pragma unroll
-    for (int jj = 0; jj < G; ++jj) {  // uniform indices into the argument, selected per lane
-        if (jj == j) {
-            xb = tab.x[g0 + jj];
-            yb = tab.y[g0 + jj];
-            row = tab.row[g0 + jj];
-        }
-#pragma unroll
-        for (int cc = 0; cc < 8; ++cc)
-            if (jj == j && cc == c) {
-                yr = acc[jj][cc][0];
-                yi = acc[jj][cc][1];
-            }
-    }
-    const size_t e = c < 3 ? 3 * (size_t)i + c : 3 * (size_t)N + 5 * (size_t)qi + (c - 3);
-    const double2 xv = xb[e];
-    const double2 sc = selfc[(size_t)row * N + i];
-    if (parts & MPM_PART_REAL) {
-        const double fr = c < 3 ? sc.x + self_perp : 2.5 * sc.x + 0.5 * self_grad;
-        const double fi = c < 3 ? sc.y : 2.5 * sc.y;
-        yr += fr * xv.x - fi * xv.y;
-        yi += fr * xv.y + fi * xv.x;
-    }
-    double2 inv = make_double2(1.0, 0.0);
-    if (jacobi) {
-        const double den = sc.x * sc.x + sc.y * sc.y;
-        if (den > 1e-30) inv = make_double2(sc.x / den, -sc.y / den);
-    }
-    yb[e] = make_double2(yr * inv.x - yi * inv.y, yr * inv.y + yi * inv.x);
-}
-
-// ---------------------------------------------------------------------------
 // Direct (open-boundary) field in the solver's mode, after
 // src/cpp/electric_field/direct_electric_field.cu:37-300 (direct_field_kernel,
 // SOLVER_AX).  A thread per target particle and G right-hand sides; the sources
@@ -4466,6 +3362,7 @@ EwaldOp::EwaldOp(const mpm_op_desc& d) {
     fft_backend = d.fft_backend;
     MPM_REQUIRE(S.width <= kMaxWidth, MPM_ERR_UNSUPPORTED,
                 "stencil wider than " + std::to_string(kMaxWidth) + " points per axis");
+    quads_full = d.layout == 1;
     self_perp = dipole_self_term(xi);
     V = (size_t)S.n[0] * S.n[1] * S.n[2];
     table = std::make_unique<PairTable>(xi);
@@ -4770,62 +3667,10 @@ void EwaldOp::set_quads(const int* idx, int64_t nq) {
     quads_all = nq < 0;
     qreq_h.assign(idx && nq > 0 ? idx : nullptr, idx && nq > 0 ? idx + nq : nullptr);
     if (direct) return;
-    force_full = 1;  // the slab kernels carry dipoles only
+    force_full = 1;  // the layout callers see; the applies choose their own (quads_full)
     table->build_quads(xi);
+    quad_self_grad = table->self_grad;
     build_kspace();
-}
-
-// Per-frame stencils with quadrupoles: the W^3 points of every particle, their
-// wrapped voxels and Gaussian weights C exp(-2 xi^2 sum gd^2/eta) (the dipole
-// weights, monodisperse...cu:687-816), and the voxel -> entry lists.
-void EwaldOp::setup_quad_stencils(const std::vector<double>& pos, int Nn) {
-    const int W = S.width, half = S.half;
-    const int SS = W * W * W;
-    MPM_REQUIRE((int64_t)Nn * SS < (1LL << 31), MPM_ERR_UNSUPPORTED, "too many stencil points");
-    const double prod_eta = S.eta[0] * S.eta[1] * S.eta[2];
-    const double Cs = std::pow(2.0 * xi * xi / kPi, 1.5) * std::sqrt(1.0 / prod_eta);
-    std::vector<double> sw((size_t)Nn * SS);
-    std::vector<int> pidx((size_t)Nn * SS), cnt(V + 1, 0);
-    for (int i = 0; i < Nn; ++i) {
-        int g[3];
-        double dd[3];
-        for (int d = 0; d < 3; ++d) {
-            const double p = pos[(size_t)d * Nn + i];
-            g[d] = (int)std::round(p / S.h[d]);
-            dd[d] = g[d] * S.h[d] - p;
-        }
-        int o = 0;
-        for (int ox = -half; ox <= half; ++ox)
-            for (int oy = -half; oy <= half; ++oy)
-                for (int oz = -half; oz <= half; ++oz, ++o) {
-                    const int off[3] = {ox, oy, oz};
-                    double a = 0.0;
-                    int w[3];
-                    for (int d = 0; d < 3; ++d) {
-                        w[d] = ((g[d] + off[d]) % S.n[d] + S.n[d]) % S.n[d];
-                        const double gd = dd[d] + off[d] * S.h[d];
-                        a += gd * gd / S.eta[d];
-                    }
-                    const size_t item = (size_t)i * SS + o;
-                    const int v = (w[0] * S.n[1] + w[1]) * S.n[2] + w[2];
-                    pidx[item] = v;
-                    sw[item] = Cs * std::exp(-2.0 * xi * xi * a);
-                    cnt[v + 1]++;
-                }
-    }
-    for (size_t v = 0; v < V; ++v) cnt[v + 1] += cnt[v];
-    std::vector<int> items((size_t)Nn * SS);
-    {
-        std::vector<int> fill(cnt.begin(), cnt.end() - 1);
-        for (size_t item = 0; item < (size_t)Nn * SS; ++item) items[fill[pidx[item]]++] = (int)item;
-    }
-    std::vector<float> sw32(sw.begin(), sw.end());
-    d_sw64.upload(sw.data(), sw.size());
-    d_sw32.upload(sw32.data(), sw32.size());
-    d_pidx.upload(pidx.data(), pidx.size());
-    d_vox_start.upload(cnt.data(), cnt.size());
-    d_vox_items.upload(items.data(), items.size());
-    build_quad_slots(Nn);
 }
 
 void EwaldOp::build_quad_slots(int Nn) {
@@ -4834,7 +3679,8 @@ void EwaldOp::build_quad_slots(int Nn) {
         for (int i = 0; i < Nn; ++i) qidx_h.push_back(i);
     else
         qidx_h = qreq_h;
-    std::vector<int> qmap(Nn, -1);
+    std::vector<int>& qmap = qmap_h;
+    qmap.assign(Nn, -1);
     for (size_t q = 0; q < qidx_h.size(); ++q) {
         MPM_REQUIRE(qidx_h[q] >= 0 && qidx_h[q] < Nn, MPM_ERR_INVALID_ARGUMENT, "quadrupole index out of range");
         MPM_REQUIRE(qmap[qidx_h[q]] < 0, MPM_ERR_INVALID_ARGUMENT, "repeated quadrupole index");
@@ -4871,17 +3717,15 @@ KParams EwaldOp::kparams() const {
 void EwaldOp::build_kspace() {
     // the full-grid coefficient table is built lazily (only the full-grid path reads it)
     kspace_ready = false;
+    quad_coef_valid = false;
 }
 
 void EwaldOp::ensure_kspace_table() {
-    const int key = quads ? 6000 : (poly ? 5000 : (!slab ? 0 : (zcontig ? 2 + Zs : 1) + (kt ? 1000 : 0)));
+    const int key = quads ? 6000 + (slab ? Zs : 0) : (poly ? 5000 : (!slab ? 0 : (zcontig ? 2 + Zs : 1) + (kt ? 1000 : 0)));
     if (kspace_ready && kspace_key == key) return;
     const int threads = 256;
     if (quads) {
-        d_kq64.resize(16 * V);
-        d_kq32.resize(16 * V);
-        const int blocks = (int)std::min<size_t>((V + threads - 1) / threads, 65535);
-        hipLaunchKernelGGL(quad_kspace_kernel, dim3(blocks), dim3(threads), 0, nullptr, d_kq64.p, d_kq32.p, kparams());
+        build_quad_tables();
     } else if (poly) {
         d_k64.resize(V);
         d_k32.resize(V);
@@ -5293,6 +4137,11 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
     last_xyz.clear();
     N = n;
     HostLaps laps;
+    if (quads) {
+        MPM_REQUIRE(n * S.width * S.width * S.width < (1LL << 31), MPM_ERR_UNSUPPORTED, "too many stencil points");
+        quad_stencils_valid = false;
+        build_quad_slots(Nn);
+    }
     const int W = S.width, half = S.half;
     std::vector<double> pos(3 * (size_t)Nn);
     std::vector<int> base(3 * (size_t)Nn);
@@ -5342,7 +4191,12 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
         for (int a = 0; a < nzl; ++a) zl[a] = (z0 + a) % nz;
     }
     const int zsb = zs_bucket((int)zl.size());
-    const bool want_slab = force_full == 0 && zsb > 0 && (int)zl.size() * 2 <= nz &&
+    // (quadrupoles: up to the planes their coupling kernel holds in registers, with two real
+    // in-plane axes)
+    const bool may_slab = quads ? !quads_full && zsb <= kQuadSlabPlanes && S.n[0] > 1 && S.n[1] > 1 &&
+                                      LineFft::fits(S.n[0]) && LineFft::fits(S.n[1])
+                                : force_full == 0;
+    const bool want_slab = may_slab && zsb > 0 && (int)zl.size() * 2 <= nz &&
                            zfused_lds(zsb, nz, sizeof(double)) <= 64 * 1024;
     slab = want_slab;
     Zs = slab ? (int)zl.size() : 0;
@@ -5370,7 +4224,7 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
     reg_full = false;
     reg_npb = 1;
     reg_pblk = 0;
-    if (slab || (!poly && !quads)) {
+    if (!poly) {
         const int RX = slab ? (zs_bucket(Zs) <= 10 ? 4 : 2) : 4, RY = kMfmaRY;
         const int arow = slab ? 1 : 2;  // axis of the 16 contiguous rows
         int pblk = slab ? Zs : kFullRegionPlanes;
@@ -5464,12 +4318,17 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
         // grow-only: the slot count changes a little from frame to frame
         d_reg_start.assign(rs.data(), rs.size());
         d_reg_items.assign(ri.data(), ri.size());
+        if (quads) {  // each slot's quadrupole (-1: none)
+            std::vector<int> rq(ri.size(), -1);
+            for (int q = 0; q < rs[nreg]; ++q) rq[q] = qmap_h[ri[q]];
+            d_reg_quads.assign(rq.data(), rq.size());
+        }
         d_ps_start.assign(pss.data(), pss.size());
         d_ps_items.assign(psi.data(), psi.size());
         // one buffer for both precisions (an apply runs in one of them at a time), with an
         // eighth of headroom so that the next frames' slot counts fit without reallocation
         {
-            const size_t need = (size_t)std::max(rs[nreg], 1) * 6 * kMaxSlots;
+            const size_t need = (size_t)std::max(rs[nreg], 1) * (quads ? 16 : 6) * kMaxSlots;
             if (need > d_partial64.n) d_partial64.reserve(need + need / 8);
         }
         reg_slots = rs[nreg];
@@ -5718,15 +4577,16 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
         auto pass = [&](std::vector<LinePass>& v, int a, LineGeom gi, LineGeom go, int src, int dst) {
             v.push_back(LinePass{a, gi, go, src, dst});
         };
+        const long long nc = poly ? 1 : (quads ? 8 : 3);  // components of a right-hand side
         if (kt_ok) {
-            // [3][Zs][nx][nyp] -> y transform written transposed to the k-space
-            // buffer [3][Zs][ky][nxp] -> x transform in place on contiguous lines
-            lf->rhs_elems = 3LL * Zs * std::max((long long)nx * nyp, (long long)ny * nxp);
+            // [nc][Zs][nx][nyp] -> y transform written transposed to the k-space
+            // buffer [nc][Zs][ky][nxp] -> x transform in place on contiguous lines
+            lf->rhs_elems = nc * Zs * std::max((long long)nx * nyp, (long long)ny * nxp);
             const int ay = axis(ny), ax = axis(nx);
             lf->kt_x = ax;
-            const LineGeom yrun{3LL * Zs * nx, 1, 0, nyp, 1};
-            const LineGeom ytr{3LL * Zs * nx, nx, 1, (long long)ny * nxp, nxp};
-            const LineGeom xrun{3LL * Zs * ny, 1, 0, nxp, 1};
+            const LineGeom yrun{nc * Zs * nx, 1, 0, nyp, 1};
+            const LineGeom ytr{nc * Zs * nx, nx, 1, (long long)ny * nxp, nxp};
+            const LineGeom xrun{nc * Zs * ny, 1, 0, nxp, 1};
             pass(lf->fwd, ay, yrun, ytr, 0, 1);
             pass(lf->fwd, ax, xrun, xrun, 1, 1);
             pass(lf->inv, ax, xrun, xrun, 1, 1);
@@ -5746,7 +4606,6 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
                 pass(lf->inv, a, g, g, 0, 0);
             }
         } else {  // [comps][nx][ny][nz]: z, y, x lines in place (one component for the polydisperse grid)
-            const long long nc = poly ? 1 : (quads ? 8 : 3);
             lf->rhs_elems = nc * nxy * nzz;
             const LineGeom gz{nc * nxy, 1, 0, nzz, 1};
             const LineGeom gy{nc * nx * nzz, nzz, 1, (long long)ny * nzz, nzz};
@@ -5768,7 +4627,7 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
     kt = slab && lfft && fft_backend == 0 && S.n[0] > 1 && S.n[1] > 1;
     if (!fft || fft_key != key) {
         if (slab)
-            fft = std::make_unique<FftPlans>(std::vector<size_t>{(size_t)S.n[1], (size_t)S.n[0]}, 3 * Zs);
+            fft = std::make_unique<FftPlans>(std::vector<size_t>{(size_t)S.n[1], (size_t)S.n[0]}, (quads ? 8 : 3) * Zs);
         else
             fft = std::make_unique<FftPlans>(std::vector<size_t>{(size_t)S.n[2], (size_t)S.n[1], (size_t)S.n[0]},
                                              poly ? 1 : (quads ? 8 : 3));
@@ -5781,8 +4640,6 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
     if (quads) {
         MPM_REQUIRE(lfft != nullptr && fft_backend == 0, MPM_ERR_UNSUPPORTED,
                     "quadrupoles run on the built-in FFT only");
-        setup_quad_stencils(pos, Nn);
-        build_pair_coefs();  // with the quadrupole table values
     }
     // default self coefficients: zero (reference base_electric_field.cu allocates them zeroed)
     if (self_rows == 0 || d_selfc.n != (size_t)self_rows * Nn) {
@@ -5813,14 +4670,49 @@ void EwaldOp::set_self_coef_device(const double* coef, int rows, hipStream_t s) 
     self_rows = rows;
 }
 
+template <typename R>
+void EwaldOp::line_fft(void* grid, void* kgrid, int B, bool forward, hipStream_t s) {
+    using CT = typename C2<R>::T;
+    lfft->exec<R>(reinterpret_cast<CT*>(grid), reinterpret_cast<CT*>(kgrid), B, forward, s);
+}
+template void EwaldOp::line_fft<float>(void*, void*, int, bool, hipStream_t);
+template void EwaldOp::line_fft<double>(void*, void*, int, bool, hipStream_t);
+
 size_t EwaldOp::grid_elems_per_rhs() const {
     if (poly) return V;
-    if (quads) return 8 * V;
-    return slab ? 3 * (size_t)Zs * S.n[0] * nyp : 3 * V;
+    const size_t nc = quads ? 8 : 3;
+    return slab ? nc * Zs * S.n[0] * nyp : nc * V;
 }
-size_t EwaldOp::kgrid_elems_per_rhs() const { return 3 * (size_t)Zs * kspace_cols(); }
+size_t EwaldOp::kgrid_elems_per_rhs() const { return (quads ? 8 : 3) * (size_t)Zs * kspace_cols(); }
 // columns of one slab plane in the k-space buffer (padding columns included)
 int EwaldOp::kspace_cols() const { return kt ? S.n[1] * nxp : S.n[0] * S.n[1]; }
+
+RegionGeom EwaldOp::region_geom(bool on_slab) const {
+    RegionGeom rg;
+    rg.nx = S.n[0];
+    rg.nrr = reg_nry;
+    rg.npb = reg_npb;
+    rg.pblk = reg_pblk;
+    if (on_slab) {
+        rg.nrow = S.n[1];
+        rg.nplane = Zs;
+        rg.xs = (unsigned)nyp;
+        rg.ps = (unsigned)(S.n[0] * nyp);
+        rg.cs = (unsigned)((size_t)Zs * S.n[0] * nyp);
+    } else {
+        rg.nrow = S.n[2];
+        rg.nplane = S.n[1];
+        rg.xs = (unsigned)(S.n[1] * S.n[2]);
+        rg.ps = (unsigned)S.n[2];
+        rg.cs = (unsigned)V;
+    }
+    return rg;
+}
+
+RegionSet EwaldOp::region_set(bool on_slab) const {
+    return RegionSet{on_slab,        on_slab ? zs_bucket(Zs) : reg_pblk, reg_nrx * reg_npb * reg_nry, reg_slots,
+                     d_reg_start.p, d_reg_items.p,                      d_reg_quads.p};
+}
 
 template <typename R, bool SLAB>
 void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int jacobi) {
@@ -5847,24 +4739,7 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
     g.nyp = slab ? nyp : S.n[1];
     const R* regw = fp32 ? reinterpret_cast<const R*>(d_regw32.p) : reinterpret_cast<const R*>(d_regw64.p);
     const int Ni = (int)N;
-    RegionGeom rg;
-    rg.nx = S.n[0];
-    rg.nrr = reg_nry;
-    rg.npb = reg_npb;
-    rg.pblk = reg_pblk;
-    if (SLAB) {
-        rg.nrow = S.n[1];
-        rg.nplane = Zs;
-        rg.xs = (unsigned)nyp;
-        rg.ps = (unsigned)(S.n[0] * nyp);
-        rg.cs = (unsigned)((size_t)Zs * S.n[0] * nyp);
-    } else {
-        rg.nrow = S.n[2];
-        rg.nplane = S.n[1];
-        rg.xs = (unsigned)(S.n[1] * S.n[2]);
-        rg.ps = (unsigned)S.n[2];
-        rg.cs = (unsigned)V;
-    }
+    const RegionGeom rg = region_geom(SLAB);
     // the matrix-core kernels address the grid with 32-bit element offsets
     const int nreg = reg_nrx * reg_npb * reg_nry;
     const bool regions = reg_rx > 0 && 2ull * (unsigned long long)B * grid_elems_per_rhs() < (1ull << 32);
@@ -5878,39 +4753,7 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
         if (phases & 1) {
             if (regions) {
                 ProfScope ps("spread", s, B);
-                // 32 columns per block, or 16 where a batch has no more, and on the full grid
-                // while those blocks are fewer than eight per CU (7001 particles on
-                // 47 x 47 x 48, 5 right-hand sides: 36.2 -> 28.8 us; the slab's regions hold
-                // about one chunk of candidates, which leaves nothing to prefetch)
-                const int cpb = 6 * B <= 16 || (!SLAB && (long long)nreg * ((6 * B + 31) / 32) < 2048) ? 16 : 32;
-                const dim3 gs((unsigned)nreg, (unsigned)((6 * B + cpb - 1) / cpb));
-    #define MPM_SM1(RXV, ZSV, CPBV)                                                                                   \
-        do {                                                                                                          \
-            ps.kernel("spread_mfma_kernel", {type_name<R>(), #RXV, #ZSV, #CPBV});                                     \
-            hipLaunchKernelGGL((spread_mfma_kernel<R, RXV, ZSV, CPBV>), gs, dim3(256), 0, s, t, B, rg, regw,          \
-                               d_reg_start.p, d_reg_items.p, grid);                                                   \
-        } while (0)
-    #define MPM_SM(RXV, ZSV)                   \
-        case ZSV:                              \
-            if (cpb == 16)                     \
-                MPM_SM1(RXV, ZSV, 16);         \
-            else                               \
-                MPM_SM1(RXV, ZSV, 32);         \
-            break;
-                switch (SLAB ? zs_bucket(Zs) : reg_pblk) {
-                    MPM_SM(4, 4)
-                    MPM_SM(4, 6)
-                    MPM_SM(4, 8)
-                    MPM_SM(4, 10)
-                    MPM_SM(2, 12)
-                    MPM_SM(2, 14)
-                    MPM_SM(2, 16)
-                    default:
-                        throw Error(MPM_ERR_RUNTIME, "slab size out of range");
-                }
-    #undef MPM_SM
-    #undef MPM_SM1
-                MPM_HIP(hipGetLastError());
+                region_spread<R, 3>(ps, s, region_set(SLAB), rg, t, B, regw, 0, grid);
             } else {
                 ProfScope ps("spread", s, B);
                 ps.kernel("spread_kernel", {type_name<R>(), B == 1 ? "1" : "4", tbool(SLAB)});
@@ -6097,6 +4940,7 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
     }
     if (!(phases & 4)) return;
     const R* part = nullptr;
+    bool part64 = false;  // FP64 partial sums
     // The contraction as part of the per-particle gather instead of on the regions: for
     // batches that take that kernel anyway (B < 4, below) and give it no more than a wave per
     // SIMD (launches and latency decide; 400 particles on the slab, 3 right-hand sides: 76
@@ -6109,89 +4953,30 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
                               (!SLAB && (S.width <= 5 || (B == 1 && 4ll * nreg < (long long)N)));
     if (regions && !per_particle && (parts & MPM_PART_RECIP)) {
         ProfScope ps("contract", s, B);
-        // column groups of 16 per block: 4 when there are enough right-hand sides,
-        // else fewer, with the region's planes split over the remaining waves; slab
-        // with one or two column groups: one wave per candidate block instead
-        const int ngrp = (6 * B + 15) / 16;
-        const int ncg = ngrp >= 4 ? 4 : (ngrp >= 2 ? 2 : 1);
-        const dim3 gs((unsigned)nreg, (unsigned)((ngrp + ncg - 1) / ncg));
-        const dim3 gn((unsigned)nreg, (unsigned)ngrp);
+        // dense regions of the full grid sum in FP64 over either grid, as the gather does past
+        // each lane's few terms; the others in the grid's precision
+        part64 = !fp32;
+        if constexpr (std::is_same<R, float>::value && !SLAB) part64 = dense_regions(region_set(false));
         R* pbuf = reinterpret_cast<R*>(d_partial64.p);  // sized for FP64, shared by FP32
-        // full grid with more than 32 candidates per region on average: four waves per region
-        // and column group take a candidate block each (30,000 particles, 4 right-hand sides:
-        // an apply 814 us, 839 with contract_full_mfma_kernel, 984 with contract_mfma_kernel)
-        if (!SLAB && (reg_pblk == 4 || reg_slots > 32ll * nreg)) {
-#define MPM_CF(ZSV, VECV)                                                                                      \
-    do {                                                                                                       \
-        ps.kernel("contract_nb_mfma_kernel", {type_name<R>(), "4", #ZSV, #VECV});                              \
-        hipLaunchKernelGGL((contract_nb_mfma_kernel<R, 4, ZSV, VECV>), gn, dim3(256), 0, s, B, rg, regw,       \
-                           d_reg_start.p, d_reg_items.p, Ni, grid, pbuf);                                      \
-    } while (0)
-            if (reg_pblk == 4) {
-                if (vec) MPM_CF(4, true);
-                else MPM_CF(4, false);
-            } else {
-                if (vec) MPM_CF(8, true);
-                else MPM_CF(8, false);
-            }
-#undef MPM_CF
-        } else if (!SLAB && vec) {
-            ps.kernel("contract_full_mfma_kernel",
-                      {type_name<R>(), "4", std::to_string(kFullRegionPlanes), std::to_string(kFullContractNB)});
-            const int nitems = nreg * ngrp;
-            hipLaunchKernelGGL((contract_full_mfma_kernel<R, 4, kFullRegionPlanes, kFullContractNB>),
-                               dim3((unsigned)((nitems + 3) / 4)), dim3(256), 0, s, B, rg, regw, d_reg_start.p, nitems,
-                               ngrp, grid, pbuf);
-        } else if (!SLAB) {
-            ps.kernel("contract_mfma_kernel", {type_name<R>(), "4", std::to_string(kFullRegionPlanes),
-                                               std::to_string(kFullContractNB), "false"});
-            hipLaunchKernelGGL((contract_mfma_kernel<R, 4, kFullRegionPlanes, kFullContractNB, false>), gs, dim3(256),
-                               0, s, B, rg, regw, d_reg_start.p, d_reg_items.p, Ni, grid, pbuf, ncg);
-        } else {
-#define MPM_CM(RXV, ZSV)                                                                                          \
-    case ZSV:                                                                                                     \
-        if (ngrp <= 2) {                                                                                          \
-            ps.kernel("contract_nb_mfma_kernel", {type_name<R>(), #RXV, #ZSV, tbool(vec)});                       \
-            if (vec)                                                                                              \
-                hipLaunchKernelGGL((contract_nb_mfma_kernel<R, RXV, ZSV, true>), gn, dim3(256), 0, s, B, rg,      \
-                                   regw, d_reg_start.p, d_reg_items.p, Ni, grid, pbuf);                          \
-            else                                                                                                  \
-                hipLaunchKernelGGL((contract_nb_mfma_kernel<R, RXV, ZSV, false>), gn, dim3(256), 0, s, B, rg,     \
-                                   regw, d_reg_start.p, d_reg_items.p, Ni, grid, pbuf);                          \
-        } else if (vec) {                                                                                         \
-            ps.kernel("contract_mfma_kernel", {type_name<R>(), #RXV, #ZSV, "4", "true"});                         \
-            hipLaunchKernelGGL((contract_mfma_kernel<R, RXV, ZSV, 4, true>), gs, dim3(256), 0, s, B, rg, regw,    \
-                               d_reg_start.p, d_reg_items.p, Ni, grid, pbuf, ncg);                               \
-        } else {                                                                                                  \
-            ps.kernel("contract_mfma_kernel", {type_name<R>(), #RXV, #ZSV, "4", "false"});                        \
-            hipLaunchKernelGGL((contract_mfma_kernel<R, RXV, ZSV, 4, false>), gs, dim3(256), 0, s, B, rg, regw,   \
-                               d_reg_start.p, d_reg_items.p, Ni, grid, pbuf, ncg);                               \
-        }                                                                                                         \
-        break;
-        switch (zs_bucket(Zs)) {
-            MPM_CM(4, 4)
-            MPM_CM(4, 6)
-            MPM_CM(4, 8)
-            MPM_CM(4, 10)
-            MPM_CM(2, 12)
-            MPM_CM(2, 14)
-            MPM_CM(2, 16)
-            default:
-                throw Error(MPM_ERR_RUNTIME, "slab size out of range");
-        }
-#undef MPM_CM
-        }
-        MPM_HIP(hipGetLastError());
+        if (part64)
+            region_contract<double, 3, R>(ps, s, region_set(SLAB), rg, vec, B, d_regw64.p, grid, d_partial64.p);
+        else
+            region_contract<R, 3, R>(ps, s, region_set(SLAB), rg, vec, B, regw, grid, pbuf);
         part = pbuf;
     }
     if (part && B >= 4) {
         ProfScope ps("gather", s, B);
-        ps.kernel("finish_kernel", {type_name<R>()});
+        ps.kernel("finish_kernel", {part64 ? "double" : "float"});
         const double h3 = S.h[0] * S.h[1] * S.h[2];
         const int blocks = (int)(((size_t)Ni * B * kFinishLanes + 255) / 256);
-        hipLaunchKernelGGL((finish_kernel<R>), dim3(blocks), dim3(256), 0, s, t, B, parts, Ni, part, d_ps_start.p,
-                           d_ps_items.p, h3, d_nb_start.p, d_nb_j.p, d_pairc.p, d_selfc.p, self_perp, jacobi,
-                           d_order.p);
+        if (part64)
+            hipLaunchKernelGGL((finish_kernel<double>), dim3(blocks), dim3(256), 0, s, t, B, parts, Ni, d_partial64.p,
+                               d_ps_start.p, d_ps_items.p, h3, d_nb_start.p, d_nb_j.p, d_pairc.p, d_selfc.p, self_perp,
+                               jacobi, d_order.p);
+        else
+            hipLaunchKernelGGL((finish_kernel<float>), dim3(blocks), dim3(256), 0, s, t, B, parts, Ni,
+                               reinterpret_cast<const float*>(part), d_ps_start.p, d_ps_items.p, h3, d_nb_start.p,
+                               d_nb_j.p, d_pairc.p, d_selfc.p, self_perp, jacobi, d_order.p);
         MPM_HIP(hipGetLastError());
     } else {
         ProfScope ps("gather", s, B);
@@ -6201,64 +4986,19 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
         if (B == 1)
             hipLaunchKernelGGL((gather_kernel<R, 1, SLAB>), dim3(blocks, 1), dim3(256), 0, s, t, B, parts, grid, g,
                                d_zmap.p, d_base.p, w, Ni, h3, d_pos.p, d_nb_start.p, d_nb_j.p, d_nb_f.p, L[0], L[1],
-                               L[2], kb[0], kb[1], d_selfc.p, self_perp, jacobi, part, d_ps_start.p, d_ps_items.p,
+                               L[2], kb[0], kb[1], d_selfc.p, self_perp, jacobi, part, part64 ? 1 : 0, d_ps_start.p, d_ps_items.p,
                                d_order.p);
         else
             hipLaunchKernelGGL((gather_kernel<R, 4, SLAB>), dim3(blocks, (B + 3) / 4), dim3(256), 0, s, t, B, parts,
                                grid, g,
                                d_zmap.p, d_base.p, w, Ni, h3, d_pos.p, d_nb_start.p, d_nb_j.p, d_nb_f.p, L[0], L[1],
-                               L[2], kb[0], kb[1], d_selfc.p, self_perp, jacobi, part, d_ps_start.p, d_ps_items.p,
+                               L[2], kb[0], kb[1], d_selfc.p, self_perp, jacobi, part, part64 ? 1 : 0, d_ps_start.p, d_ps_items.p,
                                d_order.p);
         MPM_HIP(hipGetLastError());
     }
 }
 
 static_assert(kMaxSlots % 4 == 0, "the polydisperse kernels take right-hand sides in groups of 4");
-
-template <typename R>
-void EwaldOp::launch_quads(const SlotTable& t, int B, int parts, hipStream_t s, int jacobi) {
-    using CT = typename C2<R>::T;
-    const bool fp32 = std::is_same<R, float>::value;
-    CT* grid = reinterpret_cast<CT*>(cur_grid);
-    const R* sw = fp32 ? reinterpret_cast<const R*>(d_sw32.p) : reinterpret_cast<const R*>(d_sw64.p);
-    const int SS = S.width * S.width * S.width;
-    const int Vi = (int)V, Ni = (int)N;
-    constexpr int G = 2;
-    if ((parts & MPM_PART_RECIP) && (phases & 1)) {
-        ProfScope ps("spread", s, B);
-        ps.kernel("quad_spread_kernel", {type_name<R>(), "2"});
-        hipLaunchKernelGGL((quad_spread_kernel<R, G>), dim3((unsigned)((V + 255) / 256), (unsigned)((B + G - 1) / G)),
-                           dim3(256), 0, s, t, B, Ni, Vi, SS, d_vox_start.p, d_vox_items.p, sw, d_qmap.p, grid);
-        MPM_HIP(hipGetLastError());
-    }
-    if ((parts & MPM_PART_RECIP) && (phases & 2)) {
-        {
-            ProfScope ps("fft", s, B);
-            lfft->exec<R>(grid, grid, B, true, s);
-        }
-        {
-            ProfScope ps("scale", s, B);
-            ps.kernel("quad_scale_kernel", {type_name<R>()});
-            const R* kq = fp32 ? reinterpret_cast<const R*>(d_kq32.p) : reinterpret_cast<const R*>(d_kq64.p);
-            const size_t total = (size_t)B * V;
-            const int blocks = (int)std::min<size_t>((total + 255) / 256, 16384);
-            hipLaunchKernelGGL((quad_scale_kernel<R>), dim3(blocks), dim3(256), 0, s, grid, kq, V, total);
-            MPM_HIP(hipGetLastError());
-        }
-        {
-            ProfScope ps("fft", s, B);
-            lfft->exec<R>(grid, grid, B, false, s);
-        }
-    }
-    if (!(phases & 4)) return;
-    ProfScope ps("gather", s, B);
-    ps.kernel("quad_gather_kernel", {type_name<R>(), "2"});
-    const double h3 = S.h[0] * S.h[1] * S.h[2];
-    hipLaunchKernelGGL((quad_gather_kernel<R, G>), dim3((unsigned)((Ni + 3) / 4), (unsigned)((B + G - 1) / G)),
-                       dim3(256), 0, s, t, B, parts, Ni, Vi, SS, grid, sw, d_pidx.p, d_qmap.p, h3, d_nb_start.p,
-                       d_nb_j.p, d_pairc.p, d_selfc.p, self_perp, table->self_grad, jacobi, d_order.p);
-    MPM_HIP(hipGetLastError());
-}
 
 template <typename R>
 void EwaldOp::launch_poly(const SlotTable& t, int B, int parts, hipStream_t s, int jacobi) {
@@ -6508,7 +5248,7 @@ __global__ void add_kernel(double2* __restrict__ y, const double2* __restrict__ 
 }
 
 size_t EwaldOp::stage_grid_bytes(bool fp32) const {
-    return grid_elems_per_rhs() * (fp32 ? sizeof(float2) : sizeof(double2));
+    return (quads ? 8 * V : grid_elems_per_rhs()) * (fp32 ? sizeof(float2) : sizeof(double2));
 }
 
 void EwaldOp::stage(int which, const double2* x, void* grid, double2* y, bool fp32, hipStream_t s) {
@@ -6520,6 +5260,7 @@ void EwaldOp::stage(int which, const double2* x, void* grid, double2* y, bool fp
     MPM_REQUIRE(!recip || grid, MPM_ERR_INVALID_ARGUMENT, "stage needs a grid buffer");
     MPM_REQUIRE(which == 2 || (x != nullptr && (which == 1 || y != nullptr)), MPM_ERR_INVALID_ARGUMENT,
                 "stage needs the dipoles (and, to add into, the field)");
+    if (recip) quads_on_full_grid();
     if (recip) ensure_kspace_table();
     // spread writes the grid, scale transforms it in place; contract and real space add into y
     SlotTable t;
@@ -6575,7 +5316,7 @@ void EwaldOp::stage(int which, const double2* x, void* grid, double2* y, bool fp
     }
 }
 
-void* EwaldOp::device_pointer(const std::string& name, size_t& bytes) const {
+void* EwaldOp::device_pointer(const std::string& name, size_t& bytes) {
     auto give = [&](const void* p, size_t b) {
         bytes = p ? b : 0;
         return const_cast<void*>(p);
@@ -6588,15 +5329,22 @@ void* EwaldOp::device_pointer(const std::string& name, size_t& bytes) const {
     if (name == "radius") return give(d_drad.p, d_drad.n * sizeof(double));
     if (name == "spread_coef" || name == "contract_coef") {
         if (poly) return give(d_pw64.p, d_pw64.n * sizeof(double));
-        if (quads) return give(d_sw64.p, d_sw64.n * sizeof(double));
+        if (quads) {
+            ensure_quad_stencils();
+            return give(d_sw64.p, d_sw64.n * sizeof(double));
+        }
         return give(d_w64.p, d_w64.n * sizeof(double));
     }
     if (name == "spread_coef_fp32" || name == "contract_coef_fp32") {
         if (poly) return give(d_pw32.p, d_pw32.n * sizeof(float));
-        if (quads) return give(d_sw32.p, d_sw32.n * sizeof(float));
+        if (quads) {
+            ensure_quad_stencils();
+            return give(d_sw32.p, d_sw32.n * sizeof(float));
+        }
         return give(d_w32.p, d_w32.n * sizeof(float));
     }
     if (name == "spread_idxs" || name == "contract_idxs") {
+        if (quads) ensure_quad_stencils();
         if (poly || quads) return give(d_pidx.p, d_pidx.n * sizeof(int));
         return give(d_base.p, d_base.n * sizeof(int));
     }
@@ -6607,11 +5355,17 @@ void* EwaldOp::device_pointer(const std::string& name, size_t& bytes) const {
     if (name == "pair_coef") return give(d_pairc.p, d_pairc.n * sizeof(double));
     if (name == "self_perp") return give(d_selfp.p, d_selfp.n * sizeof(double));
     if (name == "scale_coef") {
-        if (quads) return give(d_kq64.p, d_kq64.n * sizeof(double));
+        if (quads) {
+            ensure_quad_scale_coef();
+            return give(d_kq64.p, d_kq64.n * sizeof(double));
+        }
         if (slab && zcontig) return give(d_toe64.p, d_toe64.n * sizeof(double2));
         return give(d_k64.p, d_k64.n * sizeof(double));
     }
-    if (name == "fe_grid") return give(cur_grid, 0);
+    if (name == "fe_grid") {
+        quads_on_full_grid();
+        return give(cur_grid, 0);
+    }
     if (name == "fes_grid") return give(d_kgrid64.p ? (void*)d_kgrid64.p : (void*)d_kgrid32.p,
                                         d_kgrid64.p ? d_kgrid64.n * sizeof(double2) : d_kgrid32.n * sizeof(float2));
     throw Error(MPM_ERR_INVALID_ARGUMENT, "unknown device buffer name '" + name + "'");
@@ -6633,7 +5387,7 @@ void EwaldOp::info(mpm_op_info& o) const {
     o.self_coef_ewald = -4.0 * std::pow(xi, 3.0) / (3.0 * std::sqrt(kPi));
     o.bloch[0] = kb[0];
     o.bloch[1] = kb[1];
-    o.slab_planes = slab ? Zs : 0;
+    o.slab_planes = slab && !quads ? Zs : 0;  // the grid of the stages, full with quadrupoles
     o.fft_backend = (lfft && fft_backend == 0) ? 0 : 1;
     o.polydisperse = poly ? 1 : 0;
     o.num_quads = (int64_t)qidx_h.size();

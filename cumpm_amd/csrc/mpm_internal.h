@@ -182,9 +182,17 @@ struct SlotTable {
     int row[kMaxSlots];  // self-coefficient row of the slot
 };
 
+struct RegionGeom;  // extents and strides of a grid buffer as the region kernels see it
+struct RegionSet;   // the current frame's regions
 struct FftPlans;   // rocFFT plans keyed by (precision, batch)
 struct PairTable;  // sampled real-space pair functions
-struct KParams;    // k-space geometry passed to the kernels
+// k-space geometry passed to the kernels
+struct KParams {
+    int nx, ny, nz;
+    int tcols;  // slab columns ordered ky * nxp + kx (else kx * ny + ky)
+    int nxp;    // row stride of the transposed columns (nx rounded up to whole cache lines)
+    double Lx, Ly, Lz, kbx, kby, xi, etax, etay, etaz, invV;
+};
 struct LineFft;    // built-in batched line FFT
 
 class EwaldOp {
@@ -235,7 +243,7 @@ class EwaldOp {
     void stage(int which, const double2* x, void* grid, double2* y, bool fp32, hipStream_t s);
     size_t stage_grid_bytes(bool fp32) const;
     // device address and size of a named internal buffer (null when this layout has none)
-    void* device_pointer(const std::string& name, size_t& bytes) const;
+    void* device_pointer(const std::string& name, size_t& bytes);
     // Reciprocal-space configuration: layout 0 automatic / 1 full grid, FFT backend 0
     // built-in / 1 rocFFT, and (grid != null) the grid dimensions at the same support;
     // rebuilds the per-frame data of the current positions.  Every configuration is the
@@ -342,8 +350,11 @@ class EwaldOp {
     int reg_rx = 0, reg_nrx = 0, reg_nry = 0, reg_npb = 1, reg_pblk = 0;
     bool reg_full = false;       // the regions tile the full grid (monodisperse dipoles)
     int reg_slots = 0;           // (region, candidate) slots of the current frame
+    RegionGeom region_geom(bool on_slab) const;
+    RegionSet region_set(bool on_slab) const;
     DevBuf<int> d_reg_start;
     DevBuf<int> d_reg_items;
+    DevBuf<int> d_reg_quads;     // quadrupole of each slot's particle (-1: none), quadrupole operator
     DevBuf<int> d_ps_start;      // [N + 1] region slots of each particle
     DevBuf<int> d_ps_items;      // slot ids (CSR positions of d_reg_items)
     DevBuf<double> d_regw64;     // [slot][row] region-local separable weights (FP64, FP32)
@@ -381,13 +392,27 @@ class EwaldOp {
     std::vector<int> qidx_h;          // [Q] particle of each quadrupole
     DevBuf<int> d_qidx, d_qmap;       // [Q], [N] (quadrupole slot or -1)
     mutable std::vector<double> h_pair_q;     // [M][7] quadrupole table values per pair
+    std::vector<int> qmap_h;          // [N] quadrupole of each particle (-1: none)
+    double quad_self_grad = 0;        // gradient self term
+    bool quads_full = false;          // applies stay on the full grid (requested, or used stage by stage)
+    // full grid: [V][16] khat, sc, scQ, scGP, scGQ, Qfactor[5], Qdot[4]
+    DevBuf<double> d_kq64;
+    DevBuf<float> d_kq32;
+    // slab: [nz / 2 + 1][column][4] sc, scQ, scGQ, 1 / k, and [nz / 2 + 1][32] cos, sin of the planes
+    DevBuf<double> d_kqs64, d_zcs64;
+    DevBuf<float> d_kqs32;
+    // the reference's stencils and table for callers that ask for their address
+    bool quad_stencils_valid = false, quad_coef_valid = false;
     DevBuf<double> d_sw64;            // [N][W^3] Gaussian weights (spread constant included)
     DevBuf<float> d_sw32;
-    DevBuf<double> d_kq64;            // [V][16] k-space: khat, sc, scQ, scGP, scGQ, Qfactor[5], Qdot[5]
-    DevBuf<float> d_kq32;
-    void setup_quad_stencils(const std::vector<double>& pos, int Nn);
+    void ensure_quad_stencils();
+    void ensure_quad_scale_coef();
+    void build_quad_tables();
+    void quads_on_full_grid();
     template <typename R>
     void launch_quads(const SlotTable& t, int B, int parts, hipStream_t s, int jacobi);
+    template <typename R>
+    void line_fft(void* grid, void* kgrid, int B, bool forward, hipStream_t s);
 
     // ---- direct field ----
     bool direct = false;

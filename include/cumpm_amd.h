@@ -190,8 +190,10 @@ mpm_status mpm_op_stage(mpm_op* op, int stage, const double* x, void* grid, doub
  * "neighbor_start" (int [N + 1] CSR), "neighbor_list" (int [M]), "perp_para" (complex-double
  * pairs (perp, para) [M]), "pair_coef" (double per-pair coefficients), "self_perp"
  * (polydisperse, double [N]), "scale_coef" (k-space table), "fe_grid" (the grid of the last
- * apply), "fes_grid" (the slab's transposed k-space buffer).  Unknown names fail with
- * MPM_ERR_INVALID_ARGUMENT. */
+ * apply), "fes_grid" (the slab's transposed k-space buffer).  With quadrupoles the stencil
+ * buffers and "scale_coef" are built when first asked for, and the first use of "fe_grid" or
+ * of a reciprocal stage moves the operator's applies to the full grid (before the next
+ * apply "fe_grid" is then NULL).  Unknown names fail with MPM_ERR_INVALID_ARGUMENT. */
 mpm_status mpm_op_device_pointer(const mpm_op* op, const char* name, void** ptr, size_t* bytes);
 
 /* mpm_op_apply that allocates no device memory.  No counterpart in the reference: it is

@@ -18,19 +18,19 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("grid,N,support,B,spread,contract", [
     # more than 64 candidates per region, partial last chunks, narrow batches
-    ((24, 22, 20), 1301, 8, 2, "spread_mfma_kernel<double, 4, 4, 16>", "contract_nb_mfma_kernel<double, 4, 4, true>"),
-    ((24, 22, 20), 1999, 8, 4, "spread_mfma_kernel<double, 4, 4, 16>", "contract_nb_mfma_kernel<double, 4, 4, true>"),
+    ((24, 22, 20), 1301, 8, 2, "spread_mfma_kernel<double, 4, 4, 16, 3>", "contract_nb_mfma_kernel<double, 4, 4, true, 3, double>"),
+    ((24, 22, 20), 1999, 8, 4, "spread_mfma_kernel<double, 4, 4, 16, 3>", "contract_nb_mfma_kernel<double, 4, 4, true, 3, double>"),
     # odd z length (4-byte grid loads), axes shorter than the stencil (folded weights)
-    ((23, 21, 19), 1500, 6, 3, "spread_mfma_kernel<double, 4, 4, 16>", "contract_nb_mfma_kernel<double, 4, 4, false>"),
-    ((7, 9, 20), 1100, 8, 5, "spread_mfma_kernel<double, 4, 4, 16>", "contract_nb_mfma_kernel<double, 4, 4, true>"),
+    ((23, 21, 19), 1500, 6, 3, "spread_mfma_kernel<double, 4, 4, 16, 3>", "contract_nb_mfma_kernel<double, 4, 4, false, 3, double>"),
+    ((7, 9, 20), 1100, 8, 5, "spread_mfma_kernel<double, 4, 4, 16, 3>", "contract_nb_mfma_kernel<double, 4, 4, true, 3, double>"),
     # enough blocks for 32 columns each
-    ((48, 48, 48), 900, 8, 30, "spread_mfma_kernel<double, 4, 4, 32>", "contract_nb_mfma_kernel<double, 4, 4, true>"),
+    ((48, 48, 48), 900, 8, 30, "spread_mfma_kernel<double, 4, 4, 32, 3>", "contract_nb_mfma_kernel<double, 4, 4, true, 3, double>"),
     # five stencil points: gathered per particle
-    ((24, 22, 20), 1999, 4, 4, "spread_mfma_kernel<double, 4, 4, 16>", "gather_kernel<double, 4, false>"),
+    ((24, 22, 20), 1999, 4, 4, "spread_mfma_kernel<double, 4, 4, 16, 3>", "gather_kernel<double, 4, false>"),
     # no more than a wave of particles per SIMD: gathered per particle
-    ((24, 22, 20), 701, 8, 2, "spread_mfma_kernel<double, 4, 4, 16>", "gather_kernel<double, 4, false>"),
+    ((24, 22, 20), 701, 8, 2, "spread_mfma_kernel<double, 4, 4, 16, 3>", "gather_kernel<double, 4, false>"),
     # one right-hand side on few regions: gathered per particle
-    ((24, 22, 20), 1999, 8, 1, "spread_mfma_kernel<double, 4, 4, 16>", "gather_kernel<double, 1, false>"),
+    ((24, 22, 20), 1999, 8, 1, "spread_mfma_kernel<double, 4, 4, 16, 3>", "gather_kernel<double, 1, false>"),
 ])
 def test_dense_full_grid_matches_oracle(grid, N, support, B, spread, contract):
     print(f"dense full grid {grid} N={N} support={support} B={B}", flush=True)
