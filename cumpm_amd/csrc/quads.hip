@@ -147,13 +147,6 @@ __global__ void quad_kslab_kernel(double* __restrict__ k64, float* __restrict__ 
     }
 }
 
-// v of the neighbouring lane (lane ^ 1), by a lane permutation within quads.
-__device__ __forceinline__ double swap_lane1(double v) {
-    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xF, 0xF, true);
-    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xF, 0xF, true);
-    return __hiloint2double(hi, lo);
-}
-
 // Slab: for every in-plane wave vector (column) and right-hand side, the z transform of the
 // 8 components from the Zs planes to all wave numbers, the coupling, and the transform back,
 // without a k-space grid in memory.  Two lanes per column and right-hand side, one for the real
@@ -461,7 +454,6 @@ void EwaldOp::launch_quads(const SlotTable& t, int B, int parts, hipStream_t s, 
     const bool fp32 = std::is_same<R, float>::value;
     CT* grid = reinterpret_cast<CT*>(cur_grid);
     CT* kgrid = reinterpret_cast<CT*>(cur_kgrid);
-    const R* regw = fp32 ? reinterpret_cast<const R*>(d_regw32.p) : reinterpret_cast<const R*>(d_regw64.p);
     const int Ni = (int)N;
     const RegionSet rs = region_set(slab);
     const RegionGeom rg = region_geom(slab);
@@ -470,7 +462,7 @@ void EwaldOp::launch_quads(const SlotTable& t, int B, int parts, hipStream_t s, 
                 MPM_ERR_UNSUPPORTED, "reciprocal grid too large for one transform call");
     if ((parts & MPM_PART_RECIP) && (phases & 1)) {
         ProfScope ps("spread", s, B);
-        region_spread<R, 8>(ps, s, rs, rg, t, B, regw, 3 * (size_t)N, grid);
+        region_spread<R, 8>(ps, s, rs, rg, t, B, d_regw64.p, 3 * (size_t)N, grid);
     }
     if ((parts & MPM_PART_RECIP) && (phases & 2)) {
         {

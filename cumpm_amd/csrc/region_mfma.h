@@ -24,6 +24,13 @@ __device__ inline double wave_sum(double v) {
     return v;
 }
 
+// v of the neighbouring lane (lane ^ 1), by a lane permutation within quads.
+__device__ __forceinline__ double swap_lane1(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+
 // ---- spread on the matrix cores ----
 //
 // For a region of RX x (planes) x 16 rows (slab: RX x 16 y over all slab planes;
@@ -217,21 +224,27 @@ __device__ inline RegionAt region_at(const RegionGeom& rg, int reg) {
 // CPB = 16 is the form for few blocks (spread_cpb): there a region's candidates come in
 // several chunks and nothing else hides their loads, so the next chunk's values and
 // weights are fetched while the current chunk's products run.
+// Weights of the spread: with quadrupoles FP64 rows, so that each product is rounded once
+// (the reference's stencils hold the rounded product), else the grid's type.
+template <typename R, int NC>
+using SpreadW = std::conditional_t<NC == 8, double, R>;
+
 template <typename R, int RX, int ZSB, int CPB, int NC>
-__global__ __launch_bounds__(256, sizeof(R) == 4 ? 4 : 2) void spread_mfma_kernel(SlotTable tab, int B, RegionGeom rg,
-                                                          const R* __restrict__ regw,
+__global__ __launch_bounds__(256, sizeof(R) == 4 ? (NC == 3 ? 4 : 3) : 2) void spread_mfma_kernel(SlotTable tab, int B, RegionGeom rg,
+                                                          const SpreadW<R, NC>* __restrict__ regw,
                                                           const int* __restrict__ reg_start,
                                                           const int* __restrict__ reg_items,
                                                           const int* __restrict__ reg_quads, size_t n3,
                                                           typename C2<R>::T* __restrict__ out) {
     using CT = typename C2<R>::T;
     using M = Mfma<R>;
+    using WR = SpreadW<R, NC>;
     using Sh = SpreadShape<ZSB, CPB>;
     constexpr int KC = kMfmaKC, ZH = Sh::ZH;
     constexpr bool PREFETCH = CPB == 16;
     using L = RegionW<RX, ZSB>;
     __shared__ R s_v[KC][CPB + 1];
-    __shared__ __align__(16) R s_w[KC][L::NW];
+    __shared__ __align__(16) WR s_w[KC][L::NW];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int cg = wave % (CPB / 16), pg = wave / (CPB / 16);
     const int reg = blockIdx.x;
@@ -285,14 +298,15 @@ __global__ __launch_bounds__(256, sizeof(R) == 4 ? 4 : 2) void spread_mfma_kerne
         for (int t = 0; t < TV; ++t)
             vv[t] = value(id[t], scok && tid / CPB + QS * t < cnt);
     };
-    auto load_wts = [&](int c0, R (&ww)[TW]) {
+    auto load_wts = [&](int c0, WR (&ww)[TW]) {
         const int n = min(KC, k1 - c0) * L::NW;
-        const R* w = regw + (size_t)c0 * L::NW;
+        const WR* w = regw + (size_t)c0 * L::NW;
 #pragma unroll
         for (int t = 0; t < TW; ++t) ww[t] = keep_if(w[min(tid + 256 * t, n - 1)], tid + 256 * t < n);
     };
     int id[TV];
-    R vv[TV], ww[TW];
+    R vv[TV];
+    WR ww[TW];
     if (PREFETCH && k0 < k1) {
         load_ids(k0, min(KC, k1 - k0), id);
         load_vals(min(KC, k1 - k0), id, vv);
@@ -316,7 +330,7 @@ __global__ __launch_bounds__(256, sizeof(R) == 4 ? 4 : 2) void spread_mfma_kerne
 #pragma unroll
             for (int t = 0; t < TV; ++t)
                 vc[t] = value(idc[t], scok && tid / CPB + QS * t < cnt);
-            stage_weights<R, RX, ZSB>(&s_w[0][0], cnt, regw + (size_t)c0 * L::NW);
+            stage_weights<WR, RX, ZSB>(&s_w[0][0], cnt, regw + (size_t)c0 * L::NW);
 #pragma unroll
             for (int t = 0; t < TV; ++t) s_v[tid / CPB + QS * t][scol] = vc[t];
         }
@@ -331,17 +345,17 @@ __global__ __launch_bounds__(256, sizeof(R) == 4 ? 4 : 2) void spread_mfma_kerne
             for (int ks = 0; ks < cnt; ks += 4) {
                 const int kq = ks + (lane >> 4);  // rows >= cnt hold zeros
                 const R a = s_v[kq][cg * 16 + M::rowcol(i)];
-                const R wy = s_w[kq][L::Y + i];
-                R wx[RX], wz[ZH];
+                const WR wy = s_w[kq][L::Y + i];
+                WR wx[RX], wz[ZH];
 #pragma unroll
                 for (int xi = 0; xi < RX; ++xi) wx[xi] = s_w[kq][L::X + xi] * wy;
 #pragma unroll
-                for (int p = 0; p < ZH; ++p) wz[p] = (p0 + p < ZSB) ? s_w[kq][L::Z + p0 + p] : R(0);
+                for (int p = 0; p < ZH; ++p) wz[p] = (p0 + p < ZSB) ? s_w[kq][L::Z + p0 + p] : WR(0);
                 // planes past Zs carry zero weights: no branch around the accumulators
 #pragma unroll
                 for (int p = 0; p < ZH; ++p) {
 #pragma unroll
-                    for (int xi = 0; xi < RX; ++xi) acc[xi][p] = M::mac(a, wx[xi] * wz[p], acc[xi][p]);
+                    for (int xi = 0; xi < RX; ++xi) acc[xi][p] = M::mac(a, (R)(wx[xi] * wz[p]), acc[xi][p]);
                 }
             }
         }
@@ -824,7 +838,7 @@ constexpr int kQuadSlabPlanes = 10;
 
 template <typename R, int NC>
 inline void region_spread(ProfScope& ps, hipStream_t s, const RegionSet& rs, const RegionGeom& rg, const SlotTable& t,
-                          int B, const R* regw, size_t n3, typename C2<R>::T* grid) {
+                          int B, const SpreadW<R, NC>* regw, size_t n3, typename C2<R>::T* grid) {
     // 32 columns per block, or 16 where a batch has no more, and on the full grid while those
     // blocks are fewer than eight per CU (7001 particles on 47 x 47 x 48, 5 right-hand sides:
     // 36.2 -> 28.8 us; the slab's regions hold about one chunk of candidates, which leaves
