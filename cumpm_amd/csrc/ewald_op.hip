@@ -1360,6 +1360,136 @@ __global__ __launch_bounds__(256) void line_fft2_kernel(const typename C2<R>::T*
     }
 }
 
+// Lines of a length with a prime factor above kMaxPrimeRadix, as a matrix product on the FP64
+// matrix cores: with s_j = x_j + x_{n-j} and d_j = x_j - x_{n-j} (j = 1 .. n/2),
+//   A_m = x_0 + sum_j s_j cos(2 pi j m / n),  B_m = sum_j d_j sin(2 pi j m / n),
+//   X_m = A_m -+ i B_m,  X_{n-m} = A_m +- i B_m  (upper signs: forward),
+// two real products of (n/2 + 1)^2 coefficients with 16 columns (the real and imaginary parts of
+// 8 lines) each.  FP64 products over either storage type: up to n of about 128 they take no
+// longer than the lines' memory traffic, and no precision is lost to the longer sums.
+//
+// A block's waves are MT row tiles of 16 times dft_waves / MT shares of the lines; a wave keeps
+// its tile's coefficients in registers over every line of the block and of the next sets
+// of lines (blocks walk sets with the grid's stride), so that the coefficients, four times
+// the lines' size at n = 47, are read once per wave.  (Read per group of 8 lines: 18-20 us an
+// axis of 47 x 47 x 48, 5 right-hand sides; the generic radix stage, which reads every input
+// of a radix from LDS for every output: 28-29 us; here 17-19 us; 12 right-hand sides on 127^3: an apply 7.0 -> 4.5 ms.)
+static constexpr int dft_waves(int MT) { return MT <= 2 ? 4 : MT; }
+
+template <typename R, bool INV, int MT>
+__global__ __launch_bounds__(64 * dft_waves(MT)) void line_dft_kernel(const typename C2<R>::T* in,
+                                                                      typename C2<R>::T* out, LineGeom gin,
+                                                                      LineGeom gout, int n,
+                                                                      const double2* __restrict__ tab, int TL,
+                                                                      int nsets) {
+    using CT = typename C2<R>::T;
+    using M = Mfma<double>;
+    constexpr int T = 64 * dft_waves(MT), SP = dft_waves(MT) / MT, KM = 4 * MT;
+    extern __shared__ unsigned char s_raw[];
+    const int ld = n | 1;  // odd line pitch: lines of consecutive lanes on distinct banks
+    CT* const bin = reinterpret_cast<CT*>(s_raw);
+    CT* const bout = bin + TL * ld;
+    __shared__ int s_lbi[32], s_lbo[32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int H = n / 2, KK = H / 4 + 1;  // KK <= KM
+    const int mt = wave % MT, share = wave / MT;
+    const int col = lane & 15, g = lane >> 4, part = lane & 1;
+    double wc[KM], ws[KM];
+#pragma unroll
+    for (int kk = 0; kk < KM; ++kk) {
+        const double2 w = tab[(size_t)(mt * KK + min(kk, KK - 1)) * 64 + lane];
+        wc[kk] = w.x;
+        ws[kk] = w.y;
+    }
+    const float rn = 1.0f / (float)n;
+    for (int set = blockIdx.x; set < nsets; set += gridDim.x) {
+        const int l0 = set * TL;
+        const int nl = min(TL, (int)gin.nlines - l0);
+        __syncthreads();  // the previous set has been stored
+        if (tid < nl) {
+            s_lbi[tid] = line_base32(gin, l0 + tid);
+            s_lbo[tid] = line_base32(gout, l0 + tid);
+        }
+        __syncthreads();
+        const int tot = __mul24(nl, n);
+        const float rnl = 1.0f / (float)nl;
+        // eight elements per thread in flight before the first is stored to LDS
+        const bool run_in = gin.elem_stride == 1;
+        const int esi = (int)gin.elem_stride;
+        for (int e0 = tid; e0 < tot; e0 += 8 * T) {
+            CT v[8];
+            int at[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int e = min(e0 + u * T, tot - 1);
+                int li, k;
+                if (run_in) fdivmod(e, n, rn, li, k);
+                else fdivmod(e, nl, rnl, k, li);
+                at[u] = __mul24(li, ld) + k;
+                v[u] = in[s_lbi[li] + (run_in ? k : __mul24(k, esi))];
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (e0 + u * T < tot) bin[at[u]] = v[u];
+        }
+        __syncthreads();
+        for (int cg = share; cg * 8 < nl; cg += SP) {
+            // columns past the set's last line repeat its first one and are not written
+            const int line = cg * 8 + (col >> 1);
+            const bool live = line < nl;
+            const int lb = 2 * (live ? line : 0) * ld + part;
+            const R* xr = reinterpret_cast<const R*>(bin) + lb;
+            typename M::V4 ac = {0.0, 0.0, 0.0, 0.0}, as = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int kk = 0; kk < KM; ++kk) {
+                if (kk < KK) {  // uniform
+                    // j past H meets zero coefficients; j = 0 and 2 j = n are their own
+                    // partners, with halved cosines
+                    const int j = min(4 * kk + g, H);
+                    const double xa = (double)xr[2 * j], xb = (double)xr[2 * (j ? n - j : 0)];
+                    ac = M::mac(wc[kk], xa + xb, ac);
+                    as = M::mac(ws[kk], xa - xb, as);
+                }
+            }
+            R* xo = reinterpret_cast<R*>(bout) + lb;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int m = mt * 16 + M::drow(g, r);
+                // the other part's B (real part: +B_im, imaginary part: -B_re; inverse: signs
+                // turned)
+                double b = swap_lane1(as[r]);
+                if ((part != 0) != INV) b = -b;
+                if (live && m <= H) {
+                    xo[2 * m] = (R)(ac[r] + b);
+                    if (m > 0 && 2 * m < n) xo[2 * (n - m)] = (R)(ac[r] - b);
+                }
+            }
+        }
+        __syncthreads();
+        if (gout.elem_stride == 1) {
+            for (int e = tid; e < tot; e += T) {
+                int li, k;
+                fdivmod(e, n, rn, li, k);
+                out[s_lbo[li] + k] = bout[__mul24(li, ld) + k];
+            }
+        } else {
+            const int es = (int)gout.elem_stride;
+            for (int e = tid; e < tot; e += T) {
+                int k, li;
+                fdivmod(e, nl, rnl, k, li);
+                out[s_lbo[li] + __mul24(k, es)] = bout[__mul24(li, ld) + k];
+            }
+        }
+    }
+}
+
+// Row tiles of 16 the product is compiled for (0: longer than any).
+static int dft_tiles(int n) {
+    for (int mt : {1, 2, 3, 4, 6, 8})
+        if (n / 2 + 1 <= 16 * mt) return mt;
+    return 0;
+}
+
 // Full grid ([B][3][nx][ny][nz], z lines contiguous): the forward z transform, the
 // Green's tensor projection f <- sc (f . k^) k^ and the inverse z transform in one
 // pass, after the forward x and y transforms and before the inverse ones (the
@@ -1553,6 +1683,8 @@ struct LineAxis {
     LinePlan plan{};
     int cls = 0;       // radix class of the compiled kernel
     bool two = false;  // two register stages: line_fft2_kernel
+    int dft = 0;       // row tiles of line_dft_kernel (0: not used)
+    DevBuf<double2> dft_tab;  // [tile][step][lane] (cos, sin) of its coefficient operand
     DevBuf<double2> tw64;
     DevBuf<float2> tw32;
     explicit LineAxis(int n) {
@@ -1573,6 +1705,29 @@ struct LineAxis {
             cls = std::max(cls, r <= 8 ? 0 : (r <= 16 ? 1 : 2));
         }
         two = plan.nstages == 2 && plan.radix[0] <= kMaxPrimeRadix && plan.radix[1] <= kMaxPrimeRadix;
+        bool generic = false;
+        for (int st = 0; st < plan.nstages; ++st) generic = generic || plan.radix[st] > kMaxPrimeRadix;
+        // only where the generic stage is of length n or n / 2 (124 = 31 x 4, FP64, 6
+        // right-hand sides: an apply 2.86 -> 3.28 ms; 94 = 47 x 2: 1.38 -> 1.23), and past 127
+        // (four tiles), where the product outgrows the memory traffic, only of length n (251,
+        // FP64, 2 right-hand sides: 21.9 -> 13.7 ms; 236 = 59 x 4: 5.6 -> 7.2)
+        if (generic && (plan.nstages == 1 || (n <= 127 && plan.nstages == 2 && n % 2 == 0 && plan.radix[0] * 2 == n)))
+            dft = dft_tiles(n);
+        if (dft) {
+            const int H = n / 2, KK = H / 4 + 1;
+            std::vector<double2> t((size_t)dft * KK * 64, make_double2(0.0, 0.0));
+            for (int mt = 0; mt < dft; ++mt)
+                for (int kk = 0; kk < KK; ++kk)
+                    for (int l = 0; l < 64; ++l) {
+                        const int m = mt * 16 + l % 16, j = 4 * kk + l / 16;
+                        if (m > H || j > H) continue;
+                        const double a = 2.0 * kPi * (double)((m * j) % n) / (double)n;
+                        const bool own = j == 0 || 2 * j == n;  // its own partner: counted twice by the kernel
+                        t[((size_t)mt * KK + kk) * 64 + l] = make_double2(own ? 0.5 * std::cos(a) : std::cos(a),
+                                                                          own ? 0.0 : std::sin(a));
+                    }
+            dft_tab.upload(t.data(), t.size());
+        }
         std::vector<double2> t64(n);
         std::vector<float2> t32(n);
         for (int k = 0; k < n; ++k) {
@@ -1682,6 +1837,38 @@ struct LineFft {
                     MPM_L2(true)
                 }
 #undef MPM_L2
+                MPM_HIP(hipGetLastError());
+                continue;
+            }
+            if (ax.dft) {
+                // sets of 32 lines, fewer for long lines (two buffers in 64 KB of LDS) and for few
+                // lines (below two blocks per CU); at most eight blocks per CU
+                int TL = 32;
+                while (TL > 8 && ((size_t)2 * TL * (n | 1) * sizeof(CT) > 64 * 1024 - 512 || gi.nlines / TL < 512)) TL /= 2;
+                const size_t lds = (size_t)2 * TL * (n | 1) * sizeof(CT);
+                const int nsets = (int)((gi.nlines + TL - 1) / TL);
+                const dim3 gd((unsigned)std::min(nsets, 2048));
+                pscope.kernel("line_dft_kernel", {type_name<R>(), tbool(!forward), std::to_string(ax.dft)});
+#define MPM_DFT(MTV)                                                                                               \
+    case MTV:                                                                                                      \
+        if (forward)                                                                                               \
+            hipLaunchKernelGGL((line_dft_kernel<R, false, MTV>), gd, dim3(64 * dft_waves(MTV)), lds, s, in, out,   \
+                               gi, go, n, ax.dft_tab.p, TL, nsets);                                                \
+        else                                                                                                       \
+            hipLaunchKernelGGL((line_dft_kernel<R, true, MTV>), gd, dim3(64 * dft_waves(MTV)), lds, s, in, out,    \
+                               gi, go, n, ax.dft_tab.p, TL, nsets);                                                \
+        break;
+                switch (ax.dft) {
+                    MPM_DFT(1)
+                    MPM_DFT(2)
+                    MPM_DFT(3)
+                    MPM_DFT(4)
+                    MPM_DFT(6)
+                    MPM_DFT(8)
+                    default:
+                        throw Error(MPM_ERR_RUNTIME, "transform length out of range");
+                }
+#undef MPM_DFT
                 MPM_HIP(hipGetLastError());
                 continue;
             }
