@@ -1490,19 +1490,19 @@ static int dft_tiles(int n) {
     return 0;
 }
 
-// Full grid ([B][3][nx][ny][nz], z lines contiguous): the forward z transform, the
+// Full grid ([B][NC][nx][ny][nz], z lines contiguous): the forward z transform, the
 // Green's tensor projection f <- sc (f . k^) k^ and the inverse z transform in one
 // pass, after the forward x and y transforms and before the inverse ones (the
 // axes' transforms commute), so that the grid is read and written once for the
 // three steps instead of three times.  A block takes TL z lines of each of the
-// three components of one right-hand side (the projection couples them per
+// NC components (three; or one, the polydisperse operator's scalar grid, f <- sc f) of one right-hand side (the projection couples them per
 // k-point), both register stages of each transform as line_fft2_kernel, all in one
 // LDS buffer y: forward stage 1 from the grid into y, forward stage 2 in place
 // (each butterfly writes the elements it read), the projection in place, inverse
 // stage 1 with every thread's inputs read before any output is written (one
 // butterfly per thread: 3 TL P2 <= 256), inverse stage 2 from y to the grid.  kc
-// holds (k^x, k^y, k^z, sc) per voxel.
-template <typename R, int CLS>
+// holds (k^x, k^y, k^z, sc) per voxel, or sc alone.  FP64 as FP32: one kernel for three.
+template <typename R, int CLS, int NC>
 __global__ __launch_bounds__(256) void zline_scale_kernel(typename C2<R>::T* grid, int B, int nxy, int n,
                                                           int P1, int P2,
                                                           const typename C2<R>::T* __restrict__ twiddle, int TL,
@@ -1513,13 +1513,13 @@ __global__ __launch_bounds__(256) void zline_scale_kernel(typename C2<R>::T* gri
     // a line in LDS is P2 rows of P1 + 1 (padded: no bank conflicts in stage 1); after
     // the forward transform element k of a line sits at row k / P1, column k % P1
     const int ln = (n + P2) | 1;  // odd pitch: lines of consecutive lanes on distinct banks
-    CT* const y = reinterpret_cast<CT*>(s_raw);  // [3 TL][ln]
-    CT* const tw = y + 3 * TL * ln;              // forward twiddles, then their conjugates
+    CT* const y = reinterpret_cast<CT*>(s_raw);  // [NC TL][ln]
+    CT* const tw = y + NC * TL * ln;              // forward twiddles, then their conjugates
     CT* const twi = tw + n;
     const int tid = threadIdx.x;
     const int l0 = blockIdx.x * TL;
     const int nl = min(TL, B * nxy - l0);
-    const int nt = 3 * nl;  // block lines t = c nl + li
+    const int nt = NC * nl;  // block lines t = c nl + li
     for (int k = tid; k < n; k += blockDim.x) {
         const CT w = twiddle[k];
         tw[k] = w;
@@ -1529,12 +1529,12 @@ __global__ __launch_bounds__(256) void zline_scale_kernel(typename C2<R>::T* gri
     }
     // line L = xy B + b: the right-hand sides of one (x, y) follow each other, so
     // that its k-space coefficients are read from memory once, not once per b
-    __shared__ int s_base[3 * 64];  // grid offset of each block line
+    __shared__ int s_base[NC * 64];  // grid offset of each block line
     __shared__ int s_vox[64];       // voxel (x, y, 0) of each line
     if (tid < nt) {
         const int c = tid / nl, li = tid - c * nl;
         const int L = l0 + li, xy = L / B, b = L - xy * B;
-        s_base[tid] = ((b * 3 + c) * nxy + xy) * n;
+        s_base[tid] = ((b * NC + c) * nxy + xy) * n;
         if (c == 0) s_vox[li] = xy * n;
     }
     __syncthreads();
@@ -1578,9 +1578,14 @@ __global__ __launch_bounds__(256) void zline_scale_kernel(typename C2<R>::T* gri
         const int v = s_vox[li] + k;
         int kq, ka;
         fdivmod(k, P1, r1, kq, ka);
+        CT* f0 = y + li * ln + kq * (P1 + 1) + ka;
+        if constexpr (NC == 1) {
+            const R sc = kc[v];
+            f0->x *= sc;
+            f0->y *= sc;
+        } else {
         const R kx = kc[4 * (size_t)v], ky = kc[4 * (size_t)v + 1], kz = kc[4 * (size_t)v + 2],
                 sc = kc[4 * (size_t)v + 3];
-        CT* f0 = y + li * ln + kq * (P1 + 1) + ka;
         CT* f1 = f0 + nl * ln;
         CT* f2 = f1 + nl * ln;
         const CT a0 = *f0, a1 = *f1, a2 = *f2;
@@ -1596,6 +1601,7 @@ __global__ __launch_bounds__(256) void zline_scale_kernel(typename C2<R>::T* gri
         o.x = dr * kz;
         o.y = di * kz;
         *f2 = o;
+        }
     }
     __syncthreads();
     // inverse stage 1: butterfly (t, j) of radix P1 reads y[t n + j + r P2] and writes
@@ -1607,7 +1613,7 @@ __global__ __launch_bounds__(256) void zline_scale_kernel(typename C2<R>::T* gri
         CT v[PMAX];
 #pragma unroll
         for (int r = 0; r < PMAX; ++r)
-            if (act && r < P1) {
+            if (r < P1) {  // uniform; threads without a butterfly read line 0's
                 int kq, ka;
                 fdivmod(j + r * P2, P1, r1, kq, ka);
                 v[r] = y[t * ln + kq * (P1 + 1) + ka];
@@ -1757,6 +1763,7 @@ struct LineFft {
     std::vector<std::unique_ptr<LineAxis>> axes;
     std::vector<LinePass> fwd, inv;
     long long rhs_elems = 0;  // elements per RHS (grid size)
+    int comps = 0;            // components of a right-hand side on the full grid (0: slab)
     int kt_x = -1;            // transposed slab layout: the axis of the contiguous x lines
     int full_z = -1;          // full grid: the axis of the contiguous z lines
 
@@ -1808,14 +1815,39 @@ struct LineFft {
         using CT = typename C2<R>::T;
         MPM_REQUIRE((long long)B * rhs_elems < (1LL << 31), MPM_ERR_UNSUPPORTED,
                     "reciprocal grid too large for one transform call");
+        // In-place passes over whole components (the full grid) of a batch of several times the
+        // last-level cache (256 MB) run chunk by chunk of components: all passes of a chunk
+        // follow each other, so that the second finds the first's output in the cache (256^3,
+        // 12 right-hand sides, 4.8 GB: an apply 13.65 -> 12.23 ms; at 0.7 GB no gain)
+        const bool in_place = comps > 0 && std::all_of(fwd.begin(), fwd.end(), [](const LinePass& q) {
+            return q.src == 0 && q.dst == 0;
+        });
+        const long long total = in_place ? (long long)comps * B : 1;
+        long long chunk = total;
+        if (in_place) {
+            const long long comp_bytes = rhs_elems / comps * (long long)sizeof(CT);
+            if (total * comp_bytes > (1ll << 30)) chunk = std::max(1ll, (224ll << 20) / comp_bytes);
+        }
+        for (long long c0 = 0; c0 < total; c0 += chunk) {
+            const long long cn = std::min(chunk, total - c0);
+            exec_passes<R>(grid + (in_place ? c0 * (rhs_elems / comps) : 0), kgrid, B, forward, s, skip_axis,
+                           in_place ? cn : B, in_place ? comps : 1);
+        }
+    }
+
+    // The passes of `units` units of lines, a right-hand side holding `per` of them.
+    template <typename R>
+    void exec_passes(typename C2<R>::T* grid, typename C2<R>::T* kgrid, int B, bool forward, hipStream_t s, int skip_axis,
+                     long long units, long long per) {
+        using CT = typename C2<R>::T;
         static const char* kPassNames[] = {"fft_axis0", "fft_axis1", "fft_axis2"};
         for (const LinePass& ps : (forward ? fwd : inv)) {
             if (ps.axis == skip_axis) continue;
             ProfScope pscope(kPassNames[std::min(ps.axis, 2)], s, B);
             LineAxis& ax = *axes[ps.axis];
             LineGeom gi = ps.gin, go = ps.gout;
-            gi.nlines *= B;
-            go.nlines *= B;
+            gi.nlines = gi.nlines / per * units;
+            go.nlines = go.nlines / per * units;
             const int n = ax.plan.n;
             const CT* tw = std::is_same<R, float>::value ? reinterpret_cast<const CT*>(ax.tw32.p)
                                                          : reinterpret_cast<const CT*>(ax.tw64.p);
@@ -4825,6 +4857,7 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
             }
         } else {  // [comps][nx][ny][nz]: z, y, x lines in place (one component for the polydisperse grid)
             lf->rhs_elems = nc * nxy * nzz;
+            lf->comps = (int)nc;
             const LineGeom gz{nc * nxy, 1, 0, nzz, 1};
             const LineGeom gy{nc * nx * nzz, nzz, 1, (long long)ny * nzz, nzz};
             const LineGeom gx{nc * ny * nzz, (long long)ny * nzz, 1, nxy * nzz, (long long)ny * nzz};
@@ -4904,6 +4937,42 @@ size_t EwaldOp::grid_elems_per_rhs() const {
 size_t EwaldOp::kgrid_elems_per_rhs() const { return (quads ? 8 : 3) * (size_t)Zs * kspace_cols(); }
 // columns of one slab plane in the k-space buffer (padding columns included)
 int EwaldOp::kspace_cols() const { return kt ? S.n[1] * nxp : S.n[0] * S.n[1]; }
+
+// z lines per component and block of zline_scale_kernel (0: not for this length): within its
+// LDS (padded lines, twiddles and their conjugates, 1 KB of line tables), one inverse stage-1
+// butterfly per thread, and about 10 KB of FP32 lines per component (measured at 256^3 with
+// three components: 5 lines 2.39 ms, 3 lines 2.55 ms).
+template <typename CT>
+static int zline_lines(const LineAxis& ax, int nc) {
+    if (!ax.two) return 0;
+    const LinePlan& pl = ax.plan;
+    const size_t per_line = nc * (size_t)((pl.n + pl.radix[1]) | 1) * sizeof(CT);
+    const size_t fixed = 2 * (size_t)pl.n * sizeof(CT) + 1024;
+    const int by_lds = kMaxFusedLds > fixed ? (int)((kMaxFusedLds - fixed) / per_line) : 0;
+    return std::min({by_lds, 256 / (nc * pl.radix[1]), std::max(1, 1280 * 3 / (nc * pl.n)), 64});
+}
+
+template <typename R, int NC>
+static void zline_launch(ProfScope& ps, hipStream_t s, const LineAxis& ax, typename C2<R>::T* grid, int B, int nxy,
+                         int ztl, const R* kc) {
+    using CT = typename C2<R>::T;
+    const LinePlan& pl = ax.plan;
+    const size_t lds = (NC * (size_t)ztl * ((pl.n + pl.radix[1]) | 1) + 2 * (size_t)pl.n) * sizeof(CT);
+    const CT* tw = std::is_same<R, float>::value ? reinterpret_cast<const CT*>(ax.tw32.p)
+                                                 : reinterpret_cast<const CT*>(ax.tw64.p);
+    const dim3 gz((unsigned)(((long long)nxy * B + ztl - 1) / ztl));
+    ps.kernel("zline_scale_kernel", {type_name<R>(), std::to_string(ax.cls), std::to_string(NC)});
+    if (ax.cls == 0)
+        hipLaunchKernelGGL((zline_scale_kernel<R, 0, NC>), gz, dim3(256), lds, s, grid, B, nxy, pl.n, pl.radix[0],
+                           pl.radix[1], tw, ztl, kc);
+    else if (ax.cls == 1)
+        hipLaunchKernelGGL((zline_scale_kernel<R, 1, NC>), gz, dim3(256), lds, s, grid, B, nxy, pl.n, pl.radix[0],
+                           pl.radix[1], tw, ztl, kc);
+    else
+        hipLaunchKernelGGL((zline_scale_kernel<R, 2, NC>), gz, dim3(256), lds, s, grid, B, nxy, pl.n, pl.radix[0],
+                           pl.radix[1], tw, ztl, kc);
+    MPM_HIP(hipGetLastError());
+}
 
 RegionGeom EwaldOp::region_geom(bool on_slab) const {
     RegionGeom rg;
@@ -4994,21 +5063,13 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
             const int xaxis = (SLAB && zcontig && kt && lfft && fft_backend == 0) ? lfft->kt_x : -1;
             const size_t xlds = (size_t)(3 * Zs + 2) * S.n[0] * sizeof(CT);
             const bool fusedx = fp32 && xaxis >= 0 && lfft->axes[xaxis]->two && xlds <= kMaxFusedLds;
-            // full grid (FP32, built-in transform, two-stage z lines): the z transforms and
-            // the Green's tensor in one pass over z lines of three components
-            const int zaxis = (!SLAB && fp32 && lfft && fft_backend == 0) ? lfft->full_z : -1;
-            int ztl = 0;
-            if (zaxis >= 0 && lfft->axes[zaxis]->two) {
-                const LinePlan& pl = lfft->axes[zaxis]->plan;
-                const size_t per_line = 3 * (size_t)((pl.n + pl.radix[1]) | 1) * sizeof(CT);  // padded, 3 components
-                // twiddles and their conjugates, and 1 KB of the kernel's static line tables
-                const size_t fixed = 2 * (size_t)pl.n * sizeof(CT) + 1024;
-                const int by_lds = kMaxFusedLds > fixed ? (int)((kMaxFusedLds - fixed) / per_line) : 0;
-                const int by_threads = 256 / (3 * pl.radix[1]);  // one inverse stage-1 butterfly per thread
-                // about 10 KB of lines per component and block (measured at 256^3 with
-                // padded rows: 5 lines 2.39 ms, 3 lines 2.55 ms)
-                ztl = std::min({by_lds, by_threads, std::max(1, 1280 / pl.n)});
-            }
+            // full grid (built-in transform, two-stage z lines): the z transforms and the
+            // Green's tensor in one pass over z lines of three components
+            const int zaxis = (!SLAB && lfft && fft_backend == 0) ? lfft->full_z : -1;
+            // (FP64 from 64 MB of grid: 256^3, 4 right-hand sides, an apply 8.70 -> 7.41 ms; on 32^3
+            // with one the three small kernels take 0.7 us less than its many registers)
+            const bool zworth = fp32 || (size_t)B * bytes_per_rhs >= ((size_t)64 << 20);
+            const int ztl = zaxis >= 0 && zworth ? zline_lines<CT>(*lfft->axes[zaxis], 3) : 0;
             const bool fusedz = ztl >= 1;
             const int skip = fusedx ? xaxis : (fusedz ? zaxis : -1);
             {
@@ -5020,24 +5081,8 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
             }
             if (fusedz) {
                 ProfScope ps("scale", s, B);
-                const LineAxis& ax = *lfft->axes[zaxis];
-                const int nxy = S.n[0] * S.n[1], nlines = nxy * B;
-                const size_t lds =
-                    (3 * (size_t)ztl * ((ax.plan.n + ax.plan.radix[1]) | 1) + 2 * (size_t)ax.plan.n) * sizeof(CT);
-                const CT* tw = reinterpret_cast<const CT*>(ax.tw32.p);
-                const R* kc = reinterpret_cast<const R*>(d_k32.p);
-                const dim3 gz((unsigned)((nlines + ztl - 1) / ztl));
-                ps.kernel("zline_scale_kernel", {type_name<R>(), std::to_string(ax.cls)});
-                if (ax.cls == 0)
-                    hipLaunchKernelGGL((zline_scale_kernel<R, 0>), gz, dim3(256), lds, s, grid, B, nxy,
-                                       ax.plan.n, ax.plan.radix[0], ax.plan.radix[1], tw, ztl, kc);
-                else if (ax.cls == 1)
-                    hipLaunchKernelGGL((zline_scale_kernel<R, 1>), gz, dim3(256), lds, s, grid, B, nxy,
-                                       ax.plan.n, ax.plan.radix[0], ax.plan.radix[1], tw, ztl, kc);
-                else
-                    hipLaunchKernelGGL((zline_scale_kernel<R, 2>), gz, dim3(256), lds, s, grid, B, nxy,
-                                       ax.plan.n, ax.plan.radix[0], ax.plan.radix[1], tw, ztl, kc);
-                MPM_HIP(hipGetLastError());
+                const R* kc = fp32 ? reinterpret_cast<const R*>(d_k32.p) : reinterpret_cast<const R*>(d_k64.p);
+                zline_launch<R, 3>(ps, s, *lfft->axes[zaxis], grid, B, S.n[0] * S.n[1], ztl, kc);
             } else if (fusedx) {
                 ProfScope ps("zfused", s, B);
                 const CT* T = reinterpret_cast<const CT*>(d_toe32.p);
@@ -5236,22 +5281,29 @@ void EwaldOp::launch_poly(const SlotTable& t, int B, int parts, hipStream_t s, i
         MPM_HIP(hipGetLastError());
     }
     if ((parts & MPM_PART_RECIP) && (phases & 2)) {
+        const int zaxis = lfft->full_z;
+        const int ztl = zaxis >= 0 ? zline_lines<CT>(*lfft->axes[zaxis], 1) : 0;
+        const int skip = ztl >= 1 ? zaxis : -1;
+        const R* kc = fp32 ? reinterpret_cast<const R*>(d_k32.p) : reinterpret_cast<const R*>(d_k64.p);
         {
             ProfScope ps("fft", s, B);
-            lfft->exec<R>(grid, grid, B, true, s);
+            lfft->exec<R>(grid, grid, B, true, s, skip);
         }
         {
             ProfScope ps("scale", s, B);
-            ps.kernel("poly_scale_kernel", {type_name<R>()});
-            const R* kc = fp32 ? reinterpret_cast<const R*>(d_k32.p) : reinterpret_cast<const R*>(d_k64.p);
-            const size_t total = (size_t)B * V;
-            const int blocks = (int)std::min<size_t>((total + 255) / 256, 16384);
-            hipLaunchKernelGGL((poly_scale_kernel<R>), dim3(blocks), dim3(256), 0, s, grid, kc, V, total);
-            MPM_HIP(hipGetLastError());
+            if (ztl >= 1) {
+                zline_launch<R, 1>(ps, s, *lfft->axes[zaxis], grid, B, S.n[0] * S.n[1], ztl, kc);
+            } else {
+                ps.kernel("poly_scale_kernel", {type_name<R>()});
+                const size_t total = (size_t)B * V;
+                const int blocks = (int)std::min<size_t>((total + 255) / 256, 16384);
+                hipLaunchKernelGGL((poly_scale_kernel<R>), dim3(blocks), dim3(256), 0, s, grid, kc, V, total);
+                MPM_HIP(hipGetLastError());
+            }
         }
         {
             ProfScope ps("fft", s, B);
-            lfft->exec<R>(grid, grid, B, false, s);
+            lfft->exec<R>(grid, grid, B, false, s, skip);
         }
     }
     if (!(phases & 4)) return;

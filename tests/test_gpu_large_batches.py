@@ -1,0 +1,62 @@
+"""Full-grid batches of several times the last-level cache, whose transforms run chunk by chunk
+of components, against the same systems one at a time (FP32 1e-6 and FP64 1e-12 of the largest
+value: only the z pass's grouping of lines differs), with the fused z pass in both precisions;
+and the polydisperse operator's fused z pass against the oracle (FP64 1e-11, FP32 1e-5)."""
+import numpy as np
+import pytest
+
+from cumpm_amd import _capi as C
+from oracle import oracle as O
+from gpu_helpers import Op, rel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision,grid,B,tol,kernel", [
+    (C.PREC_MIXED, (256, 256, 256), 3, 1e-6, "zline_scale_kernel<float, 1, 3>"),  # 1.2 GB
+    (C.PREC_DOUBLE, (128, 180, 128), 9, 1e-12, "zline_scale_kernel<double, 1, 3>"),  # 1.3 GB, partial last chunk
+])
+def test_chunked_transforms_equal_single_systems(precision, grid, B, tol, kernel):
+    print(f"chunked transforms {grid} B={B}", flush=True)
+    rng = np.random.default_rng(47)
+    L = [40.0, 41.0, 42.0]
+    N = 60
+    pos = rng.uniform(0, 1, (N, 3)) * L
+    op = Op(L, 1e-6, 0.5, grid=grid, support=8, layout=1)
+    op.set_positions(pos)
+    op.set_self_coef(np.full(N, 0.2 - 0.1j))
+    p = rng.standard_normal((B, N, 3)) + 1j * rng.standard_normal((B, N, 3))
+    C.profile_reset()
+    C.profile_enable(True)
+    y = op.apply(p, precision, C.PART_RECIP)
+    C.profile_enable(False)
+    assert kernel in C.profile_names(), C.profile_names()
+    for b in (0, B // 2, B - 1):
+        assert rel(op.apply(p[b], precision, C.PART_RECIP)[0], y[b]) < tol
+
+
+@pytest.mark.parametrize("grid,B", [((40, 36, 48), 3), ((36, 40, 38), 5), ((36, 40, 47), 1)])
+def test_polydisperse_z_pass_matches_oracle(grid, B):
+    print(f"poly z pass {grid} B={B}", flush=True)
+    rng = np.random.default_rng(53)
+    L = [24.0, 25.0, 26.0]
+    N = 30
+    pos = rng.uniform(0, 1, (N, 3)) * L
+    rad = rng.uniform(1.0, 2.0, N)
+    op = Op(L, 1e-4, 0.5, grid=grid, radii=rad)
+    op.set_positions(pos)
+    sc = np.full(N, -0.2 + 0.1j)
+    op.set_self_coef(sc)
+    p = rng.standard_normal((B, N, 3)) + 1j * rng.standard_normal((B, N, 3))
+    C.profile_reset()
+    C.profile_enable(True)
+    y = op.apply(p, C.PREC_DOUBLE)
+    C.profile_enable(False)
+    fused = any(n.startswith("zline_scale_kernel<double") for n in C.profile_names())
+    assert fused == (grid[2] != 47)  # a prime above 23 has no two register stages
+    ref = O.PolyOperator(L, 1e-4, 0.5, rad, grid=list(grid))
+    ref.set_positions(pos)
+    for b in sorted({0, B - 1}):
+        assert rel(y[b], ref.apply(p[b], sc)) < 1e-11
+    r64 = op.apply(p, C.PREC_DOUBLE, C.PART_RECIP)
+    assert rel(op.apply(p, C.PREC_MIXED, C.PART_RECIP), r64) < 1e-5
