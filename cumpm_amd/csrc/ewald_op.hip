@@ -4038,7 +4038,10 @@ void EwaldOp::set_bloch(double kx, double ky) {
 //
 // The host keeps the O(N) cell lists (members in ascending index) and each particle's
 // cell; the device visits, for every particle i, the 27 cells around its own in the
-// host's order (dz, dy, dx = -1..1) and their members in order, so the CSR it builds is
+// host's order (dz, dy, dx = -1..1) and their members in order, a wave per particle and a
+// candidate per lane (4000 particles of a monolayer
+// 247 -> 30 us a pass, 7001 at 67 neighbours each 562 -> 81, 100,000 at 19 each, whose runs fill
+// a quarter of the lanes, 334 -> 452; a thread per particle before), so the CSR it builds is
 // the host's.  Pass 0 counts each particle's pairs, pass 1 fills them in: the neighbour,
 // x_j - x_i (minimum image), the table values (perp, para) at d_eff = max(d, 1) and, with
 // quadrupoles, the seven quadrupole table values (monodisperse_ewald_electric_field.cu
@@ -4073,21 +4076,27 @@ __global__ __launch_bounds__(256) void nb_search_kernel(int pass, int N, const d
                                                         int* __restrict__ nb_j, double* __restrict__ pair_r,
                                                         double2* __restrict__ nb_f, double* __restrict__ pair_q,
                                                         const double* __restrict__ tab) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
+    const int lane = threadIdx.x & 63;
+    const int i = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    if (i >= N) return;  // whole wave
     const double xi = pos[i], yi = pos[N + i], zi = pos[2 * N + i];
-    int k = pass ? nb_start[i] : 0;
+    int first = pass ? nb_start[i] : 0;  // the row's next free entry, the same in every lane
     int cnt = 0;
-    auto consider = [&](int j) {
+    // one candidate per lane (valid: this lane has one); accepted ones take consecutive entries
+    // in lane order
+    auto consider = [&](int j, bool valid) {
         double r[3] = {xi - pos[j], yi - pos[N + j], zi - pos[2 * N + j]};
 #pragma unroll
         for (int d = 0; d < 3; ++d) r[d] -= g.L[d] * round(r[d] / g.L[d]);
         const double d2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
-        if (!(d2 <= g.rc2)) return;
         const double dist = sqrt(d2);
-        if (!(dist < g.rc)) return;
-        ++cnt;
+        const bool take = valid && d2 <= g.rc2 && dist < g.rc;
+        const unsigned long long mask = __ballot(take);
+        cnt += __popcll(mask);
         if (!pass) return;
+        const int k = first + __popcll(mask & ((1ull << lane) - 1ull));
+        first += __popcll(mask);
+        if (!take) return;
         nb_j[k] = j;
         const double de = dist < 1.0 ? 1.0 : dist;
         nb_f[k] = make_double2(tab_interp(tab, g.ts, de), tab_interp(tab + g.ts, g.ts, de));
@@ -4098,26 +4107,29 @@ __global__ __launch_bounds__(256) void nb_search_kernel(int pass, int N, const d
             rj[d] -= g.L[d] * round(rj[d] / g.L[d]);
             pair_r[3 * (size_t)k + d] = rj[d];
         }
-        ++k;
     };
     if (g.cells) {
         const int cx = cellc[3 * i], cy = cellc[3 * i + 1], cz = cellc[3 * i + 2];
+        // the three cells along x follow each other in the lists: one run of members, unless
+        // the row wraps around the box
+        const bool run = cx > 0 && cx < g.nc[0] - 1;
         for (int dz = -1; dz <= 1; ++dz)
-            for (int dy = -1; dy <= 1; ++dy)
-                for (int dx = -1; dx <= 1; ++dx) {
-                    const int a = (cx + dx + g.nc[0]) % g.nc[0], b = (cy + dy + g.nc[1]) % g.nc[1],
-                              c = (cz + dz + g.nc[2]) % g.nc[2];
-                    const int cell = (c * g.nc[1] + b) * g.nc[0] + a;
-                    for (int m = cell_start[cell]; m < cell_start[cell + 1]; ++m) {
-                        const int j = cell_items[m];
-                        if (j != i) consider(j);
+            for (int dy = -1; dy <= 1; ++dy) {
+                const int b = (cy + dy + g.nc[1]) % g.nc[1], c = (cz + dz + g.nc[2]) % g.nc[2];
+                const int row = (c * g.nc[1] + b) * g.nc[0];
+                for (int dx = -1; dx <= (run ? -1 : 1); ++dx) {
+                    const int cell = row + (cx + dx + g.nc[0]) % g.nc[0];
+                    const int m1 = cell_start[cell + (run ? 3 : 1)];
+                    for (int m0 = cell_start[cell]; m0 < m1; m0 += 64) {
+                        const int j = cell_items[min(m0 + lane, m1 - 1)];
+                        consider(j, m0 + lane < m1 && j != i);
                     }
                 }
+            }
     } else {
-        for (int j = 0; j < N; ++j)
-            if (j != i) consider(j);
+        for (int j0 = 0; j0 < N; j0 += 64) consider(min(j0 + lane, N - 1), j0 + lane < N && j0 + lane != i);
     }
-    if (!pass) count[i] = cnt;
+    if (!pass && lane == 0) count[i] = cnt;
 }
 
 // Per-pair coefficients (u = (x_j - x_i) / d_eff, perp, para - perp, the Bloch phase
@@ -4183,7 +4195,7 @@ void EwaldOp::search_pairs_device(const std::vector<double>& pos, int Nn, bool c
     g.nq = nq;
     d_nb_count.resize((size_t)Nn + 1);
     d_nb_start.resize((size_t)Nn + 1);
-    const dim3 grid((unsigned)((Nn + 255) / 256));
+    const dim3 grid((unsigned)((Nn + 3) / 4));  // a wave per particle
     hipLaunchKernelGGL(nb_search_kernel, grid, dim3(256), 0, nullptr, 0, Nn, d_pos.p, g, d_cellc.p, d_cell_start.p,
                        d_cell_items.p, (const int*)nullptr, d_nb_count.p, (int*)nullptr, (double*)nullptr,
                        (double2*)nullptr, (double*)nullptr, d_ptab.p);
