@@ -9,20 +9,20 @@
 // does not:
 //
 //  * layout  — thin films run on a slab of the occupied z-planes (the z transform is
-//              replaced by a Toeplitz coupling of those planes); other geometries,
-//              quadrupoles and the polydisperse operator on the full grid.
+//              replaced by a Toeplitz coupling of those planes; quadrupoles: quads.hip);
+//              other geometries and the polydisperse operator on the full grid.
 //  * spread  — region products on the matrix cores (spread_mfma_kernel, separable
 //              weights V^T W^T per region, every voxel written once): x by 16-row
-//              y regions over all slab planes, or 4 x 8 x 16 (x, y, z) regions on the
-//              full grid (monodisperse dipoles); owner-computes tiles that pull in the
-//              binned particles where the regions do not apply (small full grids,
-//              quadrupoles, polydisperse); no atomics, in place of the reference's
+//              y regions over all slab planes, or 4 x 8 (or 4) x 16 (x, y, z) regions on
+//              the full grid (region_mfma.h); the polydisperse operator and grids past
+//              2^31 elements gather per voxel; no atomics, in place of the reference's
 //              atomic scatter (:1160-1298).
-//  * FFT     — the built-in batched LDS line FFT (register radices 2-23, a generic
-//              stage beyond; lines held in LDS with padded rows), 2-D on the slab with a
+//  * FFT     — the built-in batched LDS line FFT (register radices 2-23; prime and
+//              twice-prime lengths beyond as matrix products, a generic stage for the
+//              rest; lines held in LDS with padded rows), 2-D on the slab with a
 //              transposed k-space buffer and 3-D on the full grid; rocFFT as an
 //              alternative back-end.
-//  * scale   — full grid: the Green's tensor projection per voxel (:1406-1432), in FP32
+//  * scale   — full grid: the Green's tensor projection per voxel (:1406-1432), mostly
 //              fused with the forward and inverse z transforms (zline_scale_kernel);
 //              slab: xtoeplitz_kernel fuses the x transform, the plane coupling and the
 //              inverse x transform (FP32), ztoeplitz / zfused kernels otherwise.
