@@ -3971,6 +3971,7 @@ void EwaldOp::build_kspace() {
 }
 
 void EwaldOp::ensure_kspace_table() {
+    if (quads && slab) build_quad_phases();
     const int key = quads ? 6000 + (slab ? Zs : 0) : (poly ? 5000 : (!slab ? 0 : (zcontig ? 2 + Zs : 1) + (kt ? 1000 : 0)));
     if (kspace_ready && kspace_key == key) return;
     const int threads = 256;

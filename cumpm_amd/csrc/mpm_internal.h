@@ -401,6 +401,8 @@ class EwaldOp {
     // slab: [nz / 2 + 1][column][4] sc, scQ, scGQ, 1 / k, and [nz / 2 + 1][32] cos, sin of the planes
     DevBuf<double> d_kqs64, d_zcs64;
     DevBuf<float> d_kqs32;
+    std::vector<int> zcs_planes;      // the planes and z length that d_zcs64 was built for
+    int zcs_nz = 0;
     // the reference's stencils and table for callers that ask for their address
     bool quad_stencils_valid = false, quad_coef_valid = false;
     DevBuf<double> d_sw64;            // [N][W^3] Gaussian weights (spread constant included)
@@ -408,6 +410,7 @@ class EwaldOp {
     void ensure_quad_stencils();
     void ensure_quad_scale_coef();
     void build_quad_tables();
+    void build_quad_phases();
     void quads_on_full_grid();
     template <typename R>
     void launch_quads(const SlotTable& t, int B, int parts, hipStream_t s, int jacobi);

@@ -419,7 +419,7 @@ __global__ __launch_bounds__(256) void quad_finish_kernel(SlotTable tab, int B, 
     s_y[b][e] = make_double2(yr * inv.x - yi * inv.y, yr * inv.y + yi * inv.x);
 }
 
-// k-space tables of the current layout.
+// k-space tables of the current layout, positions aside.
 void EwaldOp::build_quad_tables() {
     const int threads = 256;
     if (!slab) {
@@ -430,14 +430,20 @@ void EwaldOp::build_quad_tables() {
         MPM_HIP(hipGetLastError());
         return;
     }
-    const int nz = S.n[2], nh = nz / 2 + 1;
+    const int nh = S.n[2] / 2 + 1;
     const size_t n = (size_t)nh * kspace_cols();
     d_kqs64.resize(4 * n);
     d_kqs32.resize(4 * n);
     const int blocks = (int)std::min<size_t>((n + threads - 1) / threads, 65535);
     hipLaunchKernelGGL(quad_kslab_kernel, dim3(blocks), dim3(threads), 0, nullptr, d_kqs64.p, d_kqs32.p, kparams(), nh);
     MPM_HIP(hipGetLastError());
-    // cos and sin of 2 pi kz z_a / nz, [kz][16 cos, 16 sin]
+}
+
+// cos and sin of 2 pi kz z_a / nz, [kz][16 cos, 16 sin], of the slab's planes z_a: these move
+// with the particles, also where their number stays.
+void EwaldOp::build_quad_phases() {
+    if (zcs_planes == zlist && zcs_nz == S.n[2]) return;
+    const int nz = S.n[2], nh = nz / 2 + 1;
     std::vector<double> zc((size_t)32 * nh, 0.0);
     for (int k = 0; k < nh; ++k)
         for (int a = 0; a < Zs; ++a) {
@@ -445,7 +451,10 @@ void EwaldOp::build_quad_tables() {
             zc[32 * (size_t)k + a] = std::cos(2.0 * kPi * m / nz);
             zc[32 * (size_t)k + 16 + a] = 2 * m == nz || m == 0 ? 0.0 : std::sin(2.0 * kPi * m / nz);
         }
+    zcs_planes.clear();
     d_zcs64.upload(zc.data(), zc.size());
+    zcs_planes = zlist;
+    zcs_nz = nz;
 }
 
 template <typename R>

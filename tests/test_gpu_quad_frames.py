@@ -1,0 +1,71 @@
+"""One quadrupole operator over several frames (a trajectory's use): every set_positions and
+set_bloch against the oracle's operator at the same positions, FP64 to 1e-11 of the largest
+value, where the occupied z-planes change their places and not their number.
+"""
+import numpy as np
+import pytest
+
+from cumpm_amd import _capi as C
+from oracle import oracle as O
+from gpu_helpers import Op, rel
+
+pytestmark = pytest.mark.gpu
+
+L, GRID, N = [23.0, 22.0, 40.0], (30, 28, 60), 60
+
+
+def layers(rng, z_planes):
+    """Every other particle in the layer of each of two z grid planes."""
+    z = np.empty(N)
+    for k, p in enumerate(z_planes):
+        z[k::2] = (p + rng.uniform(-0.3, 0.3, z[k::2].size)) * L[2] / GRID[2]
+    return np.stack([rng.uniform(0, 1, N) * L[0], rng.uniform(0, 1, N) * L[1], z], 1)
+
+
+def check(op, pos, x, sc, kb=None):
+    ref = O.Operator(L, 1e-6, 0.5, grid=list(GRID), P=4)
+    if kb is not None:
+        ref.set_bloch(*kb)
+    ref.set_positions(pos)
+    ref.set_quads(None)
+    y = op.apply(x)
+    for b in range(len(x)):
+        assert rel(y[b], ref.apply(x[b], sc).reshape(-1)) < 1e-11, b
+
+
+@pytest.mark.parametrize("first,second", [
+    ((5, 15), (5, 21)),   # two separated layers, another gap
+    ((5, 10), (5, 15)),   # one run of ten planes, then two of five
+    ((5, 15), (5, 10)),   # and back
+    ((5, 15), (0, 10)),   # the same gap across the end of the box: another plane order
+    ((5, 10), (57, 62)),  # one run across the end of the box
+])
+def test_frames_with_equally_many_planes(first, second):
+    print(f"quad frames {first} {second}", flush=True)
+    rng = np.random.default_rng(61)
+    op = Op(L, 1e-6, 0.5, grid=GRID, support=4, quads=True)
+    sc = np.full(N, -0.3 + 0.05j)
+    x = rng.standard_normal((2, 8 * N)) + 1j * rng.standard_normal((2, 8 * N))
+    C.profile_reset()
+    C.profile_enable(True)
+    for pos in (layers(rng, first), layers(rng, second)):
+        op.set_positions(pos)
+        op.set_self_coef(sc)
+        check(op, pos, x, sc)
+    C.profile_enable(False)
+    assert "quad_zcouple_kernel<double, 10>" in C.profile_names(), C.profile_names()
+
+
+def test_frames_with_bloch_vectors():
+    print("quad frames with Bloch vectors", flush=True)
+    rng = np.random.default_rng(67)
+    op = Op(L, 1e-6, 0.5, grid=GRID, support=4, quads=True)
+    sc = np.full(N, 0.2 - 0.1j)
+    x = rng.standard_normal((1, 8 * N)) + 1j * rng.standard_normal((1, 8 * N))
+    for planes, kb in (((5, 15), (0.0, 0.0)), ((5, 15), (0.07, -0.04)), ((5, 19), (0.07, -0.04)),
+                       ((5, 10), (0.0, 0.03))):
+        pos = layers(rng, planes)
+        op.set_bloch(*kb)
+        op.set_positions(pos)
+        op.set_self_coef(sc)
+        check(op, pos, x, sc, kb)
