@@ -5011,7 +5011,7 @@ RegionGeom EwaldOp::region_geom(bool on_slab) const {
 
 RegionSet EwaldOp::region_set(bool on_slab) const {
     return RegionSet{on_slab,        on_slab ? zs_bucket(Zs) : reg_pblk, reg_nrx * reg_npb * reg_nry, reg_slots,
-                     d_reg_start.p, d_reg_items.p,                      d_reg_quads.p};
+                     d_reg_start.p, d_reg_items.p,                      qidx_h.empty() ? nullptr : d_reg_quads.p};
 }
 
 template <typename R, bool SLAB>

@@ -267,8 +267,9 @@ __global__ __launch_bounds__(256, sizeof(R) == 4 ? (NC == 3 ? 4 : 3) : 2) void s
     constexpr int QS = 256 / CPB, TV = KC / QS;
     constexpr int TW = (KC * L::NW + 255) / 256;  // weight-row entries of this thread
     const int scol = tid % CPB, sqc = col_base + scol;
-    // columns past the batch read column 0 and stage zeros
-    const bool scok = sqc < ncols;
+    // columns past the batch, and the gradient columns when no particle has a quadrupole
+    // (reg_quads null: the vectors end at n3), read column 0 and stage zeros
+    const bool scok = sqc < ncols && (NC == 3 || reg_quads || (sqc >> 1) % NC < 3);
     const int sq = scok ? sqc : 0;
     // vectors of unknowns: 3 components per particle, with quadrupoles (NC = 8) followed
     // after n3 = 3 N values by 5 per quadrupole; a candidate's entry e of this thread's column
@@ -826,7 +827,7 @@ __global__ __launch_bounds__(256) void contract_full_mfma_kernel(int B, RegionGe
 
 // The regions of the current frame: layout, planes compiled for (slab: bucket of Zs; full
 // grid: planes per region), number of regions and of (region, candidate) slots, the candidates
-// (CSR) and their quadrupoles (-1: none; read with NC = 8 only).
+// (CSR) and their quadrupoles (-1: none; read with NC = 8 only, null when no particle has one).
 struct RegionSet {
     bool slab;
     int zsb, nreg, slots;
