@@ -4369,6 +4369,29 @@ static int zs_bucket(int Zs) {
     return 0;
 }
 
+// Transforms of the full grid [comps][nx][ny][nz]: z, y, x lines in place (one component for the
+// polydisperse grid); null where a length does not fit the built-in transform.
+static std::unique_ptr<LineFft> full_grid_fft(const int n[3], long long comps) {
+    const long long nx = n[0], ny = n[1], nz = n[2];
+    auto lf = std::make_unique<LineFft>();
+    lf->rhs_elems = comps * nx * ny * nz;
+    lf->comps = (int)comps;
+    const LineGeom g3[3] = {{comps * nx * ny, 1, 0, nz, 1},
+                            {comps * nx * nz, nz, 1, ny * nz, nz},
+                            {comps * ny * nz, ny * nz, 1, nx * ny * nz, ny * nz}};
+    const int n3[3] = {n[2], n[1], n[0]};
+    for (int d = 0; d < 3; ++d) {
+        if (n3[d] <= 1) continue;
+        if (!LineFft::fits(n3[d])) return nullptr;
+        lf->axes.push_back(std::make_unique<LineAxis>(n3[d]));
+        const int a = (int)lf->axes.size() - 1;
+        if (d == 0) lf->full_z = a;
+        lf->fwd.push_back(LinePass{a, g3[d], g3[d], 0, 0});
+        lf->inv.push_back(LinePass{a, g3[d], g3[d], 0, 0});
+    }
+    return lf;
+}
+
 void EwaldOp::set_positions(const double* xyz, int64_t n) {
     MPM_REQUIRE(n > 0, MPM_ERR_INVALID_ARGUMENT, "no particles");
     MPM_REQUIRE(n < (1LL << 31) / 1024, MPM_ERR_INVALID_ARGUMENT, "too many particles");
@@ -4455,9 +4478,9 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
     }
     const int zsb = zs_bucket((int)zl.size());
     // (quadrupoles: up to the planes their coupling kernel holds in registers, with two real
-    // in-plane axes)
+    // in-plane axes and every length within the built-in transform)
     const bool may_slab = quads ? !quads_full && zsb <= kQuadSlabPlanes && S.n[0] > 1 && S.n[1] > 1 &&
-                                      LineFft::fits(S.n[0]) && LineFft::fits(S.n[1])
+                                      LineFft::fits(S.n[0]) && LineFft::fits(S.n[1]) && LineFft::fits(nz)
                                 : force_full == 0;
     const bool want_slab = may_slab && zsb > 0 && (int)zl.size() * 2 <= nz &&
                            zfused_lds(zsb, nz, sizeof(double)) <= 64 * 1024;
@@ -4828,7 +4851,7 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
     nxp = kt_ok ? (S.n[0] + 15) / 16 * 16 : S.n[0];
     const int key = slab ? Zs : -1;
     if (!lfft || fft_key != key) {
-        const int nx = S.n[0], ny = S.n[1], nzz = S.n[2];
+        const int nx = S.n[0], ny = S.n[1];
         const long long nxy = (long long)nx * ny;
         auto lf = std::make_unique<LineFft>();
         bool ok = true;
@@ -4868,24 +4891,10 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
                 pass(lf->fwd, a, g, g, 0, 0);
                 pass(lf->inv, a, g, g, 0, 0);
             }
-        } else {  // [comps][nx][ny][nz]: z, y, x lines in place (one component for the polydisperse grid)
-            lf->rhs_elems = nc * nxy * nzz;
-            lf->comps = (int)nc;
-            const LineGeom gz{nc * nxy, 1, 0, nzz, 1};
-            const LineGeom gy{nc * nx * nzz, nzz, 1, (long long)ny * nzz, nzz};
-            const LineGeom gx{nc * ny * nzz, (long long)ny * nzz, 1, nxy * nzz, (long long)ny * nzz};
-            const int n3[3] = {nzz, ny, nx};
-            const LineGeom g3[3] = {gz, gy, gx};
-            for (int d = 0; d < 3; ++d) {
-                if (n3[d] <= 1) continue;
-                const int a = axis(n3[d]);
-                if (d == 0) lf->full_z = a;
-                pass(lf->fwd, a, g3[d], g3[d], 0, 0);
-                pass(lf->inv, a, g3[d], g3[d], 0, 0);
-            }
         }
-        lfft = ok ? std::move(lf) : nullptr;
+        lfft = !slab ? full_grid_fft(S.n, nc) : (ok ? std::move(lf) : nullptr);
     }
+    if (quads && slab && !lfft_stage) lfft_stage = full_grid_fft(S.n, 8);
     // the slab's k-space data sits transposed ([ky][kx] columns) in its own
     // buffer when the built-in transform runs the slab with two real axes
     kt = slab && lfft && fft_backend == 0 && S.n[0] > 1 && S.n[1] > 1;
@@ -4941,6 +4950,14 @@ void EwaldOp::line_fft(void* grid, void* kgrid, int B, bool forward, hipStream_t
 }
 template void EwaldOp::line_fft<float>(void*, void*, int, bool, hipStream_t);
 template void EwaldOp::line_fft<double>(void*, void*, int, bool, hipStream_t);
+
+template <typename R>
+void EwaldOp::stage_fft(void* grid, bool forward, hipStream_t s) {
+    using CT = typename C2<R>::T;
+    lfft_stage->exec<R>(reinterpret_cast<CT*>(grid), reinterpret_cast<CT*>(grid), 1, forward, s);
+}
+template void EwaldOp::stage_fft<float>(void*, bool, hipStream_t);
+template void EwaldOp::stage_fft<double>(void*, bool, hipStream_t);
 
 size_t EwaldOp::grid_elems_per_rhs() const {
     if (poly) return V;
@@ -5470,6 +5487,7 @@ void EwaldOp::apply(const SlotTable& t, int B, bool fp32, int parts, hipStream_t
         return;
     }
     if (quads) {
+        cur_quad_slab = slab;
         if (fp32) launch_quads<float>(t, B, parts, s, jac);
         else launch_quads<double>(t, B, parts, s, jac);
         return;
@@ -5523,6 +5541,7 @@ void EwaldOp::configure(int layout, int backend, const int* grid) {
     fft_backend = backend;
     lfft.reset();
     fft.reset();
+    lfft_stage.reset();
     fft_key = -2;
     kspace_ready = false;
     kspace_key = -1;
@@ -5554,7 +5573,6 @@ void EwaldOp::stage(int which, const double2* x, void* grid, double2* y, bool fp
     MPM_REQUIRE(!recip || grid, MPM_ERR_INVALID_ARGUMENT, "stage needs a grid buffer");
     MPM_REQUIRE(which == 2 || (x != nullptr && (which == 1 || y != nullptr)), MPM_ERR_INVALID_ARGUMENT,
                 "stage needs the dipoles (and, to add into, the field)");
-    if (recip) quads_on_full_grid();
     if (recip) ensure_kspace_table();
     // spread writes the grid, scale transforms it in place; contract and real space add into y
     SlotTable t;
@@ -5570,7 +5588,10 @@ void EwaldOp::stage(int which, const double2* x, void* grid, double2* y, bool fp
     }
     cur_grid = grid;
     cur_kgrid = nullptr;
-    if (kt && which == 2) {
+    cur_quad_slab = false;
+    // with quadrupoles the stages' grids are full grids, also where the applies take the slab
+    const bool full_stage = recip && quads && slab;
+    if (kt && which == 2 && !full_stage) {
         const size_t ke = kgrid_elems_per_rhs();
         if (fp32) {
             d_kgrid32.reserve(ke);
@@ -5589,6 +5610,9 @@ void EwaldOp::stage(int which, const double2* x, void* grid, double2* y, bool fp
     if (direct) {
         if (fp32) launch_direct<float>(t, 1, parts, s, 0);
         else launch_direct<double>(t, 1, parts, s, 0);
+    } else if (full_stage) {
+        if (fp32) stage_quads_full<float>(which, x, grid, t.y[0], s);
+        else stage_quads_full<double>(which, x, grid, t.y[0], s);
     } else if (quads) {
         if (fp32) launch_quads<float>(t, 1, parts, s, 0);
         else launch_quads<double>(t, 1, parts, s, 0);
@@ -5656,10 +5680,7 @@ void* EwaldOp::device_pointer(const std::string& name, size_t& bytes) {
         if (slab && zcontig) return give(d_toe64.p, d_toe64.n * sizeof(double2));
         return give(d_k64.p, d_k64.n * sizeof(double));
     }
-    if (name == "fe_grid") {
-        quads_on_full_grid();
-        return give(cur_grid, 0);
-    }
+    if (name == "fe_grid") return give(cur_quad_slab ? nullptr : cur_grid, 0);
     if (name == "fes_grid") return give(d_kgrid64.p ? (void*)d_kgrid64.p : (void*)d_kgrid32.p,
                                         d_kgrid64.p ? d_kgrid64.n * sizeof(double2) : d_kgrid32.n * sizeof(float2));
     throw Error(MPM_ERR_INVALID_ARGUMENT, "unknown device buffer name '" + name + "'");

@@ -374,6 +374,7 @@ class EwaldOp {
     // or the caller's workspace)
     void* cur_grid = nullptr;
     void* cur_kgrid = nullptr;
+    bool cur_quad_slab = false;  // the last apply's grid was a quadrupole slab
     int phases = 7;  // parts of a launch: 1 spread, 2 transforms and Green's tensor, 4 contraction
     DevBuf<double2> d_grid64;
     DevBuf<float2> d_grid32;
@@ -394,7 +395,7 @@ class EwaldOp {
     mutable std::vector<double> h_pair_q;     // [M][7] quadrupole table values per pair
     std::vector<int> qmap_h;          // [N] quadrupole of each particle (-1: none)
     double quad_self_grad = 0;        // gradient self term
-    bool quads_full = false;          // applies stay on the full grid (requested, or used stage by stage)
+    bool quads_full = false;          // applies stay on the full grid (the descriptor's layout = 1)
     // full grid: [V][16] khat, sc, scQ, scGP, scGQ, Qfactor[5], Qdot[4]
     DevBuf<double> d_kq64;
     DevBuf<float> d_kq32;
@@ -411,7 +412,11 @@ class EwaldOp {
     void ensure_quad_scale_coef();
     void build_quad_tables();
     void build_quad_phases();
-    void quads_on_full_grid();
+    template <typename R>
+    void stage_quads_full(int which, const double2* x, void* grid, double2* y, hipStream_t s);
+    std::unique_ptr<LineFft> lfft_stage;  // full-grid transforms of the slab operator's stages
+    template <typename R>
+    void stage_fft(void* grid, bool forward, hipStream_t s);
     template <typename R>
     void launch_quads(const SlotTable& t, int B, int parts, hipStream_t s, int jacobi);
     template <typename R>

@@ -38,38 +38,42 @@ __device__ inline void quad_scalars(const KParams& q, double kx, double ky, doub
     o[3] = 1.0 / k;
 }
 
-// Full grid, per voxel: khat (3), sc, scQ, scGP, scGQ, Qfactor (5), Qdot (first 4 of 5).
+// Full grid, coefficients of a voxel: khat (3), sc, scQ, scGP, scGQ, Qfactor (5), Qdot (first 4
+// of 5; the last, 2 h1 h2, is formed from khat).
+__device__ inline void quad_voxel(const KParams& q, size_t v, double o[16]) {
+    const int ix = (int)(v / ((size_t)q.ny * q.nz)), iy = (int)((v / q.nz) % q.ny), iz = (int)(v % q.nz);
+    const double Gx = freq(ix, q.nx) * 2.0 * kPi / q.Lx, Gy = freq(iy, q.ny) * 2.0 * kPi / q.Ly,
+                 Gz = freq(iz, q.nz) * 2.0 * kPi / q.Lz;
+    const double kx = Gx - q.kbx, ky = Gy - q.kby, kz = Gz;
+    double f[4];
+    for (int c = 0; c < 16; ++c) o[c] = 0.0;
+    quad_scalars(q, kx, ky, kz, Gx * Gx * q.etax + Gy * Gy * q.etay + Gz * Gz * q.etaz, f);
+    if (f[3] == 0.0) return;
+    const double k = sqrt(kx * kx + ky * ky + kz * kz);
+    const double h0 = kx / k, h1 = ky / k, h2 = kz / k;
+    o[0] = h0;
+    o[1] = h1;
+    o[2] = h2;
+    o[3] = f[0];
+    o[4] = f[1];
+    o[5] = -2.0 * f[1];
+    o[6] = f[2];
+    o[7] = h0 * h0 - 1.0 / 3.0;
+    o[8] = h0 * h1;
+    o[9] = h0 * h2;
+    o[10] = h1 * h1 - 1.0 / 3.0;
+    o[11] = h1 * h2;
+    o[12] = h0 * h0 - h2 * h2;
+    o[13] = 2.0 * h0 * h1;
+    o[14] = 2.0 * h0 * h2;
+    o[15] = h1 * h1 - h2 * h2;
+}
+
 __global__ void quad_kspace_kernel(double* __restrict__ k64, float* __restrict__ k32, KParams q) {
     const size_t V = (size_t)q.nx * q.ny * q.nz;
     for (size_t v = blockIdx.x * (size_t)blockDim.x + threadIdx.x; v < V; v += (size_t)gridDim.x * blockDim.x) {
-        const int ix = (int)(v / ((size_t)q.ny * q.nz)), iy = (int)((v / q.nz) % q.ny), iz = (int)(v % q.nz);
-        const double Gx = freq(ix, q.nx) * 2.0 * kPi / q.Lx, Gy = freq(iy, q.ny) * 2.0 * kPi / q.Ly,
-                     Gz = freq(iz, q.nz) * 2.0 * kPi / q.Lz;
-        const double kx = Gx - q.kbx, ky = Gy - q.kby, kz = Gz;
-        double o[16], f[4];
-        for (int c = 0; c < 16; ++c) o[c] = 0.0;
-        quad_scalars(q, kx, ky, kz, Gx * Gx * q.etax + Gy * Gy * q.etay + Gz * Gz * q.etaz, f);
-        if (f[3] != 0.0) {
-            const double k = sqrt(kx * kx + ky * ky + kz * kz);
-            const double h0 = kx / k, h1 = ky / k, h2 = kz / k;
-            o[0] = h0;
-            o[1] = h1;
-            o[2] = h2;
-            o[3] = f[0];
-            o[4] = f[1];
-            o[5] = -2.0 * f[1];
-            o[6] = f[2];
-            o[7] = h0 * h0 - 1.0 / 3.0;
-            o[8] = h0 * h1;
-            o[9] = h0 * h2;
-            o[10] = h1 * h1 - 1.0 / 3.0;
-            o[11] = h1 * h2;
-            o[12] = h0 * h0 - h2 * h2;
-            o[13] = 2.0 * h0 * h1;
-            o[14] = 2.0 * h0 * h2;
-            o[15] = h1 * h1 - h2 * h2;
-        }
-        // Qdot[4] = 2 h1 h2 does not fit the 16 slots: the scale kernel forms it from khat
+        double o[16];
+        quad_voxel(q, v, o);
         for (int c = 0; c < 16; ++c) {
             k64[16 * v + c] = o[c];
             k32[16 * v + c] = (float)o[c];
@@ -77,53 +81,167 @@ __global__ void quad_kspace_kernel(double* __restrict__ k64, float* __restrict__
     }
 }
 
-// Full grid: joint k-space coupling of field and gradient grids (scale_kernel_joint,
-// :1435-1487): Edk = E.khat, GQ = G.Qdot; E <- (sc Edk + i scQ GQ) khat,
-// G <- (i scGP Edk + scGQ GQ) Qfactor.  A thread per voxel and right-hand sides
-// blockIdx.y, blockIdx.y + gridDim.y, ...: the voxel's 16 coefficients are read once for
-// all of them.
+// Full grid: joint k-space coupling of field and gradient grids at a voxel with coefficients k
+// (scale_kernel_joint, :1435-1487): Edk = E.khat, GQ = G.Qdot; E <- (sc Edk + i scQ GQ) khat,
+// G <- (i scGP Edk + scGQ GQ) Qfactor.
+template <typename R>
+__device__ inline void quad_couple(const R (&k)[16], typename C2<R>::T* __restrict__ g, size_t V) {
+    using CT = typename C2<R>::T;
+    const R h0 = k[0], h1 = k[1], h2 = k[2];
+    const R qd[5] = {k[12], k[13], k[14], k[15], R(2) * h1 * h2};
+    CT f[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) f[c] = g[c * V];
+    const R er = f[0].x * h0 + f[1].x * h1 + f[2].x * h2, ei = f[0].y * h0 + f[1].y * h1 + f[2].y * h2;
+    R gr = R(0), gi = R(0);
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+        gr += f[3 + c].x * qd[c];
+        gi += f[3 + c].y * qd[c];
+    }
+    // i a (x + i y) = -a y + i a x
+    const R sr = k[3] * er - k[4] * gi, si = k[3] * ei + k[4] * gr;
+    const R tr = -k[5] * ei + k[6] * gr, ti = k[5] * er + k[6] * gi;
+    const R hh[3] = {h0, h1, h2};
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        CT o;
+        o.x = sr * hh[c];
+        o.y = si * hh[c];
+        g[c * V] = o;
+    }
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+        CT o;
+        o.x = tr * k[7 + c];
+        o.y = ti * k[7 + c];
+        g[(3 + c) * V] = o;
+    }
+}
+
+// A thread per voxel and right-hand sides blockIdx.y, blockIdx.y + gridDim.y, ...: the voxel's
+// 16 coefficients are read once for all of them.
 template <typename R>
 __global__ __launch_bounds__(256) void quad_scale_kernel(typename C2<R>::T* __restrict__ grid,
                                                          const R* __restrict__ kq, size_t V, int B) {
-    using CT = typename C2<R>::T;
     const size_t v = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
     if (v >= V) return;
     R k[16];
 #pragma unroll
     for (int c = 0; c < 16; ++c) k[c] = kq[16 * v + c];
-    const R h0 = k[0], h1 = k[1], h2 = k[2];
-    const R qd[5] = {k[12], k[13], k[14], k[15], R(2) * h1 * h2};
-    for (int b = blockIdx.y; b < B; b += gridDim.y) {
-        CT* g = grid + (size_t)b * 8 * V + v;
-        CT f[8];
+    for (int b = blockIdx.y; b < B; b += gridDim.y) quad_couple<R>(k, grid + (size_t)b * 8 * V + v, V);
+}
+
+// ---- single stages of an operator whose applies run on the slab ----
+//
+// The caller's grid is a full grid [8][nx][ny][nz] of one right-hand side.  These kernels work
+// from the slab's own region lists and weights and compute the coefficients they need, so that
+// a stage allocates nothing and changes nothing of the operator (applies in flight go on).  A
+// debugging path: one thread per voxel, one wave per particle, no matrix cores.
+
+// Spread: a thread per voxel sums the candidates of its region in ascending particle order.
+template <typename R>
+__global__ __launch_bounds__(256) void quad_stage_spread_kernel(
+    const double2* __restrict__ x, size_t n3, int nx, int ny, int nz, int RX, int nry, int zsb4,
+    const double* __restrict__ regw, const int* __restrict__ reg_start, const int* __restrict__ reg_items,
+    const int* __restrict__ reg_quads, const int* __restrict__ zmap, typename C2<R>::T* __restrict__ out) {
+    using CT = typename C2<R>::T;
+    const size_t V = (size_t)nx * ny * nz;
+    const size_t v = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+    if (v >= V) return;
+    const int ix = (int)(v / ((size_t)ny * nz)), iy = (int)((v / nz) % ny), iz = (int)(v % nz);
+    const int NW = 4 + zsb4 + kMfmaRY, p = zmap[iz];
+    R ar[8], ai[8];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) f[c] = g[c * V];
-        const R er = f[0].x * h0 + f[1].x * h1 + f[2].x * h2, ei = f[0].y * h0 + f[1].y * h1 + f[2].y * h2;
-        R gr = R(0), gi = R(0);
+    for (int c = 0; c < 8; ++c) ar[c] = ai[c] = R(0);
+    if (p >= 0) {
+        const int reg = (ix / RX) * nry + iy / kMfmaRY;
+        const int k1 = reg_start[reg + 1];
+        for (int k = reg_start[reg]; k < k1; ++k) {
+            const double* w = regw + (size_t)k * NW;
+            const R ww = (R)(w[ix % RX] * w[4 + zsb4 + iy % kMfmaRY] * w[4 + p]);
+            if (ww == R(0)) continue;
+            const double2* xp = x + 3 * (size_t)reg_items[k];
 #pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            gr += f[3 + c].x * qd[c];
-            gi += f[3 + c].y * qd[c];
-        }
-        // i a (x + i y) = -a y + i a x
-        const R sr = k[3] * er - k[4] * gi, si = k[3] * ei + k[4] * gr;
-        const R tr = -k[5] * ei + k[6] * gr, ti = k[5] * er + k[6] * gi;
-        const R hh[3] = {h0, h1, h2};
+            for (int c = 0; c < 3; ++c) {
+                ar[c] += ww * (R)xp[c].x;
+                ai[c] += ww * (R)xp[c].y;
+            }
+            const int q = reg_quads ? reg_quads[k] : -1;
+            if (q < 0) continue;
+            const double2* xq = x + n3 + 5 * (size_t)q;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            CT o;
-            o.x = sr * hh[c];
-            o.y = si * hh[c];
-            g[c * V] = o;
-        }
-#pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            CT o;
-            o.x = tr * k[7 + c];
-            o.y = ti * k[7 + c];
-            g[(3 + c) * V] = o;
+            for (int c = 0; c < 5; ++c) {
+                ar[3 + c] += ww * (R)xq[c].x;
+                ai[3 + c] += ww * (R)xq[c].y;
+            }
         }
     }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        CT o;
+        o.x = ar[c];
+        o.y = ai[c];
+        out[c * V + v] = o;
+    }
+}
+
+// Coupling with coefficients computed in place of the table's, rounded as the table's.
+template <typename R>
+__global__ __launch_bounds__(256) void quad_stage_scale_kernel(typename C2<R>::T* __restrict__ grid, KParams q) {
+    const size_t V = (size_t)q.nx * q.ny * q.nz;
+    const size_t v = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+    if (v >= V) return;
+    double o[16];
+    quad_voxel(q, v, o);
+    R k[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) k[c] = (R)o[c];
+    quad_couple<R>(k, grid + v, V);
+}
+
+// Contraction: a wave per particle over its W^3 stencil voxels, summed in FP64.
+template <typename R>
+__global__ __launch_bounds__(256) void quad_stage_contract_kernel(
+    const typename C2<R>::T* __restrict__ grid, int N, int nx, int ny, int nz, int W, const int* __restrict__ base,
+    const double* __restrict__ w64, const int* __restrict__ qmap, double h3, double2* __restrict__ y) {
+    const int lane = threadIdx.x & 63;
+    const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (i >= N) return;  // whole wave
+    const size_t V = (size_t)nx * ny * nz;
+    const int half = W / 2, qi = qmap[i];
+    const int b0 = base[i] - half, b1 = base[N + i] - half, b2 = base[2 * (size_t)N + i] - half;
+    const double* w = w64 + (size_t)i * 3 * W;
+    double acc[8][2];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) acc[c][0] = acc[c][1] = 0.0;
+    for (int o = lane; o < W * W * W; o += 64) {
+        const int oz = o % W, oy = (o / W) % W, ox = o / (W * W);
+        // base lies in the box; the stencil may be wider than an axis
+        int vx = (b0 + ox) % nx, vy = (b1 + oy) % ny, vz = (b2 + oz) % nz;
+        vx += vx < 0 ? nx : 0;
+        vy += vy < 0 ? ny : 0;
+        vz += vz < 0 ? nz : 0;
+        const double ww = w[ox] * w[W + oy] * w[2 * W + oz] * h3;
+        const typename C2<R>::T* g = grid + ((size_t)vx * ny + vy) * nz + vz;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            acc[c][0] += ww * (double)g[c * V].x;
+            acc[c][1] += ww * (double)g[c * V].y;
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        acc[c][0] = wave_sum(acc[c][0]);
+        acc[c][1] = wave_sum(acc[c][1]);
+    }
+    if (lane) return;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) y[3 * (size_t)i + c] = make_double2(acc[c][0], acc[c][1]);
+    if (qi < 0) return;
+#pragma unroll
+    for (int c = 0; c < 5; ++c)
+        y[3 * (size_t)N + 5 * (size_t)qi + c] = make_double2(acc[3 + c][0], acc[3 + c][1]);
 }
 
 // Slab: coupling scalars (sc, scQ, scGQ, 1 / |k|) of every column and wave number kz = 0 ..
@@ -590,16 +708,41 @@ void EwaldOp::ensure_quad_scale_coef() {
     quad_coef_valid = true;
 }
 
-// The dev pipeline's grids are full grids: an operator used stage by stage (or asked for its
-// grid) leaves the slab for good.
-void EwaldOp::quads_on_full_grid() {
-    if (!quads || !slab || N == 0) return;
-    quads_full = true;
-    cur_grid = nullptr;
-    const std::vector<double> xyz = last_xyz;
-    const int64_t n = N;
-    last_xyz.clear();
-    set_positions(xyz.data(), n);
+// Stage `which` (1 spread, 2 transforms and coupling, 3 contraction into y) of one right-hand
+// side on a full grid, for an operator whose applies run on the slab.
+template <typename R>
+void EwaldOp::stage_quads_full(int which, const double2* x, void* grid, double2* y, hipStream_t s) {
+    using CT = typename C2<R>::T;
+    CT* g = reinterpret_cast<CT*>(grid);
+    const dim3 gv((unsigned)((V + 255) / 256)), blk(256);
+    if (which == 1) {
+        ProfScope ps("spread", s, 1);
+        ps.kernel("quad_stage_spread_kernel", {type_name<R>()});
+        hipLaunchKernelGGL((quad_stage_spread_kernel<R>), gv, blk, 0, s, x, 3 * (size_t)N, S.n[0], S.n[1], S.n[2],
+                           reg_rx, reg_nry, (region_set(true).zsb + 3) & ~3, d_regw64.p, d_reg_start.p, d_reg_items.p,
+                           qidx_h.empty() ? nullptr : d_reg_quads.p, d_zmap.p, g);
+    } else if (which == 2) {
+        {
+            ProfScope ps("fft", s, 1);
+            stage_fft<R>(grid, true, s);
+        }
+        {
+            ProfScope ps("scale", s, 1);
+            ps.kernel("quad_stage_scale_kernel", {type_name<R>()});
+            hipLaunchKernelGGL((quad_stage_scale_kernel<R>), gv, blk, 0, s, g, kparams());
+            MPM_HIP(hipGetLastError());
+        }
+        ProfScope ps("fft", s, 1);
+        stage_fft<R>(grid, false, s);
+    } else {
+        ProfScope ps("contract", s, 1);
+        ps.kernel("quad_stage_contract_kernel", {type_name<R>()});
+        hipLaunchKernelGGL((quad_stage_contract_kernel<R>), dim3((unsigned)((N + 3) / 4)), blk, 0, s, g, (int)N, S.n[0],
+                           S.n[1], S.n[2], S.width, d_base.p, d_w64.p, d_qmap.p, S.h[0] * S.h[1] * S.h[2], y);
+    }
+    MPM_HIP(hipGetLastError());
 }
+template void EwaldOp::stage_quads_full<float>(int, const double2*, void*, double2*, hipStream_t);
+template void EwaldOp::stage_quads_full<double>(int, const double2*, void*, double2*, hipStream_t);
 
 }  // namespace mpm

@@ -602,6 +602,8 @@ class MonodisperseEwaldElectricField(_EwaldField):
         if grid is not None:
             d.grid[:] = [int(g) for g in grid]
         d.support = int(support)
+        # this class shows its grid (dev_fe_grid), with quadrupoles the full one
+        d.layout = 1 if solve_quadrupoles else 0
         self._box = (float(box_x), float(box_y), float(box_z))
         self._errortol = float(errortol)
         self._xi = float(xi)

@@ -143,7 +143,8 @@ mpm_status mpm_op_set_positions(mpm_op* op, const double* xyz, int64_t n_particl
  * :1871-1999): quadrupoles on particles idx[nq] (every particle when nq < 0).  Call before
  * mpm_op_set_positions.  Vectors then hold 3N dipole components followed by 5 components
  * (xx, xy, xz, yy, yz of the traceless moment) per quadrupole, in idx order; the operator
- * returns field and field gradient in the same layout.  Full-grid layout and built-in FFT.
+ * returns field and field gradient in the same layout.  Built-in FFT.  Applies take the z-plane
+ * slab where layout = 0 allows it (at most 10 planes); the grids of mpm_op_stage are full grids.
  * The dipole-quadrupole real-space couplings take the signs of the reference's Python
  * formulation (tests/quadrupole_field.py:214-215); the CUDA kernel has both flipped. */
 mpm_status mpm_op_set_quads(mpm_op* op, const int* idx, int64_t nq);
@@ -190,10 +191,10 @@ mpm_status mpm_op_stage(mpm_op* op, int stage, const double* x, void* grid, doub
  * "neighbor_start" (int [N + 1] CSR), "neighbor_list" (int [M]), "perp_para" (complex-double
  * pairs (perp, para) [M]), "pair_coef" (double per-pair coefficients), "self_perp"
  * (polydisperse, double [N]), "scale_coef" (k-space table), "fe_grid" (the grid of the last
- * apply), "fes_grid" (the slab's transposed k-space buffer).  With quadrupoles the stencil
- * buffers and "scale_coef" are built when first asked for, and the first use of "fe_grid" or
- * of a reciprocal stage moves the operator's applies to the full grid (before the next
- * apply "fe_grid" is then NULL).  Unknown names fail with MPM_ERR_INVALID_ARGUMENT. */
+ * apply or stage), "fes_grid" (the slab's transposed k-space buffer).  With quadrupoles the
+ * stencil buffers and "scale_coef" are built when first asked for, and "fe_grid" is NULL after
+ * an apply on the slab, whose grid is not the stages' full grid (create the operator with
+ * layout = 1 for applies on the full grid).  Unknown names fail with MPM_ERR_INVALID_ARGUMENT. */
 mpm_status mpm_op_device_pointer(const mpm_op* op, const char* name, void** ptr, size_t* bytes);
 
 /* mpm_op_apply that allocates no device memory.  No counterpart in the reference: it is

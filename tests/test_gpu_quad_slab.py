@@ -129,4 +129,4 @@ def test_stages_of_a_slab_operator_work_on_the_full_grid():
     out = np.zeros_like(x)
     yb.download(out)
     assert rel(out, y) < 1e-11
-    assert rel(op.apply(x), y) < 1e-11  # applies stay on the full grid from here on
+    assert rel(op.apply(x), y) < 1e-11  # as before the stages
