@@ -4032,6 +4032,7 @@ void EwaldOp::set_bloch(double kx, double ky) {
     if (N > 0) {
         build_pair_coefs();
         ensure_kspace_table();
+        refresh_quad_addresses();
     }
 }
 
@@ -4926,6 +4927,7 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
     ensure_kspace_table();
     laps.lap("host_setup_kspace");
     last_xyz.assign(xyz, xyz + 3 * n);
+    refresh_quad_addresses();
 }
 
 void EwaldOp::set_self_coef(const double* coef, int rows) {

@@ -404,8 +404,11 @@ class EwaldOp {
     DevBuf<float> d_kqs32;
     std::vector<int> zcs_planes;      // the planes and z length that d_zcs64 was built for
     int zcs_nz = 0;
-    // the reference's stencils and table for callers that ask for their address
+    // the reference's stencils and table for callers that ask for their address, kept current
+    // once one has asked
     bool quad_stencils_valid = false, quad_coef_valid = false;
+    bool quad_stencils_wanted = false, quad_coef_wanted = false;
+    void refresh_quad_addresses();
     DevBuf<double> d_sw64;            // [N][W^3] Gaussian weights (spread constant included)
     DevBuf<float> d_sw32;
     void ensure_quad_stencils();

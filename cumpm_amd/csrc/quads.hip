@@ -656,8 +656,10 @@ template void EwaldOp::launch_quads<double>(const SlotTable&, int, int, hipStrea
 
 // The W^3 points of every particle, their wrapped voxels and Gaussian weights
 // C exp(-2 xi^2 sum gd^2/eta) (the dipole weights, :687-816) as the reference keeps them; the
-// kernels work from separable weights, so these exist for callers that ask for their address.
+// kernels work from separable weights, so these exist for callers that ask for their address:
+// built when first asked for, and from then on by every set_positions.
 void EwaldOp::ensure_quad_stencils() {
+    quad_stencils_wanted = true;
     if (quad_stencils_valid || N == 0 || last_xyz.empty()) return;
     const int W = S.width, half = S.half, Nn = (int)N;
     const int SS = W * W * W;
@@ -696,8 +698,10 @@ void EwaldOp::ensure_quad_stencils() {
     quad_stencils_valid = true;
 }
 
-// The full-grid coefficient table, for callers that ask for its address.
+// The full-grid coefficient table, for callers that ask for its address (kept current from
+// then on, as the stencils).
 void EwaldOp::ensure_quad_scale_coef() {
+    quad_coef_wanted = true;
     if (!slab || N == 0 || quad_coef_valid) return;
     d_kq64.resize(16 * V);
     d_kq32.resize(16 * V);
@@ -706,6 +710,11 @@ void EwaldOp::ensure_quad_scale_coef() {
     MPM_HIP(hipGetLastError());
     MPM_HIP(hipDeviceSynchronize());
     quad_coef_valid = true;
+}
+
+void EwaldOp::refresh_quad_addresses() {
+    if (quad_stencils_wanted) ensure_quad_stencils();
+    if (quad_coef_wanted) ensure_quad_scale_coef();
 }
 
 // Stage `which` (1 spread, 2 transforms and coupling, 3 contraction into y) of one right-hand

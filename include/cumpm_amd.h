@@ -192,7 +192,8 @@ mpm_status mpm_op_stage(mpm_op* op, int stage, const double* x, void* grid, doub
  * pairs (perp, para) [M]), "pair_coef" (double per-pair coefficients), "self_perp"
  * (polydisperse, double [N]), "scale_coef" (k-space table), "fe_grid" (the grid of the last
  * apply or stage), "fes_grid" (the slab's transposed k-space buffer).  With quadrupoles the
- * stencil buffers and "scale_coef" are built when first asked for, and "fe_grid" is NULL after
+ * stencil buffers and "scale_coef" are built when first asked for (and from then on with every
+ * set_positions / set_bloch), and "fe_grid" is NULL after
  * an apply on the slab, whose grid is not the stages' full grid (create the operator with
  * layout = 1 for applies on the full grid).  Unknown names fail with MPM_ERR_INVALID_ARGUMENT. */
 mpm_status mpm_op_device_pointer(const mpm_op* op, const char* name, void** ptr, size_t* bytes);

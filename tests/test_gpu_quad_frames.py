@@ -2,6 +2,8 @@
 set_bloch against the oracle's operator at the same positions, FP64 to 1e-11 of the largest
 value, where the occupied z-planes change their places and not their number.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -89,3 +91,42 @@ def test_no_quadrupoles_equals_the_dipole_operator(n, B, layout):
     assert rel(y[1][0], y[0][0]) < 1e-11
     # FP32 grids: 125 rounded products on either side of transforms of 50,400 points
     assert rel(y[1][1], y[0][0]) < 1e-6
+
+
+def read(op, name, dtype):
+    ptr, nb = ctypes.c_void_p(), ctypes.c_size_t()
+    C.check(C.load().mpm_op_device_pointer(op.h, name.encode(), ctypes.byref(ptr), ctypes.byref(nb)))
+    return ptr.value, fetch(ptr.value, nb.value // np.dtype(dtype).itemsize, dtype)
+
+
+def fetch(address, count, dtype):
+    out = np.zeros(count, dtype)
+    C.check(C.load().mpm_buffer_download(out.ctypes.data_as(ctypes.c_void_p), ctypes.c_void_p(address), out.nbytes))
+    return out
+
+
+ADDRESSES = (("spread_coef", np.float64), ("spread_coef_fp32", np.float32), ("spread_idxs", np.int32),
+             ("scale_coef", np.float64))
+
+
+def test_buffers_asked_for_stay_current():
+    print("quad buffers by address over frames", flush=True)
+    rng = np.random.default_rng(97)
+    op = Op(L, 1e-6, 0.5, grid=GRID, support=4, quads=True)
+    a, b = layers(rng, (5, 15)), layers(rng, (5, 19))
+
+    def fresh(pos, kb):
+        o = Op(L, 1e-6, 0.5, grid=GRID, support=4, quads=True)
+        o.set_bloch(*kb)
+        o.set_positions(pos)
+        return o
+
+    op.set_positions(a)
+    got = {name: read(op, name, dt) for name, dt in ADDRESSES}
+    for pos, kb in ((b, (0.0, 0.0)), (b, (0.07, -0.04)), (a, (0.07, -0.04))):
+        op.set_bloch(*kb)
+        op.set_positions(pos)
+        want = fresh(pos, kb)
+        for name, dt in ADDRESSES:  # the sizes stay, and so do the addresses
+            address, old = got[name]
+            np.testing.assert_array_equal(fetch(address, old.size, dt), read(want, name, dt)[1], err_msg=name)
