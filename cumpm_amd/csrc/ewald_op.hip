@@ -3965,7 +3965,7 @@ KParams EwaldOp::kparams() const {
 }
 
 void EwaldOp::build_kspace() {
-    // the full-grid coefficient table is built lazily (only the full-grid path reads it)
+    // the tables of the old grid or wave vector no longer hold; ensure_kspace_table builds new ones
     kspace_ready = false;
     quad_coef_valid = false;
 }
@@ -5530,7 +5530,7 @@ void EwaldOp::configure(int layout, int backend, const int* grid) {
     const bool regrid = grid && (grid[0] != S.n[0] || grid[1] != S.n[1] || grid[2] != S.n[2]);
     if (poly || quads)
         MPM_REQUIRE(layout == 1 && backend == 0, MPM_ERR_UNSUPPORTED,
-                    "the polydisperse and quadrupole operators run on the full grid with the built-in FFT");
+                    "the polydisperse and quadrupole operators keep their layout and the built-in FFT");
     MPM_REQUIRE(!(poly && regrid), MPM_ERR_UNSUPPORTED, "the polydisperse operator keeps its grid");
     if (regrid) {
         Sizing T;
@@ -5545,7 +5545,7 @@ void EwaldOp::configure(int layout, int backend, const int* grid) {
     fft.reset();
     lfft_stage.reset();
     fft_key = -2;
-    kspace_ready = false;
+    build_kspace();
     kspace_key = -1;
     if (N > 0) {
         const std::vector<double> xyz = last_xyz;

@@ -105,7 +105,7 @@ void autotune(EwaldOp& op, int B, bool fp32, int flags, hipStream_t s, mpm_tune_
                 if (grow) add(l, b, gs);
             }
     } else if (op.has_quads() && grow) {
-        add(1, 0, gs);  // quadrupoles: full grid and built-in FFT, on a grown grid
+        add(1, 0, gs);  // quadrupoles: the operator's own layout and built-in FFT, on a grown grid
     }
     const size_t nu = op.n_unknowns();
     DevBuf<double2> x, y;

@@ -130,3 +130,23 @@ def test_buffers_asked_for_stay_current():
         for name, dt in ADDRESSES:  # the sizes stay, and so do the addresses
             address, old = got[name]
             np.testing.assert_array_equal(fetch(address, old.size, dt), read(want, name, dt)[1], err_msg=name)
+
+
+def test_coefficients_asked_for_follow_the_tuned_grid():
+    print("quad coefficients by address over a grown grid", flush=True)
+    rng = np.random.default_rng(101)
+    grid = (93, 87, 60)  # 3 x 31 and 3 x 29: 96 and 90 transform faster
+    op = Op(L, 1e-6, 0.5, grid=grid, support=4, quads=True)
+    pos = layers(rng, (5, 15))
+    op.set_positions(pos)
+    op.set_self_coef(np.zeros(N))
+    assert read(op, "scale_coef", np.float64)[1].size == 16 * 93 * 87 * 60
+    tuned = C.TuneInfo()
+    C.check(C.load().mpm_op_autotune(op.h, 4, C.PREC_DOUBLE, C.TUNE_GRID | C.TUNE_FORCE, ctypes.byref(tuned)))
+    print("tuned grid", list(tuned.grid), flush=True)
+    want = Op(L, 1e-6, 0.5, grid=list(tuned.grid), support=4, quads=True)
+    want.set_positions(pos)
+    for name, dt in ADDRESSES:
+        a, b = read(op, name, dt)[1], read(want, name, dt)[1]
+        assert a.size == b.size, name
+        np.testing.assert_array_equal(a, b, err_msg=name)
