@@ -5248,10 +5248,14 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
                               (!SLAB && (S.width <= 5 || (B == 1 && 4ll * nreg < (long long)N)));
     if (regions && !per_particle && (parts & MPM_PART_RECIP)) {
         ProfScope ps("contract", s, B);
-        // dense regions of the full grid sum in FP64 over either grid, as the gather does past
-        // each lane's few terms; the others in the grid's precision
+        // FP64 sums over either grid where the gather, which sums in FP64 past each lane's few
+        // terms, ran instead of the regions: dense regions of the full grid, and grids and
+        // batches with fewer region waves than a quarter of the gather's; the others sum in the
+        // grid's precision
         part64 = !fp32;
-        if constexpr (std::is_same<R, float>::value && !SLAB) part64 = dense_regions(region_set(false));
+        if constexpr (std::is_same<R, float>::value && !SLAB)
+            part64 = dense_regions(region_set(false)) ||
+                     4ll * nreg * ((6 * B + 15) / 16) < (long long)N * ((B + 3) / 4);
         R* pbuf = reinterpret_cast<R*>(d_partial64.p);  // sized for FP64, shared by FP32
         if (part64)
             region_contract<double, 3, R>(ps, s, region_set(SLAB), rg, vec, B, d_regw64.p, grid, d_partial64.p);
