@@ -2862,10 +2862,14 @@ __global__ __launch_bounds__(256) void gather_kernel(
             for (int j = 0; j < G; ++j)
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
-                    acc[j][c][0] = (sizeof(R) == 8 ? 0.0 : acc[j][c][0]) + (double)racc[j][c][0];
-                    acc[j][c][1] = (sizeof(R) == 8 ? 0.0 : acc[j][c][1]) + (double)racc[j][c][1];
-                    acc[j][c][0] *= h3;
-                    acc[j][c][1] *= h3;
+                    // (FP64: acc holds nothing yet, and 0.0 + x is an addition to the compiler)
+                    if constexpr (sizeof(R) == 8) {
+                        acc[j][c][0] = racc[j][c][0] * h3;
+                        acc[j][c][1] = racc[j][c][1] * h3;
+                    } else {
+                        acc[j][c][0] = (acc[j][c][0] + (double)racc[j][c][0]) * h3;
+                        acc[j][c][1] = (acc[j][c][1] + (double)racc[j][c][1]) * h3;
+                    }
                 }
         }
         if (parts & MPM_PART_REAL) {
