@@ -569,14 +569,14 @@ ProfScope::ProfScope(const char* n, hipStream_t s, int64_t u) : name(n), units(u
     MPM_HIP(hipEventCreate(&e1));
     MPM_HIP(hipEventRecord(e0, stream));
 }
-void ProfScope::kernel(const char* base, std::initializer_list<std::string> targs) {
+void ProfScope::kernel(const char* base, std::initializer_list<Arg> targs) {
     if (!e0) return;
     kname = base;
     kname += '<';
     bool first = true;
-    for (const std::string& a : targs) {
+    for (const Arg& a : targs) {
         if (!first) kname += ", ";
-        kname += a;
+        kname += a.text ? std::string(a.text) : std::to_string(a.number);
         first = false;
     }
     kname += '>';
@@ -1858,7 +1858,7 @@ struct LineFft {
                 const size_t lds = ((size_t)TL * ((n + ax.plan.radix[1]) | 1) + n) * sizeof(CT);  // padded rows
                 const int nsets = (int)((gi.nlines + TL - 1) / TL);
                 const dim3 gd((unsigned)nsets);
-                pscope.kernel("line_fft2_kernel", {type_name<R>(), tbool(!forward), std::to_string(ax.cls)});
+                pscope.kernel("line_fft2_kernel", {type_name<R>(), tbool(!forward), ax.cls});
 #define MPM_L2(INV)                                                                       \
     if (ax.cls == 0) launch2<R, INV, 0>(gd, lds, s, in, out, gi, go, ax.plan, tw, TL);    \
     else if (ax.cls == 1) launch2<R, INV, 1>(gd, lds, s, in, out, gi, go, ax.plan, tw, TL); \
@@ -1880,7 +1880,7 @@ struct LineFft {
                 const size_t lds = (size_t)2 * TL * (n | 1) * sizeof(CT);
                 const int nsets = (int)((gi.nlines + TL - 1) / TL);
                 const dim3 gd((unsigned)std::min(nsets, 2048));
-                pscope.kernel("line_dft_kernel", {type_name<R>(), tbool(!forward), std::to_string(ax.dft)});
+                pscope.kernel("line_dft_kernel", {type_name<R>(), tbool(!forward), ax.dft});
 #define MPM_DFT(MTV)                                                                                               \
     case MTV:                                                                                                      \
         if (forward)                                                                                               \
@@ -1908,7 +1908,7 @@ struct LineFft {
             const size_t lds = ((size_t)2 * TL * n + 2 * n) * sizeof(CT);
             const long long blocks = (gi.nlines + TL - 1) / TL;
             const dim3 gd((unsigned)blocks);
-            pscope.kernel("line_fft_kernel", {type_name<R>(), tbool(!forward), std::to_string(ax.cls)});
+            pscope.kernel("line_fft_kernel", {type_name<R>(), tbool(!forward), ax.cls});
             if (forward) {
                 if (ax.cls == 0) launch<R, false, 0>(gd, lds, s, in, out, gi, go, ax.plan, tw, TL);
                 else if (ax.cls == 1) launch<R, false, 1>(gd, lds, s, in, out, gi, go, ax.plan, tw, TL);
@@ -4997,7 +4997,7 @@ static void zline_launch(ProfScope& ps, hipStream_t s, const LineAxis& ax, typen
     const CT* tw = std::is_same<R, float>::value ? reinterpret_cast<const CT*>(ax.tw32.p)
                                                  : reinterpret_cast<const CT*>(ax.tw64.p);
     const dim3 gz((unsigned)(((long long)nxy * B + ztl - 1) / ztl));
-    ps.kernel("zline_scale_kernel", {type_name<R>(), std::to_string(ax.cls), std::to_string(NC)});
+    ps.kernel("zline_scale_kernel", {type_name<R>(), ax.cls, NC});
     if (ax.cls == 0)
         hipLaunchKernelGGL((zline_scale_kernel<R, 0, NC>), gz, dim3(256), lds, s, grid, B, nxy, pl.n, pl.radix[0],
                            pl.radix[1], tw, ztl, kc);
@@ -5162,7 +5162,7 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
                 const bool ri = (S.n[2] & 1) != 0;  // odd nz: real / imaginary table entries
     #define MPM_ZT(ZSV)                                                                                           \
         case ZSV:                                                                                                 \
-            ps.kernel("ztoeplitz_kernel", {type_name<R>(), #ZSV, std::to_string(ztoe_as<R, ZSV>()), tbool(ri)}); \
+            ps.kernel("ztoeplitz_kernel", {type_name<R>(), #ZSV, ztoe_as<R, ZSV>(), tbool(ri)}); \
             if (ri)                                                                                               \
                 hipLaunchKernelGGL((ztoeplitz_kernel<R, ZSV, ztoe_as<R, ZSV>(), true>), gridz, dim3(256), 0, s,   \
                                    kgrid, B, ncols, Zs, rb, T);                                                   \

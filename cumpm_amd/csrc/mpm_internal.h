@@ -124,12 +124,20 @@ struct DevBuf {
 // Profiling (HIP events around kernel classes, on the launch stream).
 // ---------------------------------------------------------------------------
 struct ProfScope {
+    // a template argument of a kernel's name: text or a whole number, made a string only when
+    // the launch is recorded
+    struct Arg {
+        const char* text;
+        int number;
+        Arg(const char* t) : text(t), number(0) {}
+        Arg(int n) : text(nullptr), number(n) {}
+    };
     // units: right-hand sides the bracketed launches process (summed per class)
     ProfScope(const char* name, hipStream_t s, int64_t units = 0);
     ~ProfScope();
     // Also account the bracketed launch under the kernel's own name, written the way
     // profilers print template instances: base<arg0, arg1, ...>.
-    void kernel(const char* base, std::initializer_list<std::string> targs);
+    void kernel(const char* base, std::initializer_list<Arg> targs);
     const char* name;
     std::string kname;
     int64_t units;
@@ -154,8 +162,8 @@ struct HostLaps {
     bool on;
 };
 template <typename R>
-inline std::string type_name() { return std::is_same<R, float>::value ? "float" : "double"; }
-inline std::string tbool(bool b) { return b ? "true" : "false"; }
+inline const char* type_name() { return std::is_same<R, float>::value ? "float" : "double"; }
+inline const char* tbool(bool b) { return b ? "true" : "false"; }
 bool profiling_enabled();
 
 // ---------------------------------------------------------------------------

@@ -849,7 +849,7 @@ inline void region_spread(ProfScope& ps, hipStream_t s, const RegionSet& rs, con
     const dim3 gs((unsigned)rs.nreg, (unsigned)((ncols + cpb - 1) / cpb));
 #define MPM_SM1(RXV, ZSV, CPBV)                                                                                   \
     do {                                                                                                          \
-        ps.kernel("spread_mfma_kernel", {type_name<R>(), #RXV, #ZSV, #CPBV, std::to_string(NC)});                 \
+        ps.kernel("spread_mfma_kernel", {type_name<R>(), #RXV, #ZSV, #CPBV, NC});                 \
         hipLaunchKernelGGL((spread_mfma_kernel<R, RXV, ZSV, CPBV, NC>), gs, dim3(256), 0, s, t, B, rg, regw,      \
                            rs.start, rs.items, rs.quads, n3, grid);                                               \
         MPM_HIP(hipGetLastError());                                                                               \
@@ -897,16 +897,15 @@ inline void region_contract(ProfScope& ps, hipStream_t s, const RegionSet& rs, c
     const int ncg = ngrp >= 4 ? 4 : (ngrp >= 2 ? 2 : 1);
     const dim3 gs((unsigned)rs.nreg, (unsigned)((ngrp + ncg - 1) / ncg));
     const dim3 gn((unsigned)rs.nreg, (unsigned)ngrp);
-    const std::string ncs = std::to_string(NC) + ", " + type_name<GR>();
 #define MPM_NB1(RXV, ZSV, VECV)                                                                               \
     do {                                                                                                      \
-        ps.kernel("contract_nb_mfma_kernel", {type_name<R>(), #RXV, #ZSV, #VECV, ncs});                       \
+        ps.kernel("contract_nb_mfma_kernel", {type_name<R>(), #RXV, #ZSV, #VECV, NC, type_name<GR>()});                       \
         hipLaunchKernelGGL((contract_nb_mfma_kernel<R, RXV, ZSV, VECV, NC, GR>), gn, dim3(256), 0, s, B, rg,      \
                            regw, rs.start, rs.items, grid, pbuf);                                             \
     } while (0)
 #define MPM_CM1(RXV, ZSV, NBV, VECV)                                                                          \
     do {                                                                                                      \
-        ps.kernel("contract_mfma_kernel", {type_name<R>(), #RXV, #ZSV, std::to_string(NBV), #VECV, ncs});     \
+        ps.kernel("contract_mfma_kernel", {type_name<R>(), #RXV, #ZSV, NBV, #VECV, NC, type_name<GR>()});     \
         hipLaunchKernelGGL((contract_mfma_kernel<R, RXV, ZSV, NBV, VECV, NC, GR>), gs, dim3(256), 0, s, B, rg,    \
                            regw, rs.start, rs.items, grid, pbuf, ncg);                                        \
     } while (0)
@@ -920,7 +919,7 @@ inline void region_contract(ProfScope& ps, hipStream_t s, const RegionSet& rs, c
         }
     } else if (!rs.slab && vec) {
         ps.kernel("contract_full_mfma_kernel",
-                  {type_name<R>(), "4", std::to_string(kFullRegionPlanes), std::to_string(kFullContractNB), ncs});
+                  {type_name<R>(), "4", kFullRegionPlanes, kFullContractNB, NC, type_name<GR>()});
         const int nitems = rs.nreg * ngrp;
         hipLaunchKernelGGL((contract_full_mfma_kernel<R, 4, kFullRegionPlanes, kFullContractNB, NC, GR>),
                            dim3((unsigned)((nitems + 3) / 4)), dim3(256), 0, s, B, rg, regw, rs.start, nitems, ngrp,
