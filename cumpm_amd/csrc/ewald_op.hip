@@ -4044,10 +4044,7 @@ void EwaldOp::set_bloch(double kx, double ky) {
 //
 // The host keeps the O(N) cell lists (members in ascending index) and each particle's
 // cell; the device visits, for every particle i, the 27 cells around its own in the
-// host's order (dz, dy, dx = -1..1) and their members in order, a wave per particle and a
-// candidate per lane (4000 particles of a monolayer
-// 247 -> 30 us a pass, 7001 at 67 neighbours each 562 -> 81, 100,000 at 19 each, whose runs fill
-// a quarter of the lanes, 334 -> 452; a thread per particle before), so the CSR it builds is
+// host's order (dz, dy, dx = -1..1) and their members in order, so the CSR it builds is
 // the host's.  Pass 0 counts each particle's pairs, pass 1 fills them in: the neighbour,
 // x_j - x_i (minimum image), the table values (perp, para) at d_eff = max(d, 1) and, with
 // quadrupoles, the seven quadrupole table values (monodisperse_ewald_electric_field.cu
@@ -4074,6 +4071,9 @@ __device__ inline double tab_interp(const double* __restrict__ y, int ts, double
     return y[idx] * (1.0 - t) + y[idx + 1] * t;
 }
 
+// WAVE: a wave per particle and a candidate per lane, else a thread per particle (4000 particles
+// of a monolayer 247 -> 30 us a pass with waves, 7001 at 67 neighbours each 562 -> 81).
+template <bool WAVE>
 __global__ __launch_bounds__(256) void nb_search_kernel(int pass, int N, const double* __restrict__ pos, NbGeom g,
                                                         const int* __restrict__ cellc,
                                                         const int* __restrict__ cell_start,
@@ -4082,26 +4082,33 @@ __global__ __launch_bounds__(256) void nb_search_kernel(int pass, int N, const d
                                                         int* __restrict__ nb_j, double* __restrict__ pair_r,
                                                         double2* __restrict__ nb_f, double* __restrict__ pair_q,
                                                         const double* __restrict__ tab) {
-    const int lane = threadIdx.x & 63;
-    const int i = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (i >= N) return;  // whole wave
+    constexpr int NL = WAVE ? 64 : 1;  // lanes per particle
+    const int lane = threadIdx.x % NL;
+    const int i = blockIdx.x * (blockDim.x / NL) + threadIdx.x / NL;
+    if (i >= N) return;  // WAVE: the whole wave
     const double xi = pos[i], yi = pos[N + i], zi = pos[2 * N + i];
     int first = pass ? nb_start[i] : 0;  // the row's next free entry, the same in every lane
     int cnt = 0;
     // one candidate per lane (valid: this lane has one); accepted ones take consecutive entries
     // in lane order
     auto consider = [&](int j, bool valid) {
+        if (!WAVE && !valid) return;
         double r[3] = {xi - pos[j], yi - pos[N + j], zi - pos[2 * N + j]};
 #pragma unroll
         for (int d = 0; d < 3; ++d) r[d] -= g.L[d] * round(r[d] / g.L[d]);
         const double d2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+        if (!WAVE && !(d2 <= g.rc2)) return;
         const double dist = sqrt(d2);
         const bool take = valid && d2 <= g.rc2 && dist < g.rc;
-        const unsigned long long mask = __ballot(take);
-        cnt += __popcll(mask);
+        int k = first, n = take ? 1 : 0;
+        if (WAVE) {
+            const unsigned long long mask = __ballot(take);
+            k += __popcll(mask & ((1ull << lane) - 1ull));
+            n = __popcll(mask);
+        }
+        cnt += n;
         if (!pass) return;
-        const int k = first + __popcll(mask & ((1ull << lane) - 1ull));
-        first += __popcll(mask);
+        first += n;
         if (!take) return;
         nb_j[k] = j;
         const double de = dist < 1.0 ? 1.0 : dist;
@@ -4118,7 +4125,7 @@ __global__ __launch_bounds__(256) void nb_search_kernel(int pass, int N, const d
         const int cx = cellc[3 * i], cy = cellc[3 * i + 1], cz = cellc[3 * i + 2];
         // the three cells along x follow each other in the lists: one run of members, unless
         // the row wraps around the box
-        const bool run = cx > 0 && cx < g.nc[0] - 1;
+        const bool run = WAVE && cx > 0 && cx < g.nc[0] - 1;
         for (int dz = -1; dz <= 1; ++dz)
             for (int dy = -1; dy <= 1; ++dy) {
                 const int b = (cy + dy + g.nc[1]) % g.nc[1], c = (cz + dz + g.nc[2]) % g.nc[2];
@@ -4126,14 +4133,14 @@ __global__ __launch_bounds__(256) void nb_search_kernel(int pass, int N, const d
                 for (int dx = -1; dx <= (run ? -1 : 1); ++dx) {
                     const int cell = row + (cx + dx + g.nc[0]) % g.nc[0];
                     const int m1 = cell_start[cell + (run ? 3 : 1)];
-                    for (int m0 = cell_start[cell]; m0 < m1; m0 += 64) {
+                    for (int m0 = cell_start[cell]; m0 < m1; m0 += NL) {
                         const int j = cell_items[min(m0 + lane, m1 - 1)];
                         consider(j, m0 + lane < m1 && j != i);
                     }
                 }
             }
     } else {
-        for (int j0 = 0; j0 < N; j0 += 64) consider(min(j0 + lane, N - 1), j0 + lane < N && j0 + lane != i);
+        for (int j0 = 0; j0 < N; j0 += NL) consider(min(j0 + lane, N - 1), j0 + lane < N && j0 + lane != i);
     }
     if (!pass && lane == 0) count[i] = cnt;
 }
@@ -4201,10 +4208,28 @@ void EwaldOp::search_pairs_device(const std::vector<double>& pos, int Nn, bool c
     g.nq = nq;
     d_nb_count.resize((size_t)Nn + 1);
     d_nb_start.resize((size_t)Nn + 1);
-    const dim3 grid((unsigned)((Nn + 3) / 4));  // a wave per particle
-    hipLaunchKernelGGL(nb_search_kernel, grid, dim3(256), 0, nullptr, 0, Nn, d_pos.p, g, d_cellc.p, d_cell_start.p,
-                       d_cell_items.p, (const int*)nullptr, d_nb_count.p, (int*)nullptr, (double*)nullptr,
-                       (double2*)nullptr, (double*)nullptr, d_ptab.p);
+    // A thread per particle takes about the time of its own walk until its blocks fill the GPU, a
+    // wave per particle a time that grows with N and, while a run of three cells has fewer
+    // candidates than a wave has lanes, hardly with their number.  Both passes, in us, thread /
+    // wave: 20,000 particles with 6 candidates a run 265 / 204, 30,000 249 / 276, 100,000
+    // 378 / 778; with 14 a run 40,000 474 / 399, 60,000 510 / 557, 100,000 706 / 883; with 19 a
+    // run 100,000 910 / 916, and with 48 2553 / 1393.
+    size_t filled = 0;
+    for (size_t c = 0; c + 1 < cell_start.size(); ++c) filled += cell_start[c + 1] > cell_start[c];
+    const double run = 3.0 * Nn / (double)std::max<size_t>(filled, 1);
+    const bool wave = !cells || run >= 18.0 || Nn < 12000 + 2500 * run;
+    auto search = [&](int pass) {
+        auto go = [&](auto kernel, int per_block) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)((Nn + per_block - 1) / per_block)), dim3(256), 0, nullptr, pass, Nn,
+                               d_pos.p, g, d_cellc.p, d_cell_start.p, d_cell_items.p,
+                               pass ? d_nb_start.p : (const int*)nullptr, pass ? (int*)nullptr : d_nb_count.p,
+                               pass ? d_nb_j.p : (int*)nullptr, pass ? d_pair_r.p : (double*)nullptr,
+                               pass ? d_nb_f.p : (double2*)nullptr, pass && nq ? d_pairq.p : (double*)nullptr, d_ptab.p);
+        };
+        if (wave) go(nb_search_kernel<true>, 4);
+        else go(nb_search_kernel<false>, 256);
+    };
+    search(0);
     MPM_HIP(hipGetLastError());
     MPM_HIP(hipMemsetAsync(d_nb_count.p + Nn, 0, sizeof(int), nullptr));
     size_t tmp = 0;
@@ -4219,9 +4244,7 @@ void EwaldOp::search_pairs_device(const std::vector<double>& pos, int Nn, bool c
     d_pair_r.resize(3 * M);
     d_nb_f.resize(M);
     if (nq) d_pairq.resize(7 * M);
-    hipLaunchKernelGGL(nb_search_kernel, grid, dim3(256), 0, nullptr, 1, Nn, d_pos.p, g, d_cellc.p, d_cell_start.p,
-                       d_cell_items.p, (const int*)d_nb_start.p, (int*)nullptr, d_nb_j.p, d_pair_r.p, d_nb_f.p,
-                       nq ? d_pairq.p : (double*)nullptr, d_ptab.p);
+    search(1);
     MPM_HIP(hipGetLastError());
     if (total == 0) {  // the kernels read one entry: a harmless zero pair
         MPM_HIP(hipMemsetAsync(d_nb_j.p, 0, sizeof(int), nullptr));
