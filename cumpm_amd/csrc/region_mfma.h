@@ -406,7 +406,6 @@ template <typename R, int RX, int ZSB, int NB, bool VEC, int NC, typename GR>
 __global__ __launch_bounds__(256, sizeof(R) == 4 ? 3 : 2) void contract_mfma_kernel(int B, RegionGeom rg,
                                                                                     const R* __restrict__ regw,
                                                             const int* __restrict__ reg_start,
-                                                            const int* __restrict__ reg_items,
                                                             const typename C2<GR>::T* __restrict__ grid,
                                                             R* __restrict__ partial, int ncg) {
     using M = Mfma<R>;
@@ -577,7 +576,6 @@ __global__ __launch_bounds__(256, sizeof(R) == 4 ? 3 : 2) void contract_mfma_ker
 template <typename R, int RX, int ZSB, bool VEC, int NC, typename GR>
 __global__ __launch_bounds__(256) void contract_nb_mfma_kernel(int B, RegionGeom rg, const R* __restrict__ regw,
                                                                const int* __restrict__ reg_start,
-                                                               const int* __restrict__ reg_items,
                                                                const typename C2<GR>::T* __restrict__ grid,
                                                                R* __restrict__ partial) {
     using M = Mfma<R>;
@@ -849,9 +847,9 @@ inline void region_spread(ProfScope& ps, hipStream_t s, const RegionSet& rs, con
     const dim3 gs((unsigned)rs.nreg, (unsigned)((ncols + cpb - 1) / cpb));
 #define MPM_SM1(RXV, ZSV, CPBV)                                                                                   \
     do {                                                                                                          \
-        ps.kernel("spread_mfma_kernel", {type_name<R>(), #RXV, #ZSV, #CPBV, NC});                 \
+        ps.kernel("spread_mfma_kernel", {type_name<R>(), #RXV, #ZSV, #CPBV, NC});                             \
         hipLaunchKernelGGL((spread_mfma_kernel<R, RXV, ZSV, CPBV, NC>), gs, dim3(256), 0, s, t, B, rg, regw,      \
-                           rs.start, rs.items, rs.quads, n3, grid);                                               \
+                           rs.start, rs.items, rs.quads, n3, grid);                                           \
         MPM_HIP(hipGetLastError());                                                                               \
         return;                                                                                                   \
     } while (0)
@@ -899,15 +897,15 @@ inline void region_contract(ProfScope& ps, hipStream_t s, const RegionSet& rs, c
     const dim3 gn((unsigned)rs.nreg, (unsigned)ngrp);
 #define MPM_NB1(RXV, ZSV, VECV)                                                                               \
     do {                                                                                                      \
-        ps.kernel("contract_nb_mfma_kernel", {type_name<R>(), #RXV, #ZSV, #VECV, NC, type_name<GR>()});                       \
+        ps.kernel("contract_nb_mfma_kernel", {type_name<R>(), #RXV, #ZSV, #VECV, NC, type_name<GR>()});       \
         hipLaunchKernelGGL((contract_nb_mfma_kernel<R, RXV, ZSV, VECV, NC, GR>), gn, dim3(256), 0, s, B, rg,      \
-                           regw, rs.start, rs.items, grid, pbuf);                                             \
+                           regw, rs.start, grid, pbuf);                                                       \
     } while (0)
 #define MPM_CM1(RXV, ZSV, NBV, VECV)                                                                          \
     do {                                                                                                      \
         ps.kernel("contract_mfma_kernel", {type_name<R>(), #RXV, #ZSV, NBV, #VECV, NC, type_name<GR>()});     \
         hipLaunchKernelGGL((contract_mfma_kernel<R, RXV, ZSV, NBV, VECV, NC, GR>), gs, dim3(256), 0, s, B, rg,    \
-                           regw, rs.start, rs.items, grid, pbuf, ncg);                                        \
+                           regw, rs.start, grid, pbuf, ncg);                                                  \
     } while (0)
     if (dense_regions(rs)) {
         if (rs.zsb == 4) {
@@ -926,7 +924,7 @@ inline void region_contract(ProfScope& ps, hipStream_t s, const RegionSet& rs, c
                            grid, pbuf);
     } else if (!rs.slab) {
         MPM_CM1(4, 8, kFullContractNB, false);
-    } else {
+    } else if constexpr (NC == 8 || std::is_same<R, GR>::value) {  // dipole slabs sum in the grid's type
 #define MPM_CM(RXV, ZSV)                                   \
     case ZSV:                                              \
         if constexpr (NC == 3 || ZSV <= kQuadSlabPlanes) { \
@@ -952,6 +950,8 @@ inline void region_contract(ProfScope& ps, hipStream_t s, const RegionSet& rs, c
                 throw Error(MPM_ERR_RUNTIME, "slab size out of range");
         }
 #undef MPM_CM
+    } else {
+        throw Error(MPM_ERR_RUNTIME, "no contraction of this slab in FP64");
     }
 #undef MPM_CM1
 #undef MPM_NB1
