@@ -4506,9 +4506,14 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
     }
     const int zsb = zs_bucket((int)zl.size());
     // (quadrupoles: up to the planes their coupling kernel holds in registers, with two real
-    // in-plane axes and every length within the built-in transform)
+    // in-plane axes and every length within the built-in transform, and where the slab's two padded
+    // buffers are no larger than the full grid, so that an apply never needs more scratch than on
+    // the full grid; 4 voxels cover the second buffer's alignment)
+    const auto pad16 = [](int n) { return (size_t)((n + 15) / 16 * 16); };
+    const size_t slab_voxels = zl.size() * (S.n[0] * pad16(S.n[1]) + S.n[1] * pad16(S.n[0]));
     const bool may_slab = quads ? !quads_full && zsb <= kQuadSlabPlanes && S.n[0] > 1 && S.n[1] > 1 &&
-                                      LineFft::fits(S.n[0]) && LineFft::fits(S.n[1]) && LineFft::fits(nz)
+                                      LineFft::fits(S.n[0]) && LineFft::fits(S.n[1]) && LineFft::fits(nz) &&
+                                      slab_voxels + 4 <= V
                                 : force_full == 0;
     const bool want_slab = may_slab && zsb > 0 && (int)zl.size() * 2 <= nz &&
                            zfused_lds(zsb, nz, sizeof(double)) <= 64 * 1024;

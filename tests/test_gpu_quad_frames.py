@@ -150,3 +150,23 @@ def test_coefficients_asked_for_follow_the_tuned_grid():
         a, b = read(op, name, dt)[1], read(want, name, dt)[1]
         assert a.size == b.size, name
         np.testing.assert_array_equal(a, b, err_msg=name)
+
+
+def test_small_cells_need_no_more_scratch_than_the_full_grid():
+    # ten of 20 planes, rows of 33 padded to 48: two slab buffers would exceed the 64 MiB that
+    # the full grid's 24 right-hand sides fit
+    print("quad scratch", flush=True)
+    rng = np.random.default_rng(109)
+    grid, B = (33, 33, 20), 24
+    z = np.where(np.arange(N) % 2 == 0, 4, 14) * L[2] / grid[2]
+    pos = np.stack([rng.uniform(0, 1, N) * L[0], rng.uniform(0, 1, N) * L[1], z], 1)
+    op = Op(L, 1e-6, 0.5, grid=grid, support=4, quads=True)
+    op.set_positions(pos)
+    op.set_self_coef(np.full(N, 0.2 - 0.1j))
+    x = rng.standard_normal((B, op.n)) + 1j * rng.standard_normal((B, op.n))
+    xb, yb = C.DeviceBuffer(x.nbytes), C.DeviceBuffer(x.nbytes)
+    xb.upload(x)
+    C.check(C.load().mpm_op_apply_noalloc(op.h, xb.ptr, yb.ptr, B, C.PREC_DOUBLE, C.PART_ALL, None))
+    y = np.zeros_like(x)
+    yb.download(y)
+    assert rel(y, op.apply(x)) < 1e-12

@@ -64,7 +64,7 @@ def stages(op, x, precision):
     ((30, 28, 61), 8, (0.2,), True, (0.0, 0.0)),
     ((30, 27, 60), 4, (5.3, 15.1), [0, 3, 7], (0.07, -0.11)),
     ((9, 11, 60), 4, (59.8,), True, (0.0, 0.0)),  # a stencil over the end of the box
-    ((5, 4, 40), 6, (20.0,), [], (0.02, 0.0)),  # axes shorter than the stencil, no quadrupole
+    ((5, 6, 120), 6, (60.2,), [], (0.02, 0.0)),  # axes shorter than the stencil, no quadrupole
 ])
 def test_stages_match_the_full_grid_operator(grid, support, z_planes, quads, kb):
     print(f"quad stages {grid} support={support}", flush=True)
