@@ -423,6 +423,7 @@ class EwaldOp {
     void ensure_quad_scale_coef();
     void build_quad_tables();
     void build_quad_phases();
+    bool quad_gather(int B) const;
     template <typename R>
     void stage_quads_full(int which, const double2* x, void* grid, double2* y, hipStream_t s);
     std::unique_ptr<LineFft> lfft_stage;  // full-grid transforms of the slab operator's stages

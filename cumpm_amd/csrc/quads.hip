@@ -396,17 +396,26 @@ __global__ __launch_bounds__(2 * kQuadCols, ZS < 10 ? 2 : 1) void quad_zcouple_k
     }
 }
 
-// Eight lanes per (particle, right-hand side), lanes then right-hand sides fastest, particles
-// in spatial order: the particle's region contractions (partial [slot][16 B], null: none), the
+// NL lanes per (particle, right-hand side), lanes then right-hand sides fastest, particles
+// in spatial order: the particle's region contractions (partial [slot][16 B], null: none) or with
+// GATHER the contraction itself over the particle's stencil voxels of the full grid, the
 // real-space couplings of every neighbour's dipole and quadrupole (dipole -> field,
 // quadrupole -> field, dipole -> gradient, quadrupole -> gradient, :1631-1869 with the
 // cross-term signs of tests/quadrupole_field.py:214-215), the self terms (sc + self_perp for
 // the field, 2.5 sc + self_grad / 2 for the gradient) and the optional left Jacobi scaling.
-// Each lane takes every eighth slot and neighbour; a butterfly sum over the lanes (fixed order)
-// leaves component c of the result in lane c, which stores it.  FP64 sums.  Pair data [16]:
+// Each lane takes every NL-th slot or voxel and neighbour; a butterfly sum over the lanes (fixed
+// order) leaves component c of the result in lane c, which stores it.  FP64 sums.  Pair data [16]:
 // u (3), perp, para - perp, cos, sin, field_quad_1..3, grad_quad_1..4.
 constexpr int kQuadLanes = 8;
 
+// Stencils of the full grid for the gather.
+struct QuadStencil {
+    int n[3], W, m;           // m = 65536 / W + 1: o / W = o m >> 16 for o < W^3 <= 13^3
+    const int* base;          // [3][N] wrapped base voxel
+    const double* w64;        // [N][3][W]
+};
+
+template <int NL, bool GATHER, typename R>
 __global__ __launch_bounds__(256) void quad_finish_kernel(SlotTable tab, int B, int parts, int N,
                                                           const double* __restrict__ partial,
                                                           const int* __restrict__ ps_start,
@@ -417,8 +426,9 @@ __global__ __launch_bounds__(256) void quad_finish_kernel(SlotTable tab, int B, 
                                                           const double* __restrict__ pairq,
                                                           const double2* __restrict__ selfc, double self_perp,
                                                           double self_grad, int jacobi,
-                                                          const int* __restrict__ order) {
-    constexpr int NL = kQuadLanes;
+                                                          const int* __restrict__ order,
+                                                          const typename C2<R>::T* __restrict__ grid,
+                                                          QuadStencil st) {
     __shared__ const double2* s_x[kMaxSlots];
     __shared__ double2* s_y[kMaxSlots];
     __shared__ int s_row[kMaxSlots];
@@ -440,7 +450,36 @@ __global__ __launch_bounds__(256) void quad_finish_kernel(SlotTable tab, int B, 
     double acc[8][2];
 #pragma unroll
     for (int c = 0; c < 8; ++c) acc[c][0] = acc[c][1] = 0.0;
-    if (partial) {
+    if constexpr (GATHER) {
+        if (parts & MPM_PART_RECIP) {
+            const size_t plane = (size_t)st.n[1] * st.n[2], V = st.n[0] * plane;
+            const typename C2<R>::T* g = grid + (size_t)b * 8 * V;
+            const double* w = st.w64 + (size_t)i * 3 * st.W;
+            int s[3];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                s[d] = (st.base[(size_t)d * N + i] - st.W / 2) % st.n[d];
+                s[d] += s[d] < 0 ? st.n[d] : 0;
+            }
+            const int SS = st.W * st.W * st.W;
+            for (int o = sub; o < SS; o += NL) {
+                const int oxy = o * st.m >> 16, ox = oxy * st.m >> 16;
+                const int oy = oxy - ox * st.W, oz = o - oxy * st.W;
+                int v[3] = {s[0] + ox, s[1] + oy, s[2] + oz};
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                    while (v[d] >= st.n[d]) v[d] -= st.n[d];  // more than once where W exceeds the axis
+                const double ww = w[ox] * w[st.W + oy] * w[2 * st.W + oz];
+                const typename C2<R>::T* gv = g + v[0] * plane + (size_t)v[1] * st.n[2] + v[2];
+#pragma unroll
+                for (int c = 0; c < 8; ++c)
+                    if (c < 3 || qi >= 0) {
+                        acc[c][0] += ww * (double)gv[c * V].x;
+                        acc[c][1] += ww * (double)gv[c * V].y;
+                    }
+            }
+        }
+    } else if (partial) {
         const int s1 = ps_start[i + 1];
         for (int sl = ps_start[i] + sub; sl < s1; sl += NL) {
             const double* pp = partial + ((size_t)ps_items[sl] * B + b) * 16;
@@ -450,6 +489,8 @@ __global__ __launch_bounds__(256) void quad_finish_kernel(SlotTable tab, int B, 
                 acc[c][1] += pp[2 * c + 1];
             }
         }
+    }
+    if (GATHER || partial) {
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
             acc[c][0] *= h3;
@@ -575,6 +616,14 @@ void EwaldOp::build_quad_phases() {
     zcs_nz = nz;
 }
 
+// The contraction as part of the finish step, a wave per particle and right-hand side over the
+// stencil voxels of the full grid: up to three waves per SIMD one launch and more lanes decide
+// (FP32, an apply with the gather / on the regions: 900 particles with 7-point stencils, 1
+// right-hand side 61 / 87 us, 2 70 / 92, 4 108 / 121, 8 152 / 160; 1500 with 9-point stencils, 1 86 /
+// 102, 2 113 / 122, 4 184 / 157; 3000 with 5-point stencils, 1 77 / 87, 2 99 / 93).  The slab, whose
+// regions hold all planes, is faster on the regions at every size.
+bool EwaldOp::quad_gather(int B) const { return !slab && N * B <= 3072; }
+
 template <typename R>
 void EwaldOp::launch_quads(const SlotTable& t, int B, int parts, hipStream_t s, int jacobi) {
     using CT = typename C2<R>::T;
@@ -634,8 +683,9 @@ void EwaldOp::launch_quads(const SlotTable& t, int B, int parts, hipStream_t s, 
         }
     }
     if (!(phases & 4)) return;
+    const bool gather = quad_gather(B);
     const double* part = nullptr;
-    if (parts & MPM_PART_RECIP) {  // summed in FP64 over either grid
+    if (!gather && (parts & MPM_PART_RECIP)) {  // summed in FP64 over either grid
         ProfScope ps("contract", s, B);
         const bool aligned = (reinterpret_cast<uintptr_t>(grid) % 32) == 0;
         const bool vec = aligned && (slab ? (nyp % 2 == 0 && S.n[1] % 2 == 0) : S.n[2] % 2 == 0);
@@ -643,12 +693,16 @@ void EwaldOp::launch_quads(const SlotTable& t, int B, int parts, hipStream_t s, 
         part = d_partial64.p;
     }
     ProfScope ps("gather", s, B);
-    ps.kernel("quad_finish_kernel", {});
     const double h3 = S.h[0] * S.h[1] * S.h[2];
-    const size_t lanes = (size_t)Ni * B * kQuadLanes;
-    hipLaunchKernelGGL(quad_finish_kernel, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, s, t, B, parts, Ni,
-                       part, d_ps_start.p, d_ps_items.p, d_qmap.p, h3, d_nb_start.p, d_nb_j.p, d_pairc.p, d_selfc.p,
-                       self_perp, quad_self_grad, jacobi, d_order.p);
+    const QuadStencil st{{S.n[0], S.n[1], S.n[2]}, S.width, 65536 / S.width + 1, d_base.p, d_w64.p};
+    auto finish = [&](auto kernel, int lanes) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(((size_t)Ni * B * lanes + 255) / 256)), dim3(256), 0, s, t, B, parts,
+                           Ni, part, d_ps_start.p, d_ps_items.p, d_qmap.p, h3, d_nb_start.p, d_nb_j.p, d_pairc.p,
+                           d_selfc.p, self_perp, quad_self_grad, jacobi, d_order.p, grid, st);
+    };
+    ps.kernel("quad_finish_kernel", {gather ? 64 : kQuadLanes, tbool(gather), type_name<R>()});
+    if (gather) finish(quad_finish_kernel<64, true, R>, 64);
+    else finish(quad_finish_kernel<kQuadLanes, false, R>, kQuadLanes);
     MPM_HIP(hipGetLastError());
 }
 template void EwaldOp::launch_quads<float>(const SlotTable&, int, int, hipStream_t, int);

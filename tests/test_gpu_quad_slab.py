@@ -2,7 +2,8 @@
 regions, against the oracle's operator on the same grid (FP64 to 1e-11 of the largest value):
 every plane count the coupling kernel is compiled for, even and odd z lengths (Nyquist
 plane), separated layers, Bloch wave vectors, quadrupoles on a subset, narrow and wide batches;
-dense and sparse regions.  The FP32 reciprocal part to 1e-5 of the FP64 one: sums of at most
+dense and sparse regions, and the
+per-particle gather of small problems.  The FP32 reciprocal part to 1e-5 of the FP64 one: sums of at most
 9^3 rounded products on either side of transforms of at most 65,536 points, each about 1e-7.
 The stage-by-stage pipeline, whose grids are full grids, equals the apply.
 """
@@ -73,10 +74,17 @@ def test_quadrupole_slab_matches_oracle(grid, support, layers, quads, B, kb, ker
 
 
 @pytest.mark.parametrize("grid,N,support,quads,B,contract", [
-    ((24, 22, 20), 701, 8, True, 3, "contract_nb_mfma_kernel<double, 4, 4, true, 8, double>"),
-    ((23, 21, 19), 700, 4, list(range(0, 700, 3)), 2, "contract_nb_mfma_kernel<double, 4, 4, false, 8, double>"),
-    ((40, 36, 44), 60, 6, True, 4, "contract_full_mfma_kernel<double, 4, 8, 2, 8, double>"),
-    ((40, 36, 45), 60, 6, True, 1, "contract_mfma_kernel<double, 4, 8, 2, false, 8, double>"),
+    ((24, 22, 20), 701, 8, True, 5, "contract_nb_mfma_kernel<double, 4, 4, true, 8, double>"),
+    ((23, 21, 19), 700, 4, list(range(0, 700, 3)), 5, "contract_nb_mfma_kernel<double, 4, 4, false, 8, double>"),
+    ((40, 36, 44), 190, 6, True, 17, "contract_full_mfma_kernel<double, 4, 8, 2, 8, double>"),
+    ((40, 36, 45), 100, 6, True, 31, "contract_mfma_kernel<double, 4, 8, 2, false, 8, double>"),
+    # up to 3072 particles x right-hand sides: gathered per particle
+    ((24, 22, 20), 701, 8, True, 3, "quad_finish_kernel<64, true, double>"),
+    ((23, 21, 19), 700, 4, list(range(0, 700, 3)), 2, "quad_finish_kernel<64, true, double>"),
+    ((40, 36, 44), 60, 6, True, 4, "quad_finish_kernel<64, true, double>"),
+    ((40, 36, 45), 60, 6, True, 1, "quad_finish_kernel<64, true, double>"),
+    ((7, 9, 20), 50, 10, [1, 49], 2, "quad_finish_kernel<64, true, double>"),  # axes shorter than the stencil
+    ((30, 28, 61), 3072, 4, True, 1, "quad_finish_kernel<64, true, double>"),
 ])
 def test_quadrupole_full_grid_matches_oracle(grid, N, support, quads, B, contract):
     print(f"quad full grid={grid} N={N} support={support} B={B}", flush=True)
