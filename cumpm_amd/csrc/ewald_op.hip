@@ -2800,6 +2800,8 @@ __global__ __launch_bounds__(256) void gather_kernel(
             for (int c = 0; c < 3; ++c) acc[j][c][0] = acc[j][c][1] = 0.0;
 
         if (parts & MPM_PART_RECIP) {
+            // only an FP32 full grid comes with FP64 partial sums
+            constexpr bool MIXED = sizeof(R) == 4 && !SLAB;
             R racc[G][3][2];
 #pragma unroll
             for (int j = 0; j < G; ++j)
@@ -2818,7 +2820,7 @@ __global__ __launch_bounds__(256) void gather_kernel(
 #pragma unroll
                     for (int c = 0; c < 3; ++c) {
                         const int e = 6 * (g0 + j) + 2 * c;
-                        if (sizeof(R) == 8 || !part64) {
+                        if (!MIXED || !part64) {
                             racc[j][c][0] += pr[e];
                             racc[j][c][1] += pr[e + 1];
                         } else {
@@ -2862,13 +2864,13 @@ __global__ __launch_bounds__(256) void gather_kernel(
             for (int j = 0; j < G; ++j)
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
-                    // (FP64: acc holds nothing yet, and 0.0 + x is an addition to the compiler)
-                    if constexpr (sizeof(R) == 8) {
-                        acc[j][c][0] = racc[j][c][0] * h3;
-                        acc[j][c][1] = racc[j][c][1] * h3;
-                    } else {
+                    // (else acc holds nothing yet, and 0.0 + x is an addition to the compiler)
+                    if constexpr (MIXED) {
                         acc[j][c][0] = (acc[j][c][0] + (double)racc[j][c][0]) * h3;
                         acc[j][c][1] = (acc[j][c][1] + (double)racc[j][c][1]) * h3;
+                    } else {
+                        acc[j][c][0] = (double)racc[j][c][0] * h3;
+                        acc[j][c][1] = (double)racc[j][c][1] * h3;
                     }
                 }
         }
