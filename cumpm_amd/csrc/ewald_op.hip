@@ -5272,13 +5272,14 @@ void EwaldOp::launch(const SlotTable& t, int B, int parts, hipStream_t s, int ja
     bool part64 = false;  // FP64 partial sums
     // The contraction as part of the per-particle gather instead of on the regions: for
     // batches that take that kernel anyway (B < 4, below) and give it no more than a wave per
-    // SIMD (launches and latency decide; 400 particles on the slab, 3 right-hand sides: 76
-    // against 85 us an apply), and on the full
+    // SIMD, where launches and latency decide, except for three right-hand sides on a slab with
+    // at least 9 stencil points (640 particles, 3 right-hand sides, FP32: 41 against 51 us an apply
+    // with 5 points, 55 against 57 with 7; 882 with 9 points 99 against 93), and on the full
     // grid with stencils of at most 5 points per axis (125 voxels per particle are cheaper
     // to gather than the zero-padded products of its regions: 30,000 particles, 10 right-hand
     // sides 830 against 893 us; with 7 points 6 right-hand sides of 15,000 particles take
     // 563 on the regions, 644 gathered) or one right-hand side and few regions
-    const bool per_particle = (B < 4 && N <= 1024) ||
+    const bool per_particle = (B < 4 && N <= 1024 && !(SLAB && B == 3 && S.width >= 9)) ||
                               (!SLAB && (S.width <= 5 || (B == 1 && 4ll * nreg < (long long)N)));
     if (regions && !per_particle && (parts & MPM_PART_RECIP)) {
         ProfScope ps("contract", s, B);
