@@ -5012,6 +5012,11 @@ template <typename CT>
 static int zline_lines(const LineAxis& ax, int nc) {
     if (!ax.two) return 0;
     const LinePlan& pl = ax.plan;
+    // FP64 butterflies of 23 points fill the registers, and a short second stage leaves half of
+    // their threads idle: separate passes (46^3, three components, 32 right-hand sides 661
+    // against 677 us an apply; one component, 10 right-hand sides 123 against 134, 69^3 261
+    // against 263; 92^3 and lengths with a radix of 17 or 19 gain up to 6 %)
+    if (sizeof(CT) == 16 && pl.radix[0] > 19 && pl.radix[1] < (nc == 1 ? 4 : 3)) return 0;
     const size_t per_line = nc * (size_t)((pl.n + pl.radix[1]) | 1) * sizeof(CT);
     const size_t fixed = 2 * (size_t)pl.n * sizeof(CT) + 1024;
     const int by_lds = kMaxFusedLds > fixed ? (int)((kMaxFusedLds - fixed) / per_line) : 0;
@@ -5353,7 +5358,13 @@ void EwaldOp::launch_poly(const SlotTable& t, int B, int parts, hipStream_t s, i
     }
     if ((parts & MPM_PART_RECIP) && (phases & 2)) {
         const int zaxis = lfft->full_z;
-        const int ztl = zaxis >= 0 ? zline_lines<CT>(*lfft->axes[zaxis], 1) : 0;
+        // (FP32 lengths below 80 with a radix of 17 to 23, and FP64 ones with a radix of 23, only for
+        // small batches: 68^3, FP32, one right-hand side 63.3 -> 61.1 us, 10 right-hand sides 122 ->
+        // 125; 92^3, FP64, 115 -> 107 and 473 -> 484)
+        const LineAxis* za = zaxis >= 0 ? lfft->axes[zaxis].get() : nullptr;
+        const bool zworth = za && (za->cls < 2 || (fp32 ? S.n[2] >= 80 : za->plan.radix[0] <= 19) ||
+                                   (size_t)B * V * sizeof(CT) < ((size_t)16 << 20));
+        const int ztl = zworth ? zline_lines<CT>(*za, 1) : 0;
         const int skip = ztl >= 1 ? zaxis : -1;
         const R* kc = fp32 ? reinterpret_cast<const R*>(d_k32.p) : reinterpret_cast<const R*>(d_k64.p);
         {

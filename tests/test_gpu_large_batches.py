@@ -60,3 +60,34 @@ def test_polydisperse_z_pass_matches_oracle(grid, B):
         assert rel(y[b], ref.apply(p[b], sc)) < 1e-11
     r64 = op.apply(p, C.PREC_DOUBLE, C.PART_RECIP)
     assert rel(op.apply(p, C.PREC_MIXED, C.PART_RECIP), r64) < 1e-5
+
+
+@pytest.mark.parametrize("nz,B,precision,fused", [
+    (46, 3, C.PREC_DOUBLE, False), (69, 1, C.PREC_DOUBLE, False),  # 23 x 2, 23 x 3
+    (46, 3, C.PREC_MIXED, True), (51, 2, C.PREC_DOUBLE, True), (92, 2, C.PREC_DOUBLE, True),
+    (92, 8, C.PREC_DOUBLE, False),  # 4.0 and 16.2 MB
+    (68, 4, C.PREC_MIXED, True), (68, 30, C.PREC_MIXED, False),  # 17 x 4: 3.0 and 22.4 MB
+])
+def test_polydisperse_z_pass_of_large_radices(nz, B, precision, fused):
+    print(f"poly z pass nz={nz} B={B} precision={precision}", flush=True)
+    rng = np.random.default_rng(59)
+    L, grid = [24.0, 25.0, 26.0], (40, 36, nz)
+    N = 20
+    pos = rng.uniform(0, 1, (N, 3)) * L
+    rad = rng.uniform(1.0, 2.0, N)
+    op = Op(L, 1e-4, 0.5, grid=grid, radii=rad)
+    op.set_positions(pos)
+    sc = np.full(N, -0.2 + 0.1j)
+    op.set_self_coef(sc)
+    p = rng.standard_normal((B, N, 3)) + 1j * rng.standard_normal((B, N, 3))
+    C.profile_reset()
+    C.profile_enable(True)
+    y = op.apply(p, precision)
+    C.profile_enable(False)
+    assert any(n.startswith("zline_scale_kernel") for n in C.profile_names()) == fused, C.profile_names()
+    ref = O.PolyOperator(L, 1e-4, 0.5, rad, grid=list(grid))
+    ref.set_positions(pos)
+    # FP32: rounded products on either side of transforms of at most 97,920 points, below 1e-6 of
+    # the largest value of the reciprocal part, which the whole field exceeds
+    for b in sorted({0, B - 1}):
+        assert rel(y[b], ref.apply(p[b], sc)) < (1e-11 if precision == C.PREC_DOUBLE else 1e-6)
