@@ -4539,7 +4539,7 @@ void EwaldOp::set_positions(const double* xyz, int64_t n) {
     }
     // regions of the matrix-core spread and contraction: every particle joins each
     // region its stencil footprint meets.  Slab: x blocks of reg_rx and y blocks of
-    // 16, all slab planes in each region; full grid (dipoles of one radius): x blocks
+    // 16, all slab planes in each region; full grid (spheres of one radius): x blocks
     // of 4, y blocks of kFullRegionPlanes planes and z blocks of 16 rows.
     reg_rx = 0;
     reg_full = false;

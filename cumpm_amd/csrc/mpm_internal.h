@@ -298,7 +298,7 @@ class EwaldOp {
     double kb[2] = {0, 0};
     size_t V = 0;
     int64_t num_pairs = 0;
-    int force_full = 0;          // 1: never use the slab layout
+    int force_full = 0;          // 1: never use the slab layout (with quadrupoles quads_full decides)
     // reciprocal layout: the full grid, or the slab of occupied z-planes
     bool slab = false;
     int Zs = 0;
@@ -356,7 +356,7 @@ class EwaldOp {
     // particles of each region (CSR, ascending ids); reg_nry row blocks and reg_npb plane
     // blocks per x block of regions
     int reg_rx = 0, reg_nrx = 0, reg_nry = 0, reg_npb = 1, reg_pblk = 0;
-    bool reg_full = false;       // the regions tile the full grid (monodisperse dipoles)
+    bool reg_full = false;       // the regions tile the full grid (else the slab)
     int reg_slots = 0;           // (region, candidate) slots of the current frame
     RegionGeom region_geom(bool on_slab) const;
     RegionSet region_set(bool on_slab) const;
@@ -367,7 +367,9 @@ class EwaldOp {
     DevBuf<int> d_ps_items;      // slot ids (CSR positions of d_reg_items)
     DevBuf<double> d_regw64;     // [slot][row] region-local separable weights (FP64, FP32)
     DevBuf<float> d_regw32;
-    DevBuf<double> d_partial64;  // [slot][6 B] per-region contractions (FP64, or FP32 in its first half)
+    // [slot][6 B] ([slot][16 B] with quadrupoles) per-region contractions (FP64, or FP32 in its
+    // first half)
+    DevBuf<double> d_partial64;
     // k-space tables: (khat x, y, z, scale) per voxel for the full grid and the
     // z-DFT slab kernel, or the Toeplitz plane coupling [Zs][6][nx*ny] for a
     // contiguous slab; kspace_key records which one is current

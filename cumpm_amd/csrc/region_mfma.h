@@ -108,8 +108,6 @@ struct RegionW {
     static constexpr int NW = Y + kMfmaRY;
 };
 
-// Copies the precomputed region-local weight rows of a chunk of cnt <= KC
-// candidates into LDS (zero rows past cnt) and ends with a barrier.
 // v where c holds, else +0, by a bit mask rather than a select: the compiler turns a
 // select of a loaded value into a branch around the load, which then waits for
 // the load at the branch's end.
@@ -120,8 +118,10 @@ __device__ __forceinline__ double keep_if(double v, bool c) {
     return __longlong_as_double(__double_as_longlong(v) & (c ? -1LL : 0LL));
 }
 
-// Blocks of 256 threads; every load is issued before the first store (one memory
-// latency per chunk, not one per element).
+// Copies the precomputed region-local weight rows of a chunk of cnt <= KC
+// candidates into LDS (zero rows past cnt) and ends with a barrier.  Blocks of 256
+// threads; every load is issued before the first store (one memory latency per chunk,
+// not one per element).
 template <typename R, int RX, int ZSB, int KC = kMfmaKC>
 __device__ inline void stage_weights(R* s_w, int cnt, const R* __restrict__ regw) {
     using L = RegionW<RX, ZSB>;
@@ -221,7 +221,7 @@ __device__ inline RegionAt region_at(const RegionGeom& rg, int reg) {
 // FP32: held to 128 registers (four waves per SIMD; at the compiler's 140 three, and the
 // N = 4000 monolayer's 1272 blocks took 1.7 rounds instead of 1.2: 39.4 against 37.0 us).
 //
-// CPB = 16 is the form for few blocks (spread_cpb): there a region's candidates come in
+// CPB = 16 is the form for few blocks (region_spread): there a region's candidates come in
 // several chunks and nothing else hides their loads, so the next chunk's values and
 // weights are fetched while the current chunk's products run.
 // Weights of the spread: with quadrupoles FP64 rows, so that each product is rounded once

@@ -2,8 +2,9 @@
 compiled for, its first and last lengths, even lengths (the unpaired middle element), each axis
 of the full grid, the transposed slab passes, few and many lines (8, 16, 32 lines per block),
 against the oracle's operator on the same grid (FP64 1e-11 of the largest value) and FP32
-against FP64 (1e-5: transforms of at most 500,000 points and 7^3 rounded products on either
-side, each about 1e-7)."""
+against FP64 (1e-6: with u = 6e-8, transforms of at most 500,000 points forth and back grow as
+sqrt(2 log2 500,000) u = 6 u, and the sums of at most 7^3 rounded products on either side, whose
+few largest dominate, by about as much)."""
 import numpy as np
 import pytest
 
@@ -55,4 +56,4 @@ def test_lengths_with_large_primes_match_oracle(grid, tiles, B, layout):
     for b in sorted({0, B - 1}):
         assert rel(y[b], ref.apply(p[b], sc)) < 1e-11, b
     r64 = op.apply(p, C.PREC_DOUBLE, C.PART_RECIP)
-    assert rel(op.apply(p, C.PREC_MIXED, C.PART_RECIP), r64) < 1e-5
+    assert rel(op.apply(p, C.PREC_MIXED, C.PART_RECIP), r64) < 1e-6
