@@ -4,8 +4,9 @@
 //
 // Spread and contraction are the region kernels of region_mfma.h with 16 real columns per
 // right-hand side (exactly one column group of the matrix cores).  The grid is the z-plane slab
-// where the dipole operator would take one (as far as quad_zcouple_kernel's registers reach),
-// else the full grid.
+// where the dipole operator would take one (as far as quad_zcouple_kernel's registers reach, and
+// where it needs no more memory), else the full grid, whose small problems contract per particle
+// in the finish step.  Single stages work on full grids always.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
