@@ -85,7 +85,8 @@ typedef struct {
     double self_perp;    /* real-space self term (table entry 0) */
     double self_coef_ewald; /* -4 xi^3 / (3 sqrt(pi)) */
     double bloch[2];
-    int slab_planes;     /* occupied z-planes of the slab layout; 0 = full grid */
+    int slab_planes;     /* occupied z-planes of the slab layout; 0 = full grid (with quadrupoles
+                            always 0: the stages' grid, whatever layout the applies take) */
     int fft_backend;     /* FFT in use: 0 = built-in, 1 = rocFFT */
     int polydisperse;    /* 1 for an operator made by mpm_op_create_poly */
     int num_unique_radii;
